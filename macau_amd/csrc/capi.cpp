@@ -450,25 +450,23 @@ int macau_cond_normal_wishart(int K, int N, const double* U, const double* mu0, 
     ~StreamGuard() { (void)hipStreamSynchronize(s); (void)hipStreamDestroy(s); }
   } guard{s};
   const int KP = pad_latent(K);
-  DevBuf dU, dmu0, dT, dpart, dws, dmu, dL, dLf, dLmu, diter, dfail;
+  DevBuf dU, dmu0, dT, dpart, dmu, dL, dLf, dLmu, diter, dfail;
   upload(dU, std::vector<double>(U, U + (size_t)K * N), s);
   upload(dmu0, std::vector<double>(mu0, mu0 + K), s);
   upload(dT, std::vector<double>(T, T + (size_t)K * K), s);
   upload(diter, std::vector<int>{iter}, s);
   upload(dfail, std::vector<int>{0}, s);
   const int nblk = hyper_stats_blocks(N);
-  dpart.alloc((size_t)nblk * (K + K * K) * sizeof(double));
-  if (nw_workspace_bytes(K)) dws.alloc(nw_workspace_bytes(K));
+  dpart.alloc((size_t)(nblk + 1) * (K + K * K) * sizeof(double));  // and the draw's random numbers
   dmu.alloc(K * sizeof(double));
   dL.alloc((size_t)K * K * sizeof(double));
   dLf.alloc((size_t)KP * KP * sizeof(float));
   dLmu.alloc(KP * sizeof(float));
-  launch_hyper_stats_f64(dU.as<double>(), K, N, K, dpart.as<double>(), nblk, s);
   NWArgs a;
   a.K = K;
   a.KP = KP;
   a.partial = dpart.as<double>();
-  a.nblk = 1;  // totals in row 0
+  a.bart = dpart.as<double>() + (size_t)nblk * (K + K * K);
   a.N = N;
   a.kappa = kappa;
   a.mu0 = dmu0.as<double>();
@@ -477,12 +475,12 @@ int macau_cond_normal_wishart(int K, int N, const double* U, const double* mu0, 
   a.seed = seed;
   a.iter = diter.as<int>();
   a.mode = mode;
-  a.ws = dws.as<double>();
   a.mu = dmu.as<double>();
   a.Lambda = dL.as<double>();
   a.Lambda_f = dLf.as<float>();
   a.Lmu_f = dLmu.as<float>();
   a.fail = dfail.as<int>();
+  launch_hyper_stats_f64(dU.as<double>(), K, N, K, dpart.as<double>(), nblk, s, bartlett_of(a));
   launch_nw_draw(a, s);
   HIPCHK(hipGetLastError());
   int fail = 0;

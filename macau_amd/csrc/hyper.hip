@@ -1,4 +1,5 @@
-// hyper.hip -- FP64 hyperprior draw, adaptive noise, evaluation, RNG probes.
+// hyper.hip -- FP64 hyperprior statistics, adaptive noise, evaluation, RNG
+// probes.
 //
 // Normal-Wishart conjugate update (CondNormalWishart, mvnormal.cpp:314-336):
 //   mu_c = (kappa mu0 + sum U) / (kappa + N),  kappa_c = kappa + N,
@@ -7,8 +8,9 @@
 //   (mvnormal.cpp:217-266);  mu ~ N(mu_c, (kappa_c Lambda)^{-1})
 //   (MvNormal_prec, mvnormal.cpp:169-184).
 // The sufficient statistics are accumulated over columns by many work-groups
-// in FP64 and reduced in place into the first partial row; the K x K draw
-// then runs in one work-group per mode.
+// in FP64 and reduced in place into the first partial row, beside work-groups
+// that make the draw's random numbers (which need no statistics); the K x K
+// draw then runs in one work-group (nwdraw.hip).
 #include "common.h"
 #include "kernels.h"
 
@@ -147,16 +149,54 @@ __global__ void __launch_bounds__(StatShape<KP>::THREADS)
   }
 }
 
+// The random numbers of the Normal-Wishart draw: the Bartlett factor C (upper;
+// C_ii = sqrt(chi2(nu_c - i)), C_ij ~ N(0,1) for i < j: WishartUnit,
+// mvnormal.cpp:217-241) at out[j K + i], and the normals of mu at out[K K + j].
+// Item q: normals C[c][4b .. 4b+3] of one Philox block, then the diagonal,
+// then mu's blocks.
+__device__ __forceinline__ void bartlett_item(const BartlettArgs& a, int q) {
+  const int K = a.K, nb = (K + 3) / 4;
+  const uint32_t it = (uint32_t)(a.iter ? *a.iter : a.iter_value);
+  if (q < K * nb) {
+    const int c = q % K, b = q / K;
+    if (4 * b + 3 <= c) return;
+    double z[4];
+    normal_f64x4(a.seed, (uint32_t)c, (uint32_t)b, it, make_tag(TAG_WISHART_Z, a.mode), z);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = 4 * b + u;
+      if (j > c && j < K) a.out[j * K + c] = z[u];
+    }
+  } else if (q < K * nb + K) {
+    const int i = q - K * nb;
+    a.out[i * K + i] = sqrt(2.0 * gamma_f64(a.seed, 0.5 * (a.nu_c - i), (uint32_t)i, it,
+                                            make_tag(TAG_WISHART_CHI, a.mode)));
+  } else if (q < K * nb + K + nb) {
+    const int b = q - K * nb - K;
+    double z[4];
+    normal_f64x4(a.seed, 0u, (uint32_t)b, it, make_tag(TAG_NW_MU, a.mode), z);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (4 * b + u < K) a.out[K * K + 4 * b + u] = z[u];
+  }
+}
+
 // partial[0][q] = sum_b partial[b][q] in a fixed order: 16 interleaved
 // strands of blocks (strand g takes b = g, g + 16, ..., eight loads in
 // flight), combined in strand order.  A work-group owns 16 entries q, so
-// each load instruction reads 16 consecutive entries of 4 blocks.
+// each load instruction reads 16 consecutive entries of 4 blocks.  The first
+// nbart work-groups make the draw's random numbers instead.
 constexpr int kRedStrands = 16, kRedEntries = 256 / kRedStrands;
 
-__global__ void __launch_bounds__(256) k_stats_reduce(double* partial, int nblk, int width) {
+__global__ void __launch_bounds__(256) k_stats_reduce(double* partial, int nblk, int width, int nbart,
+                                                      BartlettArgs bart) {
   __shared__ double red[kRedStrands][kRedEntries];
+  if ((int)blockIdx.x < nbart) {
+    bartlett_item(bart, blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
   const int e = threadIdx.x % kRedEntries, g = threadIdx.x / kRedEntries;
-  const int q = blockIdx.x * kRedEntries + e;
+  const int q = (blockIdx.x - nbart) * kRedEntries + e;
   double s = 0.0;
   if (q < width) {
     int b = g;
@@ -179,15 +219,21 @@ __global__ void __launch_bounds__(256) k_stats_reduce(double* partial, int nblk,
   }
 }
 
+static void launch_reduce(double* partial, int nblk, int width, const BartlettArgs& bart, hipStream_t s) {
+  const int nred = nblk > 1 ? (width + kRedEntries - 1) / kRedEntries : 0;
+  const int nb = (bart.K + 3) / 4;
+  const int nbart = bart.out ? (bart.K * nb + bart.K + nb + 255) / 256 : 0;
+  if (nred + nbart)
+    hipLaunchKernelGGL(k_stats_reduce, dim3(nred + nbart), dim3(256), 0, s, partial, nblk, width, nbart, bart);
+}
+
 void launch_partial_reduce(double* partial, int nblk, int width, hipStream_t s) {
-  if (nblk > 1)
-    hipLaunchKernelGGL(k_stats_reduce, dim3((width + kRedEntries - 1) / kRedEntries), dim3(256), 0, s, partial, nblk,
-                       width);
+  launch_reduce(partial, nblk, width, BartlettArgs(), s);
 }
 
 template <typename T>
 static void launch_stats(const T* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
-                         hipStream_t s) {
+                         hipStream_t s, const BartlettArgs& bart) {
   const int KP = pad_latent(K);
   const int cols = (N + nblk - 1) / nblk;
   switch (KP) {
@@ -204,724 +250,16 @@ static void launch_stats(const T* U, const float* sub, int ld, int N, int K, dou
 #undef MGPU_STATS_CASE
     default: break;
   }
-  launch_partial_reduce(partial, nblk, K + K * K, s);
+  launch_reduce(partial, nblk, K + K * K, bart, s);
 }
 
 void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
-                            hipStream_t s) {
-  launch_stats<float>(U, sub, ld, N, K, partial, nblk, s);
+                            hipStream_t s, const BartlettArgs& bart) {
+  launch_stats<float>(U, sub, ld, N, K, partial, nblk, s, bart);
 }
-void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s) {
-  launch_stats<double>(U, nullptr, ld, N, K, partial, nblk, s);
-}
-
-// ------------------------------------------------------------------
-// Block-cooperative dense FP64 helpers (col-major, ld = K).
-// ------------------------------------------------------------------
-constexpr int kNWThreads = 256;
-
-// A = L L^T in place (lower), right-looking, upper part zeroed.  Returns
-// false if a pivot is not positive.
-__device__ bool blk_chol(double* A, int K, int* sflag) {
-  const int t = threadIdx.x;
-  for (int k = 0; k < K; k++) {
-    if (t == 0) {
-      const double d = A[k + k * K];
-      if (!(d > 0.0)) *sflag = 1;
-      A[k + k * K] = sqrt(d > 0.0 ? d : 1.0);
-    }
-    __syncthreads();
-    const double inv = 1.0 / A[k + k * K];
-    for (int i = k + 1 + t; i < K; i += kNWThreads) A[i + k * K] *= inv;
-    __syncthreads();
-    const int m = K - k - 1;
-    for (int q = t; q < m * m; q += kNWThreads) {
-      const int i = k + 1 + q % m, j = k + 1 + q / m;
-      if (j <= i) A[i + j * K] -= A[i + k * K] * A[j + k * K];
-    }
-    __syncthreads();
-  }
-  for (int q = t; q < K * K; q += kNWThreads) {
-    const int i = q % K, j = q / K;
-    if (i < j) A[q] = 0.0;
-  }
-  __syncthreads();
-  return *sflag == 0;
-}
-
-// Normal-Wishart draw of one mode (CondNormalWishart, mvnormal.cpp:314-336).
-// With X = T + S + kappa mu0 mu0^T - kappa_c mu_c mu_c^T and J the reversal
-// permutation, M = chol(J X J) gives chol(X^{-1}) = J M^{-T} J (the lower
-// Cholesky factor is unique), so the Bartlett draw
-//   Lambda = L_T (C^T C) L_T^T,  L_T = chol(T_c) = chol(X^{-1})
-// (Wishart, mvnormal.cpp:243-266) becomes Lambda = B B^T with
-// B = L_T C^T = J M^{-T} J C^T.  B is lower triangular with a positive
-// diagonal, i.e. B = chol(Lambda), hence chol(kappa_c Lambda) = sqrt(kappa_c) B
-// and mu = mu_c + B^{-T} z / sqrt(kappa_c) (MvNormal_prec, mvnormal.cpp:169-184).
-// These are the reference's quantities computed through one Cholesky and one
-// triangular solve instead of an explicit inverse, three Cholesky factors and
-// three products.
-__device__ void nw_draw(const NWArgs& a, double* base) {
-  __shared__ int sflag;
-  const int K = a.K, KK = K * K, t = threadIdx.x;
-  double* A = base;       // X, then M
-  double* Bm = A + KK;    // C (Bartlett, upper), then Z, then B
-  double* D = Bm + KK;    // Lambda
-  double* v_mu = D + KK;
-  double* v_z = v_mu + K;
-  double* v_nu = v_z + K;
-  if (t == 0) sflag = 0;
-  const int it = *a.iter;
-  const double N = a.N;
-  const double kappa_c = a.kappa + N, nu_c = a.nu + N;
-  // 1. reduce the partial statistics (fixed block order, loads batched)
-  const size_t stride = (size_t)(K + KK);
-  for (int q = t; q < K + KK; q += kNWThreads) {
-    double s = 0.0;
-    int b = 0;
-    for (; b + 8 <= a.nblk; b += 8) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = a.partial[(size_t)(b + u) * stride + q];
-#pragma unroll
-      for (int u = 0; u < 8; u++) s += v[u];
-    }
-    for (; b < a.nblk; b++) s += a.partial[(size_t)b * stride + q];
-    if (q < K) v_nu[q] = s;
-    else D[q - K] = s;  // NS
-  }
-  __syncthreads();
-  // 2. mu_c and X (mvnormal.cpp:322-325); Macau adds lambda_beta beta beta^T
-  //    to T (latentprior.cpp:258-260).  A holds J X J.
-  for (int k = t; k < K; k += kNWThreads) v_mu[k] = (a.kappa * a.mu0[k] + v_nu[k]) / (a.kappa + N);
-  const double lb = a.lambda_beta ? *a.lambda_beta : 0.0;
-  __syncthreads();
-  for (int q = t; q < KK; q += kNWThreads) {
-    const int i = q % K, j = q / K;
-    double tq = a.WI[q];
-    if (a.BBt_partial) {
-      double s = 0.0;
-      for (int b = 0; b < a.bbt_nblk; b++) s += a.BBt_partial[(size_t)b * stride + K + q];
-      tq += lb * s;
-    }
-    const double x = tq + D[q] + a.kappa * a.mu0[i] * a.mu0[j] - kappa_c * v_mu[i] * v_mu[j];
-    A[(K - 1 - i) + (K - 1 - j) * K] = x;
-  }
-  // Bartlett factor C (upper): C_ii = sqrt(chi2(nu_c - i)), C_ij ~ N(0,1)
-  // (WishartUnit, mvnormal.cpp:217-241)
-  for (int q = t; q < KK; q += kNWThreads) {
-    const int i = q % K, j = q / K;
-    double c = 0.0;
-    if (i == j) {
-      c = sqrt(2.0 * gamma_f64(a.seed, 0.5 * (nu_c - i), (uint32_t)i, (uint32_t)it, make_tag(TAG_WISHART_CHI, a.mode)));
-    } else if (j > i) {
-      c = normal_f64(a.seed, (uint32_t)i, (uint32_t)j, (uint32_t)it, make_tag(TAG_WISHART_Z, a.mode));
-    }
-    Bm[q] = c;
-  }
-  for (int k = t; k < K; k += kNWThreads)
-    v_z[k] = normal_f64(a.seed, 0u, (uint32_t)k, (uint32_t)it, make_tag(TAG_NW_MU, a.mode));
-  __syncthreads();
-  // 3. M = chol(J X J)
-  bool ok = blk_chol(A, K, &sflag);
-  // 4. Z = M^{-T} R, R = J C^T (R[i][c] = C[c][K-1-i]); rows of Z from the
-  //    bottom; Z[i][c] = 0 for i + c > K - 1 (exact structural zeros)
-  for (int i = K - 1; i >= 0; i--) {
-    for (int c = t; c < K; c += kNWThreads) {
-      if (i + c <= K - 1) {
-        double s = Bm[c + (K - 1 - i) * K];  // C[c][K-1-i]
-        for (int k = i + 1; k + c <= K - 1; k++) s -= A[k + i * K] * D[k + c * K];
-        D[i + c * K] = s / A[i + i * K];
-      } else {
-        D[i + c * K] = 0.0;
-      }
-    }
-    __syncthreads();
-  }
-  // B = J Z (lower triangular)
-  for (int q = t; q < KK; q += kNWThreads) {
-    const int i = q % K, c = q / K;
-    Bm[q] = D[(K - 1 - i) + c * K];
-  }
-  __syncthreads();
-  // 5. Lambda = B B^T
-  for (int q = t; q < KK; q += kNWThreads) {
-    const int i = q % K, j = q / K;
-    const int m = i < j ? i : j;
-    double s = 0.0;
-    for (int k = 0; k <= m; k++) s += Bm[i + k * K] * Bm[j + k * K];
-    D[q] = s;
-  }
-  __syncthreads();
-  // 6. mu = mu_c + B^{-T} z / sqrt(kappa_c)  (B^T upper, column-oriented)
-  for (int j = K - 1; j >= 0; j--) {
-    if (t == 0) v_z[j] = v_z[j] / Bm[j + j * K];
-    __syncthreads();
-    const double xj = v_z[j];
-    for (int i = t; i < j; i += kNWThreads) v_z[i] -= Bm[j + i * K] * xj;
-    __syncthreads();
-  }
-  const double isk = 1.0 / sqrt(kappa_c);
-  for (int k = t; k < K; k += kNWThreads) {
-    const double m = v_mu[k] + v_z[k] * isk;
-    a.mu[k] = m;
-    v_mu[k] = m;
-  }
-  __syncthreads();
-  // 7. outputs: FP64 state and the FP32 sampler parameters
-  const int KP = a.KP;
-  for (int q = t; q < KK; q += kNWThreads) {
-    a.Lambda[q] = D[q];
-    if (a.Lchol) a.Lchol[q] = Bm[q];
-  }
-  for (int q = t; q < KP * KP; q += kNWThreads) {
-    const int i = q % KP, j = q / KP;
-    float v = (i == j) ? 1.f : 0.f;
-    if (i < K && j < K) v = (float)D[i + j * K];
-    a.Lambda_f[q] = v;
-  }
-  for (int i = t; i < KP; i += kNWThreads) {
-    double s = 0.0;
-    if (i < K)
-      for (int j = 0; j < K; j++) s += D[i + j * K] * v_mu[j];
-    a.Lmu_f[i] = (float)s;
-  }
-  if (t == 0 && !ok && a.fail) atomicMax(a.fail, kFailNormalWishart);
-}
-
-// ------------------------------------------------------------------
-// The same draw in one work-group of four waves for K <= 64, every loop
-// rolled over K with the matrices in LDS.  The factorisation and solves are
-// chains of dependent FP64 operations on one wave, so their dot products
-// carry four partial sums, the draws of the Bartlett factor (which the
-// factorisation does not need) run on the other three waves meanwhile, and
-// Lambda = B B^T is split over all four.
-//   A: J X J, then M = chol(J X J) in its lower triangle (left-looking, lane
-//      i = row i), then B (rows);
-//   C: the Bartlett factor C (rows); Z = M^{-T} R, R = J C^T, is solved in
-//      place (lane c = column c of Z; R[i][c] = C[c][K-1-i] is read once, at
-//      the step that writes Z[i][c] to the same place), which leaves
-//      C[c][m] = Z[K-1-m][c] = B[m][c], i.e. C = B^T with B = J Z.
-// ------------------------------------------------------------------
-constexpr int kNWW = 64;         // largest K of this draw
-constexpr int kNWLd = kNWW + 1;  // row stride (doubles): lanes on their own rows hit distinct banks
-constexpr int kNWThreadsW = 256;
-
-struct NWWaveLds {
-  double A[kNWW][kNWLd];
-  double C[kNWW][kNWLd];
-  double muc[kNWW];     // mu_c, then mu
-  double z[kNWW];       // normals of the mu draw
-  double invd[kNWW];    // 1 / M[k][k]
-  double lm[4][kNWW];   // Lambda mu, per wave
-};
-
-// Philox block (row i, block b) of the strictly upper Bartlett normals
-// C[i][4b .. 4b+3]: item t of the blocks holding any j with i < j < K, in
-// block-column order
-__device__ __forceinline__ bool bartlett_block(int t, int K, int& i, int& b) {
-  for (int q = 0; 4 * q < K; q++) {
-    const int rows = min(4 * q + 3, K - 1);  // i = 0 .. rows-1 have a j > i in the block
-    if (t < rows) {
-      i = t;
-      b = q;
-      return true;
-    }
-    t -= rows;
-  }
-  return false;
-}
-
-// 1/sqrt(d), d > 0: the hardware estimate (v_rsq_f64) refined by two
-// Newton-Raphson steps for f(y) = y^-2 - d, y <- y (3 - d y^2) / 2, each of
-// which roughly squares the relative error
-__device__ __forceinline__ double rsqrt_nr(double d) {
-  double y = __builtin_amdgcn_rsq(d);
-  const double h = 0.5 * d;
-  y = y * fma(-h * y, y, 1.5);
-  y = y * fma(-h * y, y, 1.5);
-  return y;
-}
-
-// sum_{j in [j0, j1)} x[j] y[j] with four partial sums
-__device__ __forceinline__ double dot4(const double* x, const double* y, int j0, int j1) {
-  double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-  int j = j0;
-  for (; j + 4 <= j1; j += 4) {
-    p0 += x[j] * y[j];
-    p1 += x[j + 1] * y[j + 1];
-    p2 += x[j + 2] * y[j + 2];
-    p3 += x[j + 3] * y[j + 3];
-  }
-  for (; j < j1; j++) p0 += x[j] * y[j];
-  return (p0 + p1) + (p2 + p3);
-}
-
-// Lambda = B B^T (B rows in A, zero beyond column K) on all waves: lane r =
-// row r, wave w takes columns j = w, w + 4, ..., four at a time.  KB bounds
-// the row length.
-template <int KB>
-__device__ __forceinline__ void nw_lambda(const NWArgs& a, NWWaveLds& s, int wave, int lane) {
-  const int K = a.K, KP = a.KP;
-  const int r = lane;
-  double lm = 0.0;
-  for (int j0 = 4 * wave; j0 < KP; j0 += 16) {
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    const double* bj[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) bj[u] = s.A[min(j0 + u, kNWW - 1)];
-#pragma unroll 2
-    for (int k = 0; k < KB; k += 8) {
-      double br[8];
-#pragma unroll
-      for (int t = 0; t < 8; t++) br[t] = s.A[r][k + t];
-#pragma unroll
-      for (int t = 0; t < 8; t++)
-#pragma unroll
-        for (int u = 0; u < 4; u++) acc[u] += br[t] * bj[u][k + t];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int j = j0 + u;
-      if (j >= KP) break;
-      const bool in = r < K && j < K;
-      if (in) {
-        lm += acc[u] * s.muc[j];
-        a.Lambda[r + j * K] = acc[u];
-      }
-      if (r < KP) a.Lambda_f[r + j * KP] = in ? (float)acc[u] : (r == j ? 1.f : 0.f);
-    }
-  }
-  s.lm[wave][r] = lm;
-}
-
-__device__ void nw_draw_w(const NWArgs& a, NWWaveLds& s) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int K = a.K;
-  const bool act = lane < K;
-  const int it = *a.iter;
-  const double N = a.N;
-  const double kappa_c = a.kappa + N, nu_c = a.nu + N;
-  bool bad = false;
-  if (wave == 0) {
-    // 1. mu_c (mvnormal.cpp:322-323) and the normals of the mu draw
-    if (act) {
-      s.z[lane] = normal_f64(a.seed, 0u, (uint32_t)lane, (uint32_t)it, make_tag(TAG_NW_MU, a.mode));
-      s.muc[lane] = (a.kappa * a.mu0[lane] + a.partial[lane]) / kappa_c;
-    }
-    lds_wait();
-    // 2. A = J X J, X = T + S + kappa mu0 mu0^T - kappa_c mu_c mu_c^T
-    //    (mvnormal.cpp:324-325; Macau adds lambda_beta beta beta^T to T,
-    //    latentprior.cpp:258-260); lane = row, loads coalesced along it
-    const double lb = a.lambda_beta ? *a.lambda_beta : 0.0;
-    const double* bbt = a.BBt_partial ? a.BBt_partial + K : a.partial + K;
-    const double lbb = a.BBt_partial ? lb : 0.0;
-    const int xi = act ? K - 1 - lane : 0;
-    const double m0i = a.mu0[xi], mci = s.muc[xi];
-#pragma unroll 8
-    for (int c = 0; c < K; c++) {
-      const int xj = K - 1 - c;
-      const int e = xi + xj * K;
-      const double x = a.WI[e] + lbb * bbt[e] + a.partial[K + e] + a.kappa * m0i * a.mu0[xj] - kappa_c * mci * s.muc[xj];
-      if (act) s.A[lane][c] = x;
-    }
-    lds_wait();
-    // 3. M = chol(A), left-looking: s_i = A[i][k] - sum_{j<k} M[i][j] M[k][j]
-    //    on lane i, the pivot from lane k
-    for (int k = 0; k < K; k++) {
-      const double sk = s.A[lane][k] - dot4(s.A[lane], s.A[k], 0, k);
-      const double d = rdlane(sk, k);
-      const bool badp = !(d > 0.0);
-      bad = bad || badp;
-      const double rs = rsqrt_nr(badp ? 1.0 : d);
-      if (act && lane >= k) s.A[lane][k] = sk * rs;  // M[i][k]
-      s.invd[k] = rs;                               // every lane stores the same value
-      lds_wait();
-    }
-  } else {
-    // 4. Bartlett factor (waves 1-3): C_ii = sqrt(chi2(nu_c - i)),
-    //    C_ij ~ N(0,1) for i < j < K (WishartUnit, mvnormal.cpp:217-241),
-    //    zero below the diagonal; normals C[i][4b..4b+3] from one Philox block
-    const int t0 = threadIdx.x - 64;
-    for (int i = wave; i < K; i += 3)
-      if (lane < i) s.C[i][lane] = 0.0;
-    for (int t = t0;; t += kNWThreadsW - 64) {
-      int i, b;
-      if (!bartlett_block(t, K, i, b)) break;
-      double zz[4];
-      normal_f64x4(a.seed, (uint32_t)i, (uint32_t)b, (uint32_t)it, make_tag(TAG_WISHART_Z, a.mode), zz);
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int j = 4 * b + u;
-        if (j > i && j < K) s.C[i][j] = zz[u];
-      }
-    }
-    for (int i = t0; i < K; i += kNWThreadsW - 64)
-      s.C[i][i] = sqrt(2.0 * gamma_f64(a.seed, 0.5 * (nu_c - i), (uint32_t)i, (uint32_t)it,
-                                       make_tag(TAG_WISHART_CHI, a.mode)));
-  }
-  __syncthreads();
-  if (wave == 0) {
-    // 5. Z = M^{-T} R from the bottom row up, lane c = column c, in place in C
-    for (int i = K - 1; i >= 0; i--) {
-      double p0 = s.C[lane][K - 1 - i], p1 = 0.0, p2 = 0.0, p3 = 0.0;
-      int k = i + 1;
-      for (; k + 4 <= K; k += 4) {
-        p0 -= s.A[k][i] * s.C[lane][K - 1 - k];
-        p1 -= s.A[k + 1][i] * s.C[lane][K - 2 - k];
-        p2 -= s.A[k + 2][i] * s.C[lane][K - 3 - k];
-        p3 -= s.A[k + 3][i] * s.C[lane][K - 4 - k];
-      }
-      for (; k < K; k++) p0 -= s.A[k][i] * s.C[lane][K - 1 - k];
-      if (act) s.C[lane][K - 1 - i] = ((p0 + p1) + (p2 + p3)) * s.invd[i];
-    }
-    lds_wait();
-    // 6. B rows into A (B[i][c] = C[c][i]), zero beyond column K
-    for (int i = 0; i < K; i++) s.A[i][lane] = act ? s.C[lane][i] : 0.0;
-    // 7. mu = mu_c + B^{-T} z / sqrt(kappa_c) (MvNormal_prec, mvnormal.cpp:169-184):
-    //    B^T x = z from the last row up; lane r holds x_r, B[j][r] = C[r][j]
-    double acc = act ? s.z[lane] : 0.0;
-    const double invb = act ? 1.0 / s.C[lane][lane] : 0.0;
-    for (int j = K - 1; j >= 0; j--) {
-      const double xj = rdlane(acc * invb, j);
-      acc = (lane < j) ? acc - s.C[lane][j] * xj : (lane == j ? xj : acc);
-    }
-    if (act) {
-      const double mu = s.muc[lane] + acc / sqrt(kappa_c);
-      s.muc[lane] = mu;
-      a.mu[lane] = mu;
-    }
-    lds_wait();
-    if (a.Lchol && act)
-      for (int r = 0; r < K; r++) a.Lchol[lane + r * K] = s.A[lane][r];  // B[lane][r]
-  }
-  __syncthreads();
-  // 8. Lambda = B B^T and Lambda mu
-  if (K <= 32) nw_lambda<32>(a, s, wave, lane);
-  else nw_lambda<64>(a, s, wave, lane);
-  __syncthreads();
-  if (wave == 0 && lane < a.KP)
-    a.Lmu_f[lane] = (float)((s.lm[0][lane] + s.lm[1][lane]) + (s.lm[2][lane] + s.lm[3][lane]));
-  if (threadIdx.x == 0 && bad && a.fail) atomicMax(a.fail, kFailNormalWishart);
-}
-
-__global__ void __launch_bounds__(kNWThreadsW) k_nw_draw_w(NWBatch b) {
-  __shared__ NWWaveLds s;
-  nw_draw_w(b.m[blockIdx.x], s);
-}
-
-// The same draw for 64 < K <= 128 with every matrix in LDS (nw_draw keeps
-// them in a global workspace there: its per-step barriers then wait on
-// global memory, ~2.5 ms at K = 128).  Triangles are packed: M = chol(J X J)
-// lower, row i at i (i + 1) / 2; the Bartlett factor C upper, column j at
-// j (j + 1) / 2.  Row i of Z = M^{-T} J C^T only needs column K - 1 - i of C
-// and is written over it, and B = J Z is then the packed lower triangle
-// read row by row; Lambda = B B^T takes M's place.  Every value goes through
-// the same operations in the same order as in nw_draw.  LDS:
-// (K (K + 1) + 3 K) doubles, 132 KB at K = 128.
-__device__ __forceinline__ int tri(int i) { return i * (i + 1) / 2; }
-
-__global__ void __launch_bounds__(kNWThreads) k_nw_draw_lds(NWBatch b) {
-  extern __shared__ double dyn[];
-  const NWArgs& a = b.m[blockIdx.x];
-  __shared__ int sflag;
-  const int K = a.K, KK = K * K, t = threadIdx.x, T2 = tri(K);
-  double* Mp = dyn;         // J X J, then M (packed lower), then Lambda (packed lower)
-  double* Cp = Mp + T2;     // C (packed upper, by columns), then Z rows, i.e. B (packed lower)
-  double* v_mu = Cp + T2;
-  double* v_z = v_mu + K;
-  double* v_nu = v_z + K;
-  if (t == 0) sflag = 0;
-  const int it = *a.iter;
-  const double N = a.N;
-  const double kappa_c = a.kappa + N, nu_c = a.nu + N;
-  const size_t stride = (size_t)(K + KK);
-  auto reduce = [&](int q) {  // the statistic q summed over the blocks, in block order
-    double sum = 0.0;
-    int bb = 0;
-    for (; bb + 8 <= a.nblk; bb += 8) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = a.partial[(size_t)(bb + u) * stride + q];
-#pragma unroll
-      for (int u = 0; u < 8; u++) sum += v[u];
-    }
-    for (; bb < a.nblk; bb++) sum += a.partial[(size_t)bb * stride + q];
-    return sum;
-  };
-  // 1. sums of the columns, mu_c
-  for (int q = t; q < K; q += kNWThreads) v_nu[q] = reduce(q);
-  __syncthreads();
-  for (int k = t; k < K; k += kNWThreads) v_mu[k] = (a.kappa * a.mu0[k] + v_nu[k]) / (a.kappa + N);
-  const double lb = a.lambda_beta ? *a.lambda_beta : 0.0;
-  __syncthreads();
-  // 2. J X J (lower: entry (r, c) = X[K-1-r][K-1-c]), the Bartlett factor, z
-  for (int e = t; e < T2; e += kNWThreads) {
-    int r = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
-    while (tri(r) > e) r--;
-    while (tri(r + 1) <= e) r++;
-    const int c = e - tri(r);
-    const int i = K - 1 - r, j = K - 1 - c, q = i + j * K;
-    double tq = a.WI[q];
-    if (a.BBt_partial) {
-      double sb = 0.0;
-      for (int bb = 0; bb < a.bbt_nblk; bb++) sb += a.BBt_partial[(size_t)bb * stride + K + q];
-      tq += lb * sb;
-    }
-    Mp[e] = tq + reduce(K + q) + a.kappa * a.mu0[i] * a.mu0[j] - kappa_c * v_mu[i] * v_mu[j];
-    // C[c'][j'] of packed slot e (column j' = r, row c' = c)
-    double cv;
-    if (c == r)
-      cv = sqrt(2.0 * gamma_f64(a.seed, 0.5 * (nu_c - c), (uint32_t)c, (uint32_t)it, make_tag(TAG_WISHART_CHI, a.mode)));
-    else
-      cv = normal_f64(a.seed, (uint32_t)c, (uint32_t)r, (uint32_t)it, make_tag(TAG_WISHART_Z, a.mode));
-    Cp[e] = cv;
-  }
-  for (int k = t; k < K; k += kNWThreads)
-    v_z[k] = normal_f64(a.seed, 0u, (uint32_t)k, (uint32_t)it, make_tag(TAG_NW_MU, a.mode));
-  __syncthreads();
-  // 3. M = chol(J X J), right-looking in blocks of 4 columns, two barriers
-  //    per block: every thread factors the 4 x 4 diagonal block itself
-  //    (pivots <= 0 flagged and replaced by 1, as column by column), thread
-  //    t solves row k0 + 4 + t of the block column, thread 0 stores the
-  //    diagonal block's factor after the barrier (once no thread reads the
-  //    old entries), and the rank-4 trailing update runs on a 16 x 16
-  //    thread grid, each row's entries loaded before any is stored
-  const int tx = t & 15, ty = t >> 4;
-  for (int k0 = 0; k0 < K; k0 += 4) {
-    const int nb = K - k0 < 4 ? K - k0 : 4;
-    double L4[4][4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      if (c >= nb) break;
-      double d = Mp[tri(k0 + c) + k0 + c];
-#pragma unroll
-      for (int m = 0; m < c; m++) d -= L4[c][m] * L4[c][m];
-      if (t == 0 && !(d > 0.0)) sflag = 1;
-      L4[c][c] = sqrt(d > 0.0 ? d : 1.0);
-#pragma unroll
-      for (int r = c + 1; r < 4; r++) {
-        if (r >= nb) break;
-        double v = Mp[tri(k0 + r) + k0 + c];
-#pragma unroll
-        for (int m = 0; m < c; m++) v -= L4[r][m] * L4[c][m];
-        L4[r][c] = v / L4[c][c];
-      }
-    }
-    for (int i = k0 + nb + t; i < K; i += kNWThreads) {
-      double l[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) l[c] = c < nb ? Mp[tri(i) + k0 + c] : 0.0;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        if (c >= nb) break;
-#pragma unroll
-        for (int m = 0; m < c; m++) l[c] -= l[m] * L4[c][m];
-        l[c] = l[c] / L4[c][c];
-      }
-#pragma unroll
-      for (int c = 0; c < 4; c++)
-        if (c < nb) Mp[tri(i) + k0 + c] = l[c];
-    }
-    __syncthreads();
-    if (t == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-#pragma unroll
-        for (int c = 0; c <= r; c++)
-          if (r < nb) Mp[tri(k0 + r) + k0 + c] = L4[r][c];
-    }
-    const int j0 = k0 + nb;
-    for (int i = j0 + ty; i < K; i += 16) {
-      double li[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) li[c] = c < nb ? Mp[tri(i) + k0 + c] : 0.0;
-      double x[8], s4[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = j0 + tx + 16 * u;
-        const bool in = j <= i;
-        x[u] = in ? Mp[tri(i) + j] : 0.0;
-        double sv = 0.0;
-#pragma unroll
-        for (int c = 0; c < 4; c++) sv += (in && c < nb) ? li[c] * Mp[tri(j) + k0 + c] : 0.0;
-        s4[u] = sv;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = j0 + tx + 16 * u;
-        if (j <= i) Mp[tri(i) + j] = x[u] - s4[u];
-      }
-    }
-    __syncthreads();
-  }
-  const bool ok = sflag == 0;
-  // 4. Z = M^{-T} R, R = J C^T, rows from the bottom, right-looking in
-  //    blocks of 4 rows: row i of R lives over column K - 1 - i of C (slots
-  //    tri(K-1-i) + c, c <= K - 1 - i).  For a block of rows b0..b0+nb-1,
-  //    thread c solves the block's 4 x 4 upper system for its column c
-  //    (rows i with c <= K - 1 - i), then every row i' < b0 subtracts
-  //    sum_k M_ki' Z_k over the block's rows k with c <= K - 1 - k (16 x 16
-  //    thread grid, each row's entries loaded before any store)
-  for (int b1 = K; b1 > 0; b1 -= 4) {
-    const int b0 = b1 - 4 > 0 ? b1 - 4 : 0, nb = b1 - b0;
-    for (int c = t; c <= K - 1 - b0; c += kNWThreads) {
-      double z[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 3; q >= 0; q--) {
-        const int i = b0 + q;
-        if (q >= nb || c > K - 1 - i) continue;
-        double v = Cp[tri(K - 1 - i) + c];
-#pragma unroll
-        for (int q2 = q + 1; q2 < 4; q2++)
-          if (q2 < nb && c <= K - 1 - (b0 + q2)) v -= Mp[tri(b0 + q2) + i] * z[q2];
-        z[q] = v / Mp[tri(i) + i];
-        Cp[tri(K - 1 - i) + c] = z[q];
-      }
-    }
-    __syncthreads();
-    const int cmax = K - 1 - b0;  // widest row of the block
-    for (int i2 = ty; i2 < b0; i2 += 16) {
-      double m[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) m[q] = q < nb ? Mp[tri(b0 + q) + i2] : 0.0;
-      const int j2 = K - 1 - i2;
-      double x[8], s4[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int c = tx + 16 * u;
-        const bool in = c <= cmax;
-        x[u] = in ? Cp[tri(j2) + c] : 0.0;
-        double sv = 0.0;
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          sv += (in && q < nb && c <= K - 1 - (b0 + q)) ? m[q] * Cp[tri(K - 1 - (b0 + q)) + c] : 0.0;
-        s4[u] = sv;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int c = tx + 16 * u;
-        if (c <= cmax) Cp[tri(j2) + c] = x[u] - s4[u];
-      }
-    }
-    __syncthreads();
-  }
-  // B[i][c] = Z[K-1-i][c] = Cp[tri(i) + c] (c <= i).
-  // 5. Lambda = B B^T (packed lower, over M), four partial sums per entry
-  for (int e = t; e < T2; e += kNWThreads) {
-    int i = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
-    while (tri(i) > e) i--;
-    while (tri(i + 1) <= e) i++;
-    const int j = e - tri(i);
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int k = 0;
-    for (; k + 4 <= j + 1; k += 4) {
-      s0 += Cp[tri(i) + k] * Cp[tri(j) + k];
-      s1 += Cp[tri(i) + k + 1] * Cp[tri(j) + k + 1];
-      s2 += Cp[tri(i) + k + 2] * Cp[tri(j) + k + 2];
-      s3 += Cp[tri(i) + k + 3] * Cp[tri(j) + k + 3];
-    }
-    for (; k <= j; k++) s0 += Cp[tri(i) + k] * Cp[tri(j) + k];
-    Mp[e] = (s0 + s1) + (s2 + s3);
-  }
-  // 6. mu = mu_c + B^{-T} z / sqrt(kappa_c): back substitution on wave 0,
-  //    lane l holding z_l and z_{l+64}, the solved value broadcast by a
-  //    shuffle (no barrier per step)
-  if (t < 64) {
-    double z0 = v_z[t], z1 = t + 64 < K ? v_z[t + 64] : 0.0;
-    for (int j = K - 1; j >= 0; j--) {
-      const double zj = j >= 64 ? __shfl(z1, j - 64, 64) : __shfl(z0, j, 64);
-      const double xj = zj / Cp[tri(j) + j];
-      if (t == j) z0 = xj;
-      if (t + 64 == j) z1 = xj;
-      if (t < j) z0 -= Cp[tri(j) + t] * xj;
-      if (t + 64 < j) z1 -= Cp[tri(j) + t + 64] * xj;
-    }
-    v_z[t] = z0;
-    if (t + 64 < K) v_z[t + 64] = z1;
-  }
-  __syncthreads();
-  const double isk = 1.0 / sqrt(kappa_c);
-  for (int k = t; k < K; k += kNWThreads) {
-    const double m = v_mu[k] + v_z[k] * isk;
-    a.mu[k] = m;
-    v_mu[k] = m;
-  }
-  __syncthreads();
-  // 7. outputs
-  const int KP = a.KP;
-  for (int q = t; q < KK; q += kNWThreads) {
-    const int i = q % K, j = q / K;
-    a.Lambda[q] = i >= j ? Mp[tri(i) + j] : Mp[tri(j) + i];
-    if (a.Lchol) a.Lchol[q] = i >= j ? Cp[tri(i) + j] : 0.0;
-  }
-  for (int q = t; q < KP * KP; q += kNWThreads) {
-    const int i = q % KP, j = q / KP;
-    float v = (i == j) ? 1.f : 0.f;
-    if (i < K && j < K) v = (float)(i >= j ? Mp[tri(i) + j] : Mp[tri(j) + i]);
-    a.Lambda_f[q] = v;
-  }
-  for (int i = t; i < KP; i += kNWThreads) {
-    double sv = 0.0;
-    if (i < K)
-      for (int j = 0; j < K; j++) sv += (i >= j ? Mp[tri(i) + j] : Mp[tri(j) + i]) * v_mu[j];
-    a.Lmu_f[i] = (float)sv;
-  }
-  if (t == 0 && !ok && a.fail) atomicMax(a.fail, kFailNormalWishart);
-}
-
-// one work-group per mode of the batch
-__global__ void __launch_bounds__(kNWThreads) k_nw_draw(NWBatch b) {
-  extern __shared__ double dyn[];
-  const NWArgs& a = b.m[blockIdx.x];
-  nw_draw(a, a.ws ? a.ws : dyn);
-}
-
-static size_t nw_lds_bytes(int K) { return (size_t)(3 * K * K + 3 * K) * sizeof(double); }
-size_t nw_workspace_bytes(int K) { return nw_lds_bytes(K) <= 48 * 1024 ? 0 : nw_lds_bytes(K); }
-
-void launch_nw_draw_batch(const NWBatch& b, hipStream_t s) {
-  if (b.n <= 0) return;
-  // one wave per mode when the statistics arrive reduced and K <= 64
-  bool wave = true;
-  for (int q = 0; q < b.n; q++) wave = wave && b.m[q].nblk == 1 && b.m[q].K <= kNWW;
-  if (wave) {
-    hipLaunchKernelGGL(k_nw_draw_w, dim3(b.n), dim3(kNWThreadsW), 0, s, b);
-    return;
-  }
-  // 64 < K <= 128: the LDS-resident draw where the device grants a
-  // work-group that much LDS (checked once per device)
-  const int K = b.m[0].K;
-  if (K > kNWW && K <= 128) {
-    const size_t bytes = (size_t)(K * (K + 1) + 3 * K) * sizeof(double);
-    static int granted[64] = {0};  // per device: 0 unknown, 1 yes, -1 no
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
-      if (granted[dev] == 0) {
-        int optin = 0;
-        granted[dev] = -1;
-        if (hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev) == hipSuccess &&
-            (size_t)optin >= (size_t)(128 * 129 + 3 * 128) * sizeof(double) &&
-            hipFuncSetAttribute((const void*)k_nw_draw_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)((size_t)(128 * 129 + 3 * 128) * sizeof(double))) == hipSuccess)
-          granted[dev] = 1;
-        (void)hipGetLastError();
-      }
-      if (granted[dev] == 1) {
-        hipLaunchKernelGGL(k_nw_draw_lds, dim3(b.n), dim3(kNWThreads), bytes, s, b);
-        return;
-      }
-    }
-  }
-  const bool lds = b.m[0].ws == nullptr;
-  hipLaunchKernelGGL(k_nw_draw, dim3(b.n), dim3(kNWThreads), lds ? nw_lds_bytes(b.m[0].K) : 0, s, b);
-}
-
-void launch_nw_draw(const NWArgs& a, hipStream_t s) {
-  NWBatch b;
-  b.m[0] = a;
-  b.n = 1;
-  launch_nw_draw_batch(b, s);
+void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s,
+                            const BartlettArgs& bart) {
+  launch_stats<double>(U, nullptr, ld, N, K, partial, nblk, s, bart);
 }
 
 // ------------------------------------------------------------------

@@ -145,42 +145,58 @@ int batched_seg_grid(const BatchPlan& p);
 // reduced in place: the totals are in partial[0] when the launch completes.
 // hyper_stats_blocks(N) is the block count to allocate and pass.
 int hyper_stats_blocks(int N);
+// The random numbers of a Normal-Wishart draw (see k_stats_reduce), made
+// beside the reduction when out is set; out has K + K*K entries
+struct BartlettArgs {
+  double* out = nullptr;
+  int K = 0;
+  double nu_c = 0;  // posterior degrees of freedom
+  uint64_t seed = 0;
+  const int* iter = nullptr;
+  int iter_value = 0;  // the iteration when iter is null
+  int mode = 0;
+};
 void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
-                            hipStream_t s);
-void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s);
+                            hipStream_t s, const BartlettArgs& bart = BartlettArgs());
+void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s,
+                            const BartlettArgs& bart = BartlettArgs());
 
 struct NWArgs {
   int K = 0, KP = 0;
-  const double* partial = nullptr;  // nblk x (K + K*K), summed over the rows
-  int nblk = 0;
-  double N = 0;                     // number of columns
+  const double* partial = nullptr;      // K + K*K: the reduced statistics
+  double N = 0;                         // number of columns
   double kappa = 2.0;
-  const double* mu0 = nullptr;      // K
-  const double* WI = nullptr;       // K x K base scale
-  const double* BBt_partial = nullptr;  // Macau: partial stats of beta (or null)
-  int bbt_nblk = 0;
+  const double* mu0 = nullptr;          // K
+  const double* WI = nullptr;           // K x K base scale
+  const double* BBt_partial = nullptr;  // Macau: reduced statistics of beta (or null)
   const double* lambda_beta = nullptr;  // device scalar (Macau)
-  double nu = 0;                    // degrees of freedom
+  double nu = 0;                        // degrees of freedom
   uint64_t seed = 0;
   const int* iter = nullptr;
+  int iter_value = 0;                   // the iteration when iter is null
   int mode = 0;
-  double* ws = nullptr;             // workspace (nw_workspace_bytes), or null for LDS
-  double* mu = nullptr;             // out K
-  double* Lambda = nullptr;         // out K x K
-  double* Lchol = nullptr;          // out chol(Lambda), K x K (or null)
-  float* Lambda_f = nullptr;        // out KP x KP
-  float* Lmu_f = nullptr;           // out KP
-  int* fail = nullptr;
+  double* bart = nullptr;               // the random numbers (BartlettArgs::out)
+  double* mu = nullptr;                 // out K
+  double* Lambda = nullptr;             // out K x K
+  double* Lchol = nullptr;              // out chol(Lambda), K x K (or null)
+  float* Lambda_f = nullptr;            // out KP x KP
+  float* Lmu_f = nullptr;               // out KP
+  int* fail = nullptr;                  // raised when a matrix is not positive definite (or null)
+  int* status = nullptr;                // out 0 or kFailNormalWishart (or null)
 };
+inline BartlettArgs bartlett_of(const NWArgs& a) {
+  BartlettArgs b;
+  b.out = a.bart;
+  b.K = a.K;
+  b.nu_c = a.nu + a.N;
+  b.seed = a.seed;
+  b.iter = a.iter;
+  b.iter_value = a.iter_value;
+  b.mode = a.mode;
+  return b;
+}
+// after launch_hyper_stats_* with bartlett_of(a)
 void launch_nw_draw(const NWArgs& a, hipStream_t s);
-// draws of several modes (same K) in one launch, one work-group per mode
-struct NWBatch {
-  NWArgs m[kMaxOther + 1];
-  int n = 0;
-};
-void launch_nw_draw_batch(const NWBatch& b, hipStream_t s);
-// global workspace the draw needs for latent size K (0: fits in LDS)
-size_t nw_workspace_bytes(int K);
 
 // --- noise and evaluation ---
 struct NoiseArgs {

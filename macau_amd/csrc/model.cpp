@@ -843,8 +843,8 @@ void ILatentPrior::init(Model& m, int mode) {
   upload(Lambda_f, Lf, m.stream);
   upload(Lmu_f, Lmuf, m.stream);
   stats_nblk = hyper_stats_blocks(m.dims[mode]);
-  stats.alloc((size_t)stats_nblk * (K + K * K) * sizeof(double));
-  if (nw_workspace_bytes(K)) nw_ws.alloc(nw_workspace_bytes(K));
+  // the blocks' partial sums, then the draw's random numbers
+  stats.alloc((size_t)(stats_nblk + 1) * (K + K * K) * sizeof(double));
   HIPCHK(hipStreamSynchronize(m.stream));
 }
 
@@ -872,7 +872,7 @@ static NWArgs nw_args(Model& m, ILatentPrior& p, int mode, double nu) {
   a.K = m.num_latent;
   a.KP = m.KP;
   a.partial = p.stats.as<double>();
-  a.nblk = 1;  // launch_hyper_stats leaves the totals in row 0
+  a.bart = p.stats.as<double>() + (size_t)p.stats_nblk * (a.K + a.K * a.K);
   a.N = m.dims[mode];
   a.kappa = 2.0;  // b0 (latentprior.cpp:97)
   a.mu0 = p.mu0.as<double>();
@@ -881,7 +881,6 @@ static NWArgs nw_args(Model& m, ILatentPrior& p, int mode, double nu) {
   a.seed = m.seed;
   a.iter = m.d_iter_prior.as<int>();
   a.mode = mode;
-  a.ws = p.nw_ws.as<double>();
   a.mu = p.mu.as<double>();
   a.Lambda = p.Lambda.as<double>();
   a.Lambda_f = p.Lambda_f.as<float>();
@@ -891,9 +890,10 @@ static NWArgs nw_args(Model& m, ILatentPrior& p, int mode, double nu) {
 }
 
 void BPMFPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:79-81
+  const NWArgs a = nw_args(m, *this, mode, (double)m.num_latent);  // df = K
   launch_hyper_stats_f32(m.d_U[mode].as<float>(), nullptr, m.KP, m.dims[mode], m.num_latent, stats.as<double>(),
-                         stats_nblk, m.stream);
-  launch_nw_draw(nw_args(m, *this, mode, (double)m.num_latent), m.stream);  // df = K
+                         stats_nblk, m.stream, bartlett_of(a));
+  launch_nw_draw(a, m.stream);
 }
 
 // ---- MacauPrior ----
@@ -1308,11 +1308,11 @@ void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
   const int K = m.num_latent, KP = m.KP, N = nrow;
   hipStream_t s = m.stream;
   // residual statistics of U - Uhat, and beta beta^T of the current beta
-  launch_hyper_stats_f32(m.d_U[mode].as<float>(), Uhat.as<float>(), KP, N, K, stats.as<double>(), stats_nblk, s);
-  launch_hyper_stats_f64(beta.as<double>(), K, nfeat, K, bbt.as<double>(), bbt_nblk, s);
   NWArgs a = nw_args(m, *this, mode, (double)K + (double)nfeat);  // df + beta.cols()
+  launch_hyper_stats_f32(m.d_U[mode].as<float>(), Uhat.as<float>(), KP, N, K, stats.as<double>(), stats_nblk, s,
+                         bartlett_of(a));
+  launch_hyper_stats_f64(beta.as<double>(), K, nfeat, K, bbt.as<double>(), bbt_nblk, s);
   a.BBt_partial = bbt.as<double>();
-  a.bbt_nblk = 1;
   a.lambda_beta = lambda_beta_d.as<double>();
   a.Lchol = Lchol.as<double>();
   launch_nw_draw(a, s);
@@ -1498,8 +1498,10 @@ void MacauOnePrior::update_prior(Model& m, int mode) {  // macauoneprior.cpp:189
   const int K = m.num_latent, KP = m.KP, N = nrow;
   hipStream_t s = m.stream;
   // sample_mu_lambda (:198-213): CondNormalWishart(U - Uhat, 0, 2, I, K), diagonal kept
-  launch_hyper_stats_f32(m.d_U[mode].as<float>(), Uhat.as<float>(), KP, N, K, stats.as<double>(), stats_nblk, s);
-  launch_nw_draw(nw_args(m, *this, mode, (double)K), s);
+  const NWArgs a = nw_args(m, *this, mode, (double)K);
+  launch_hyper_stats_f32(m.d_U[mode].as<float>(), Uhat.as<float>(), KP, N, K, stats.as<double>(), stats_nblk, s,
+                         bartlett_of(a));
+  launch_nw_draw(a, s);
   launch_uni_diag(K, KP, Lambda.as<double>(), Lambda_f.as<float>(), Lmu_f.as<float>(), mu.as<double>(), s);
   // sample_beta (:215-252) from the previous Uhat
   BetaUniArgs b;

@@ -104,7 +104,7 @@ class ILatentPrior {
   virtual const float* prior_mean_rows() const { return nullptr; }
 
   // device parameters shared with the sampler (FP64 state + FP32 copies)
-  DevBuf mu, Lambda, Lambda_f, Lmu_f, mu0, WI, stats, nw_ws;
+  DevBuf mu, Lambda, Lambda_f, Lmu_f, mu0, WI, stats;
   int stats_nblk = 0;
 };
 
