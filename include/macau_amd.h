@@ -207,7 +207,7 @@ int macau_cond_normal_wishart(int num_latent, int N, const double* U, const doub
  * K, d_Lambda_out: K x K, *d_status: 0, or nonzero when a matrix was not
  * positive definite), the work is queued asynchronously on `stream`
  * (a hipStream_t; NULL = the null stream) and no device memory is allocated
- * or freed.  Working memory is one static device array of 2,146,560 bytes per
+ * or freed.  Working memory is one static device array of 5,457,408 bytes per
  * GPU (held until the process ends), so num_latent must be in [1, 64]; larger
  * values fail with an error.  Calls that overlap on one GPU share that array
  * and race. */

@@ -456,8 +456,8 @@ int macau_cond_normal_wishart(int K, int N, const double* U, const double* mu0, 
   upload(dT, std::vector<double>(T, T + (size_t)K * K), s);
   upload(diter, std::vector<int>{iter}, s);
   upload(dfail, std::vector<int>{0}, s);
-  const int nblk = hyper_stats_blocks(N);
-  dpart.alloc((size_t)(nblk + 1) * (K + K * K) * sizeof(double));  // and the draw's random numbers
+  const int nblk = hyper_stats_blocks(N, K);
+  dpart.alloc(hyper_stats_doubles(nblk, K) * sizeof(double));
   dmu.alloc(K * sizeof(double));
   dL.alloc((size_t)K * K * sizeof(double));
   dLf.alloc((size_t)KP * KP * sizeof(float));
@@ -466,7 +466,7 @@ int macau_cond_normal_wishart(int K, int N, const double* U, const double* mu0, 
   a.K = K;
   a.KP = KP;
   a.partial = dpart.as<double>();
-  a.bart = dpart.as<double>() + (size_t)nblk * (K + K * K);
+  a.bart = hyper_stats_bart(dpart.as<double>(), K);
   a.N = N;
   a.kappa = kappa;
   a.mu0 = dmu0.as<double>();

@@ -8,144 +8,194 @@
 //   (mvnormal.cpp:217-266);  mu ~ N(mu_c, (kappa_c Lambda)^{-1})
 //   (MvNormal_prec, mvnormal.cpp:169-184).
 // The sufficient statistics are accumulated over columns by many work-groups
-// in FP64 and reduced in place into the first partial row, beside work-groups
+// in FP64 and reduced in a fixed order, beside work-groups
 // that make the draw's random numbers (which need no statistics); the K x K
 // draw then runs in one work-group (nwdraw.hip).
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
 namespace mgpu {
 
-constexpr int kMaxStatBlocks = 512;
+// ------------------------------------------------------------------
+// Sufficient statistics of x_n = U[:, n] - sub[:, n] (sub optional, FP32, same
+// ld) in FP64: sum_n x_n and sum_n x_n x_n^T.
+//
+// The scatter is a product with the columns as reduction index, so it runs on
+// v_mfma_f64_16x16x4f64, four columns a step: lane l holds entry l % 16 of each
+// 16-component tile of column l / 16, which is the A and the B operand of every
+// tile product at once.  No LDS between the loads and the products; only lower
+// tiles are formed.  With KP <= 64 each wave takes its own columns and holds
+// every tile (10 at most), and a work-group's four waves are summed through
+// LDS at the end; above, the 36 tiles are shared by the waves (rows w and 7 - w
+// of the triangle on wave w: nine each), which walk the same columns.
+// FP32 factors have their components dealt to the tiles in turn (component
+// c NT + t is entry c of tile t), so a lane's NT values are one contiguous load.
+// Statistics and reduction before (4 x 4 register tiles per thread over LDS
+// tiles of 16 columns, partials of the whole K x K) and now, alone on the card:
+// 100003 x 64 FP64 140 -> 24 us (51 MB: 2.6 TB/s in the first kernel), 3001 x
+// 128 FP32 37 -> 15 us; with the draw, 138000 x 32 FP32 79 -> 35 us.
+// ------------------------------------------------------------------
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-int hyper_stats_blocks(int N) {
-  int b = (N + 127) / 128;
-  if (b < 1) b = 1;
-  if (b > kMaxStatBlocks) b = kMaxStatBlocks;
-  return b;
+static int stats_tiles(int K) { return K <= 16 ? 1 : K <= 32 ? 2 : K <= 64 ? 4 : 8; }
+// doubles of a block's partial: the tiles' sums, then the lower tiles
+static int stats_width(int K) {
+  const int nt = stats_tiles(K);
+  return 16 * nt + 128 * nt * (nt + 1);
+}
+// One work-group per 32 columns up to one per CU; half as many above K = 64,
+// where a partial is 74 KB and the reduction's reads begin to count
+int hyper_stats_blocks(int N, int K) {
+  const int cap = K > 64 ? 128 : 256;
+  return std::max(1, std::min(cap, (N + 31) / 32));
+}
+size_t hyper_stats_doubles(int nblk, int K) { return (size_t)2 * (K + K * K) + (size_t)nblk * stats_width(K); }
+
+// component of entry c of tile t
+template <typename T, int NT>
+__host__ __device__ __forceinline__ constexpr int stats_component(int t, int c) {
+  return sizeof(T) == 4 ? c * NT + t : 16 * t + c;
 }
 
-template <int KP>
-struct StatShape {
-  static constexpr int TD = KP / 4;                       // 4 x 4 tiles per dimension
-  static constexpr int GT = TD * TD < 64 ? 64 : TD * TD;  // threads per column group
-  static constexpr int G = GT >= 256 ? 1 : 256 / GT;      // column groups per block
-  static constexpr int THREADS = GT * G;
-  static constexpr int TC = 16;                           // columns per LDS tile
-  static constexpr int EPT = TC * KP / GT;                // tile elements loaded per thread
-  static constexpr int TILE = G * 2 * TC * KP;            // doubles, double buffered
-  static constexpr int RED = G > 1 ? G * (KP + KP * KP) : 0;
-  static constexpr int SMEM = TILE > RED ? TILE : RED;
-};
-
-// Sufficient statistics of x_n = U[:, n] - sub[:, n] (sub optional, FP32,
-// same ld) over the block's run of columns, in FP64:
-//   partial[blk] = (sum_n x_n (K), sum_n x_n x_n^T (K x K, col-major)).
-// The block's columns are split between G column groups; each group streams
-// its columns through a double-buffered LDS tile of 16 columns (the loads of
-// tile t + 1 are in flight while tile t is used), and thread (ti, tj) of a
-// group owns rows 4ti..4ti+3 x columns 4tj..4tj+3 of the K x K sum in
-// registers.  The groups' sums are combined in group order.
-template <typename T, int KP>
-__global__ void __launch_bounds__(StatShape<KP>::THREADS)
+template <typename T, int NT>
+__global__ void __launch_bounds__(256)
     k_hyper_stats(const T* __restrict__ U, const float* __restrict__ sub, int ld, int N, int K, int cols,
                   double* __restrict__ partial) {
-  using S = StatShape<KP>;
-  constexpr int TD = S::TD, GT = S::GT, G = S::G, TC = S::TC, EPT = S::EPT;
-  __shared__ double smem[S::SMEM];
-  const int t = threadIdx.x, g = t / GT, gt = t % GT;
-  const int ti = gt % TD, tj = gt / TD;
-  const bool act = gt < TD * TD;
+  constexpr bool kShared = NT > 4;                      // the waves share the tiles
+  constexpr int NTILE = NT * (NT + 1) / 2;
+  constexpr int WIDTH = 16 * NT + 256 * NTILE;
+  constexpr int STEP = kShared ? 4 : 16;                // columns a work-group takes per step
+  constexpr int AHEAD = NT <= 2 ? 4 : NT == 4 ? 2 : 1;  // steps whose loads are in flight
+  __shared__ double red[kShared ? 1 : 2 * WIDTH];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = lane >> 4, c = lane & 15;
   const int b0 = blockIdx.x * cols, b1 = min(N, b0 + cols);
-  const int per = (cols + G - 1) / G;
-  const int c0 = min(b1, b0 + g * per), c1 = min(b1, c0 + per);
-  const int ntiles = (per + TC - 1) / TC;
-  double* tile = smem + (size_t)g * 2 * TC * KP;
-  double reg[EPT];
-  auto load = [&](int tt) {
+  const int first = b0 + (kShared ? 0 : 4 * wave) + g;
+  f64x4 acc[kShared ? 12 : NTILE];
 #pragma unroll
-    for (int e = 0; e < EPT; e++) {
-      const int f = gt + e * GT, c = f / KP, i = f % KP;
-      const int col = c0 + tt * TC + c;
-      double x = 0.0;
-      if (col < c1 && i < K) {
-        x = (double)U[(size_t)col * ld + i];
-        if (sub) x -= (double)sub[(size_t)col * ld + i];
+  for (int q = 0; q < (kShared ? 12 : NTILE); q++) acc[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+  double sum[NT];
+#pragma unroll
+  for (int q = 0; q < NT; q++) sum[q] = 0.0;
+
+  T raw[AHEAD][NT];
+  float rsub[AHEAD][NT];
+  auto load = [&](T(&x)[NT], float(&y)[NT], int col) {
+    const size_t at = (size_t)min(col, N - 1) * ld;
+    if constexpr (sizeof(T) == 4 && NT > 1) {  // ld = 16 NT: entries c NT .. c NT + NT - 1
+      typedef float vec __attribute__((ext_vector_type(NT == 2 ? 2 : 4)));
+      constexpr int P = NT == 2 ? 2 : 4;
+#pragma unroll
+      for (int p = 0; p < NT / P; p++) {
+        const vec v = *reinterpret_cast<const vec*>(U + at + c * NT + p * P);
+        vec w = 0.f;
+        if (sub) w = *reinterpret_cast<const vec*>(sub + at + c * NT + p * P);
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+          x[p * P + q] = v[q];
+          y[p * P + q] = w[q];
+        }
       }
-      reg[e] = x;
+    } else {
+#pragma unroll
+      for (int q = 0; q < NT; q++) {
+        const int k = min(stats_component<T, NT>(q, c), ld - 1);
+        x[q] = U[at + k];
+        y[q] = sub ? sub[at + k] : 0.f;
+      }
     }
   };
-  double acc[4][4], sum[4];
+  if (b0 < b1) {
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    sum[r] = 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) acc[r][q] = 0.0;
+    for (int u = 0; u < AHEAD; u++) load(raw[u], rsub[u], first + u * STEP);
   }
-  load(0);
-  for (int tt = 0; tt < ntiles; tt++) {
-    double* tb = tile + (tt & 1) * TC * KP;
+  for (int n0 = first - g; n0 < b1; n0 += AHEAD * STEP) {
 #pragma unroll
-    for (int e = 0; e < EPT; e++) tb[gt + e * GT] = reg[e];
+    for (int u = 0; u < AHEAD; u++) {
+      const int col = n0 + g + u * STEP;
+      double x[NT];
+#pragma unroll
+      for (int q = 0; q < NT; q++) {
+        double v = (double)raw[u][q];
+        if (sizeof(T) == 4) v -= (double)rsub[u][q];
+        x[q] = (col < b1 && stats_component<T, NT>(q, c) < K) ? v : 0.0;
+        sum[q] += x[q];
+      }
+      load(raw[u], rsub[u], col + AHEAD * STEP);
+      if constexpr (!kShared) {
+        int id = 0;
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+#pragma unroll
+          for (int j = 0; j <= i; j++, id++)
+            acc[id] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], x[j], acc[id], 0, 0, 0);
+      } else {
+        const double lo = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
+        const double hi = wave == 0 ? x[7] : wave == 1 ? x[6] : wave == 2 ? x[5] : x[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (j <= wave) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(lo, x[j], acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (j <= 7 - wave) acc[4 + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(hi, x[j], acc[4 + j], 0, 0, 0);
+      }
+    }
+  }
+  // sums over the four columns of a step
+#pragma unroll
+  for (int q = 0; q < NT; q++) {
+    sum[q] += __shfl_xor(sum[q], 16, 64);
+    sum[q] += __shfl_xor(sum[q], 32, 64);
+  }
+  double* out = partial + (size_t)blockIdx.x * WIDTH;
+  if constexpr (kShared) {
+    if (wave == 0 && g == 0) {
+#pragma unroll
+      for (int q = 0; q < NT; q++) out[16 * q + c] = sum[q];
+    }
+    auto store = [&](int i, int j, const f64x4& v) {
+      double* o = out + 16 * NT + 256 * (i * (i + 1) / 2 + j);
+#pragma unroll
+      for (int u = 0; u < 4; u++) o[64 * u + lane] = v[u];
+    };
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (j <= wave) store(wave, j, acc[j]);
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (j <= 7 - wave) store(7 - wave, j, acc[4 + j]);
+  } else {
+    // waves 1 and 3 to LDS, added by 0 and 2; then 2 to LDS, added by 0
+    auto put = [&](double* r) {
+      if (g == 0) {
+#pragma unroll
+        for (int q = 0; q < NT; q++) r[16 * q + c] = sum[q];
+      }
+#pragma unroll
+      for (int q = 0; q < NTILE; q++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) r[16 * NT + 256 * q + 64 * u + lane] = acc[q][u];
+    };
+    auto add = [&](const double* r) {
+#pragma unroll
+      for (int q = 0; q < NT; q++) sum[q] += r[16 * q + c];
+#pragma unroll
+      for (int q = 0; q < NTILE; q++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) acc[q][u] += r[16 * NT + 256 * q + 64 * u + lane];
+    };
+    if (wave & 1) put(red + (wave >> 1) * WIDTH);
     __syncthreads();
-    if (tt + 1 < ntiles) load(tt + 1);
-    if (act) {
-#pragma unroll 4
-      for (int c = 0; c < TC; c++) {
-        const double* x = tb + c * KP;
-        double xi[4], xj[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          xi[r] = x[4 * ti + r];
-          xj[r] = x[4 * tj + r];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          sum[r] += xi[r];
-#pragma unroll
-          for (int q = 0; q < 4; q++) acc[r][q] += xi[r] * xj[q];
-        }
-      }
+    if (!(wave & 1)) add(red + (wave >> 1) * WIDTH);
+    __syncthreads();
+    if (wave == 2) put(red);
+    __syncthreads();
+    if (wave == 0) {
+      add(red);
+      put(out);
     }
-  }
-  const int KK = K * K;
-  double* out = partial + (size_t)blockIdx.x * (K + KK);
-  if (G == 1) {
-    if (!act) return;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = 4 * ti + r;
-      if (i >= K) continue;
-      if (tj == 0) out[i] = sum[r];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int j = 4 * tj + q;
-        if (j < K) out[K + i + j * K] = acc[r][q];
-      }
-    }
-    return;
-  }
-  __syncthreads();  // tiles are dead: reuse the LDS for the group sums
-  double* red = smem + (size_t)g * (K + KK);
-  if (act) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = 4 * ti + r;
-      if (i >= K) continue;
-      if (tj == 0) red[i] = sum[r];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int j = 4 * tj + q;
-        if (j < K) red[K + i + j * K] = acc[r][q];
-      }
-    }
-  }
-  __syncthreads();
-  for (int q = t; q < K + KK; q += S::THREADS) {
-    double v = 0.0;
-#pragma unroll
-    for (int h = 0; h < G; h++) v += smem[(size_t)h * (K + KK) + q];
-    out[q] = v;
   }
 }
 
@@ -181,22 +231,17 @@ __device__ __forceinline__ void bartlett_item(const BartlettArgs& a, int q) {
   }
 }
 
-// partial[0][q] = sum_b partial[b][q] in a fixed order: 16 interleaved
-// strands of blocks (strand g takes b = g, g + 16, ..., eight loads in
-// flight), combined in strand order.  A work-group owns 16 entries q, so
-// each load instruction reads 16 consecutive entries of 4 blocks.  The first
-// nbart work-groups make the draw's random numbers instead.
+// sum_b partial[b][q] in a fixed order: 16 interleaved strands of blocks
+// (strand g takes b = g, g + 16, ..., eight loads in flight), combined in
+// strand order.  A work-group owns 16 entries q, so each load instruction reads
+// 16 consecutive entries of 4 blocks.  Valid on threads 0 .. 15 (entry
+// threadIdx.x of the work-group).
 constexpr int kRedStrands = 16, kRedEntries = 256 / kRedStrands;
 
-__global__ void __launch_bounds__(256) k_stats_reduce(double* partial, int nblk, int width, int nbart,
-                                                      BartlettArgs bart) {
+__device__ __forceinline__ double strands_sum(const double* partial, int nblk, int width, int q0) {
   __shared__ double red[kRedStrands][kRedEntries];
-  if ((int)blockIdx.x < nbart) {
-    bartlett_item(bart, blockIdx.x * 256 + threadIdx.x);
-    return;
-  }
   const int e = threadIdx.x % kRedEntries, g = threadIdx.x / kRedEntries;
-  const int q = (blockIdx.x - nbart) * kRedEntries + e;
+  const int q = q0 + e;
   double s = 0.0;
   if (q < width) {
     int b = g;
@@ -211,55 +256,88 @@ __global__ void __launch_bounds__(256) k_stats_reduce(double* partial, int nblk,
   }
   red[g][e] = s;
   __syncthreads();
-  if (g == 0 && q < width) {
-    double t = red[0][e];
+  double t = 0.0;
+  if (g == 0) {
+    t = red[0][e];
 #pragma unroll
     for (int h = 1; h < kRedStrands; h++) t += red[h][e];
-    partial[q] = t;
   }
+  return t;
 }
 
-static void launch_reduce(double* partial, int nblk, int width, const BartlettArgs& bart, hipStream_t s) {
-  const int nred = nblk > 1 ? (width + kRedEntries - 1) / kRedEntries : 0;
-  const int nb = (bart.K + 3) / 4;
-  const int nbart = bart.out ? (bart.K * nb + bart.K + nb + 255) / 256 : 0;
-  if (nred + nbart)
-    hipLaunchKernelGGL(k_stats_reduce, dim3(nred + nbart), dim3(256), 0, s, partial, nblk, width, nbart, bart);
+// partial[0][q] = sum_b partial[b][q], in place
+__global__ void __launch_bounds__(256) k_partial_reduce(double* partial, int nblk, int width) {
+  const int q = blockIdx.x * kRedEntries + threadIdx.x;
+  const double t = strands_sum(partial, nblk, width, blockIdx.x * kRedEntries);
+  if (threadIdx.x < kRedEntries && q < width) partial[q] = t;
 }
 
 void launch_partial_reduce(double* partial, int nblk, int width, hipStream_t s) {
-  launch_reduce(partial, nblk, width, BartlettArgs(), s);
+  if (nblk > 1)
+    hipLaunchKernelGGL(k_partial_reduce, dim3((width + kRedEntries - 1) / kRedEntries), dim3(256), 0, s, partial, nblk,
+                       width);
+}
+
+// The statistics' partials summed into out = (sum (K), scatter (K x K)).  The
+// first nbart work-groups make the Normal-Wishart draw's random numbers
+// instead, which need no statistics.
+template <typename T, int NT>
+__global__ void __launch_bounds__(256) k_stats_reduce(const double* __restrict__ partial, int nblk, int K,
+                                                      double* __restrict__ out, int nbart, BartlettArgs bart) {
+  if ((int)blockIdx.x < nbart) {
+    bartlett_item(bart, blockIdx.x * 256 + threadIdx.x);
+    return;
+  }
+  constexpr int WIDTH = 16 * NT + 128 * NT * (NT + 1);
+  const int q0 = (blockIdx.x - nbart) * kRedEntries, c = threadIdx.x;
+  const double t = strands_sum(partial, nblk, WIDTH, q0);
+  if (c >= kRedEntries) return;
+  if (q0 < 16 * NT) {
+    const int k = stats_component<T, NT>(q0 / 16, c);
+    if (k < K) out[k] = t;
+    return;
+  }
+  const int id = (q0 - 16 * NT) / 256, r = (q0 - 16 * NT) % 256 / 16;
+  int ti = 0;
+  while ((ti + 1) * (ti + 2) / 2 <= id) ti++;
+  const int tj = id - ti * (ti + 1) / 2;
+  const int i = stats_component<T, NT>(ti, r), j = stats_component<T, NT>(tj, c);
+  if (i < K && j < K) {
+    out[K + i + j * K] = t;
+    if (ti != tj) out[K + j + i * K] = t;
+  }
 }
 
 template <typename T>
-static void launch_stats(const T* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
-                         hipStream_t s, const BartlettArgs& bart) {
-  const int KP = pad_latent(K);
+static void launch_stats(const T* U, const float* sub, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
+                         const BartlettArgs& bart) {
+  double* partial = ws + 2 * (K + K * K);
   const int cols = (N + nblk - 1) / nblk;
-  switch (KP) {
-#define MGPU_STATS_CASE(P)                                                                                   \
-  case P:                                                                                                    \
-    hipLaunchKernelGGL((k_hyper_stats<T, P>), dim3(nblk), dim3(StatShape<P>::THREADS), 0, s, U, sub, ld, N, K, \
-                       cols, partial);                                                                       \
+  const int nred = stats_width(K) / kRedEntries, nb = (bart.K + 3) / 4;
+  const int nbart = bart.out ? (bart.K * nb + bart.K + nb + 255) / 256 : 0;
+  switch (stats_tiles(K)) {
+#define MGPU_STATS_CASE(NT)                                                                                       \
+  case NT:                                                                                                        \
+    hipLaunchKernelGGL((k_hyper_stats<T, NT>), dim3(nblk), dim3(256), 0, s, U, sub, ld, N, K, cols, partial);     \
+    hipLaunchKernelGGL((k_stats_reduce<T, NT>), dim3(nred + nbart), dim3(256), 0, s, partial, nblk, K, ws, nbart, \
+                       bart);                                                                                     \
     break;
+    MGPU_STATS_CASE(1)
+    MGPU_STATS_CASE(2)
+    MGPU_STATS_CASE(4)
     MGPU_STATS_CASE(8)
-    MGPU_STATS_CASE(16)
-    MGPU_STATS_CASE(32)
-    MGPU_STATS_CASE(64)
-    MGPU_STATS_CASE(128)
 #undef MGPU_STATS_CASE
     default: break;
   }
-  launch_reduce(partial, nblk, K + K * K, bart, s);
 }
 
-void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
+void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* ws, int nblk,
                             hipStream_t s, const BartlettArgs& bart) {
-  launch_stats<float>(U, sub, ld, N, K, partial, nblk, s, bart);
+  launch_stats<float>(U, sub, ld, N, K, ws, nblk, s, bart);
 }
-void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s,
+void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
                             const BartlettArgs& bart) {
-  launch_stats<double>(U, nullptr, ld, N, K, partial, nblk, s, bart);
+  launch_stats<double>(U, nullptr, ld, N, K, ws, nblk, s, bart);
 }
 
 // ------------------------------------------------------------------

@@ -141,10 +141,14 @@ int batched_seg_grid(const BatchPlan& p);
 
 // --- hyperprior (FP64) ---
 // sums of x = U[:,n] - sub[:,n] (sub may be null): sum (K) and scatter
-// (K x K, col-major), accumulated per block into partial[nblk][K + K*K] and
-// reduced in place: the totals are in partial[0] when the launch completes.
-// hyper_stats_blocks(N) is the block count to allocate and pass.
-int hyper_stats_blocks(int N);
+// (K x K, col-major) in ws[0 .. K + K*K) when the launch completes.  ws has
+// hyper_stats_doubles(nblk, K) entries, nblk = hyper_stats_blocks(N, K) or
+// fewer: the sums, room for the draw's random numbers (hyper_stats_bart), the
+// blocks' partials.  FP32: ld = the padded latent size, U and sub aligned to 16
+// bytes.
+int hyper_stats_blocks(int N, int K);
+size_t hyper_stats_doubles(int nblk, int K);
+inline double* hyper_stats_bart(double* ws, int K) { return ws + K + K * K; }
 // The random numbers of a Normal-Wishart draw (see k_stats_reduce), made
 // beside the reduction when out is set; out has K + K*K entries
 struct BartlettArgs {
@@ -156,9 +160,9 @@ struct BartlettArgs {
   int iter_value = 0;  // the iteration when iter is null
   int mode = 0;
 };
-void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* partial, int nblk,
+void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* ws, int nblk,
                             hipStream_t s, const BartlettArgs& bart = BartlettArgs());
-void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* partial, int nblk, hipStream_t s,
+void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
                             const BartlettArgs& bart = BartlettArgs());
 
 struct NWArgs {

@@ -842,9 +842,8 @@ void ILatentPrior::init(Model& m, int mode) {
   upload(WI, WIh, m.stream);
   upload(Lambda_f, Lf, m.stream);
   upload(Lmu_f, Lmuf, m.stream);
-  stats_nblk = hyper_stats_blocks(m.dims[mode]);
-  // the blocks' partial sums, then the draw's random numbers
-  stats.alloc((size_t)(stats_nblk + 1) * (K + K * K) * sizeof(double));
+  stats_nblk = hyper_stats_blocks(m.dims[mode], K);
+  stats.alloc(hyper_stats_doubles(stats_nblk, K) * sizeof(double));
   HIPCHK(hipStreamSynchronize(m.stream));
 }
 
@@ -872,7 +871,7 @@ static NWArgs nw_args(Model& m, ILatentPrior& p, int mode, double nu) {
   a.K = m.num_latent;
   a.KP = m.KP;
   a.partial = p.stats.as<double>();
-  a.bart = p.stats.as<double>() + (size_t)p.stats_nblk * (a.K + a.K * a.K);
+  a.bart = hyper_stats_bart(p.stats.as<double>(), a.K);
   a.N = m.dims[mode];
   a.kappa = 2.0;  // b0 (latentprior.cpp:97)
   a.mu0 = p.mu0.as<double>();
@@ -1162,8 +1161,9 @@ void MacauPrior::init(Model& m, int mode) {
   Lchol.alloc((size_t)K * K * sizeof(double));
   tmp.alloc((size_t)K * N * sizeof(double));
   Fty.alloc(kf * sizeof(double));
-  bbt_nblk = hyper_stats_blocks(nfeat);
-  bbt.alloc((size_t)bbt_nblk * (K + K * K) * sizeof(double));
+  bbt_nblk = hyper_stats_blocks(nfeat, K);
+  bbt.alloc(hyper_stats_doubles(bbt_nblk, K) * sizeof(double));
+  HIPCHK(hipMemsetAsync(bbt.as<void>(), 0, (K + K * K) * sizeof(double), m.stream));  // beta = 0
   partial_sumsq.alloc(256 * sizeof(double));
   // block CG buffers sized for the largest block (<= 40 right-hand sides)
   cg.alloc(std::min(K, 40), nfeat, N);
@@ -1307,11 +1307,11 @@ int blockcg_device(const CsrDev& F0, const CsrDev& Ft0, const double* reg, const
 void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
   const int K = m.num_latent, KP = m.KP, N = nrow;
   hipStream_t s = m.stream;
-  // residual statistics of U - Uhat, and beta beta^T of the current beta
+  // residual statistics of U - Uhat; bbt holds beta beta^T of the current
+  // beta since the previous lambda_beta draw
   NWArgs a = nw_args(m, *this, mode, (double)K + (double)nfeat);  // df + beta.cols()
   launch_hyper_stats_f32(m.d_U[mode].as<float>(), Uhat.as<float>(), KP, N, K, stats.as<double>(), stats_nblk, s,
                          bartlett_of(a));
-  launch_hyper_stats_f64(beta.as<double>(), K, nfeat, K, bbt.as<double>(), bbt_nblk, s);
   a.BBt_partial = bbt.as<double>();
   a.lambda_beta = lambda_beta_d.as<double>();
   a.Lchol = Lchol.as<double>();

@@ -4,8 +4,8 @@
 // The same three kernels as macau_cond_normal_wishart (k_hyper_stats,
 // k_stats_reduce, k_nw_draw), launched asynchronously on the caller's stream.
 // Working memory (per GPU, held until the process ends):
-//   partial   (kNaBlocks - 1) x (K + K^2) FP64 statistics partials, then the
-//             draw's random numbers
+//   stats     the statistics, the draw's random numbers and up to kNaBlocks
+//             FP64 statistics partials (hyper_stats_doubles)
 //   Lambda_f  64 x 64 FP32 and Lmu_f 64 FP32 (the draw's sampler copies)
 // Its host address is never used: the device address of each GPU's copy is
 // taken once per device with hipGetSymbolAddress and used everywhere.
@@ -22,13 +22,14 @@ namespace mgpu {
 namespace {
 
 constexpr int kNaMaxK = 64;     // as the array is sized
-constexpr int kNaBlocks = 64;   // rows of partials: up to 63 statistics work-groups, and the random numbers
-constexpr size_t kNaPartial = (size_t)kNaBlocks * (kNaMaxK + kNaMaxK * kNaMaxK) * sizeof(double);
+constexpr int kNaBlocks = 256;  // statistics work-groups at most (one per CU)
+constexpr size_t kNaPartial =
+    ((size_t)2 * (kNaMaxK + kNaMaxK * kNaMaxK) + (size_t)kNaBlocks * (64 + 10 * 256)) * sizeof(double);
 constexpr size_t kNaLf = (size_t)kNaMaxK * kNaMaxK * sizeof(float);
 constexpr size_t kNaLmu = (size_t)kNaMaxK * sizeof(float);
 constexpr size_t kNaOffLf = kNaPartial;
 constexpr size_t kNaOffLmu = kNaOffLf + kNaLf;
-constexpr size_t kNaBytes = kNaOffLmu + kNaLmu + 256;  // 2,146,560 bytes
+constexpr size_t kNaBytes = kNaOffLmu + kNaLmu + 256;  // 5,457,408 bytes
 
 static_assert(kNaPartial % 256 == 0 && kNaLf % 256 == 0 && kNaLmu % 256 == 0, "sections stay 256-byte aligned");
 
@@ -70,13 +71,13 @@ void cond_normal_wishart_noalloc(int K, int N, const double* U, const double* mu
   if (!U || !mu0 || !T || !mu_out || !Lambda_out || !status)
     throw std::runtime_error("null device pointer");
   unsigned char* base = static_cast<unsigned char*>(scratch_on_current_device());
-  double* partial = reinterpret_cast<double*>(base);
-  const int nblk = std::min(hyper_stats_blocks(N), kNaBlocks - 1);
+  double* ws = reinterpret_cast<double*>(base);
+  const int nblk = std::min(hyper_stats_blocks(N, K), kNaBlocks);
   NWArgs a;
   a.K = K;
   a.KP = pad_latent(K);
-  a.partial = partial;
-  a.bart = partial + (size_t)nblk * (K + K * K);
+  a.partial = ws;
+  a.bart = hyper_stats_bart(ws, K);
   a.N = N;
   a.kappa = kappa;
   a.mu0 = mu0;
@@ -90,7 +91,7 @@ void cond_normal_wishart_noalloc(int K, int N, const double* U, const double* mu
   a.Lambda_f = reinterpret_cast<float*>(base + kNaOffLf);
   a.Lmu_f = reinterpret_cast<float*>(base + kNaOffLmu);
   a.status = status;
-  launch_hyper_stats_f64(U, K, N, K, partial, nblk, s, bartlett_of(a));
+  launch_hyper_stats_f64(U, K, N, K, ws, nblk, s, bartlett_of(a));
   launch_nw_draw(a, s);
   hip_check(hipGetLastError(), "allocation-free Normal-Wishart launch");
 }
