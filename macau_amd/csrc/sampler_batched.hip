@@ -521,11 +521,13 @@ __global__ void __launch_bounds__(64, 4) k_heavy32(SampleArgs a, BatchPlan p, in
 }
 
 int batched_light_grid(const BatchPlan& p) {
+  if (p.KP == 128) return batched128_light_grid(p);
   if (p.KP >= 64) return batched64_light_grid(p);  // one row per work-group
   const int cap = p.light_cap > 0 ? p.light_cap : kDefaultLightCap;
   return p.n_pair < cap ? p.n_pair : cap;
 }
 int batched_heavy_grid(const BatchPlan& p) {
+  if (p.KP == 128) return batched128_heavy_grid(p);
   if (p.KP >= 64) return batched64_heavy_grid(p);
   const int npairs = (p.n_heavy + 1) / 2;
   const int cap = p.heavy_cap > 0 ? p.heavy_cap : kDefaultHeavyCap;

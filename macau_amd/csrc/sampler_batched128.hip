@@ -1,448 +1,604 @@
 // sampler_batched128.hip -- the batched per-row sampler for K in (64, 128]:
-// split-BF16 MFMA Gram of a 128 x 128 precision matrix, one row per
-// 256-thread work-group.
+// split-BF16 MFMA Gram of a 128 x 128 precision matrix, one row per wave.
 //
 // Same mathematics as the K <= 64 samplers (sample_latent_blas,
-// latentprior.cpp:361-385): P = Lambda + alpha G, b = alpha c + Lambda mu,
-// u = L^{-T}(L^{-1} b + z); rows above the segment length are split into
-// segments whose partial Grams are summed in segment order; light rows are
-// taken by decreasing nnz.  What changes with K = 128:
-//   * Gram: per 16-nonzero chunk, wave w gathers components 32w..32w+31
-//     (lane l: component 32w + l%32 of the chunk's nonzeros 8(l/32)..+7,
-//     the MFMA operand layout of v_mfma_f32_32x32x16_bf16), splits them into
-//     BF16 hi + lo and stores them in LDS; the ten 32 x 32 blocks (I, J),
-//     I >= J, of G are then shared out, each block taking the operands of
-//     component blocks I and J from LDS (HiHi^T + HiLo^T + LoHi^T + LoLo^T):
-//       wave 0: (0,0) (1,0) (1,1)    wave 1: (2,0) (2,1) (2,2)
-//       wave 2: (3,0) (3,1)          wave 3: (3,2) (3,3)
-//     The chunk's gathers are issued before the previous chunk's MFMAs, and
-//     its index loads one chunk earlier still.
-//   * Epilogue: each wave keeps its blocks of -P in the accumulator layout
-//     and the matrix is factored in 4-column steps as the K = 64 epilogue
-//     does within one wave: the owners of the step's block column publish
-//     its 4 columns to LDS (double-buffered by step parity); lanes of waves
-//     0 and 1 own rows 0-63 and 64-127 and each forms the 4 x 4 diagonal
-//     factor, its own row of L, the forward solve and its multipliers, which
-//     go to LDS; after a second barrier every wave applies the rank-4
-//     update to its blocks that still hold unfactored columns on
-//     v_mfma_f32_32x32x2_f32, its operands read from LDS (at most 6 MFMAs
-//     per wave and step).  L is kept as a packed triangle in LDS (over the
-//     Gram operands' buffers, three work-groups per CU); wave 0
-//     does the back solve with two rows per lane (readlane broadcasts).
+// latentprior.cpp:361-385): P = Lambda + alpha G = L L^T, b = alpha c +
+// Lambda mu, u = L^{-T}(L^{-1} b + z); rows above the segment length are split
+// into segments whose partial Grams are summed in segment order; light rows are
+// taken by decreasing nnz.
+//
+// A wave holds the row's whole matrix: 36 tiles (16 x 16) of the upper
+// triangle (P = R^T R, R = L^T) in the accumulator layout of
+// v_mfma_f32_16x16x*: lane (g, n) = (l / 16, l % 16) has in register v the
+// entry of hardware row 4g + v, column n.  Component sigma(h) = 4 (h % 4) + h / 4
+// of a 16-block sits at hardware index h, so register v holds components 4v + g
+// of the rows: a register is then at once the operand (four consecutive rows)
+// of the product that these rows enter, and the factorisation and both solves
+// run on registers alone.  LDS holds only Lambda (one copy for the work-group's
+// eight waves, in tiles), a 1 KB transposition buffer per wave, and the normals.
+//   * Gram: per 32-nonzero chunk lane (g, n) gathers component sigma(n) of each
+//     block of nonzeros 8g .. 8g + 7, which is the operand layout of
+//     v_mfma_f32_16x16x32_bf16 (HiHi^T + HiLo^T + LoHi^T + LoLo^T per tile).
+//   * Factorisation by 16 columns: the diagonal tile gives L_kk^{-1} (see
+//     diag_factor), row k's tiles become R_kj = L_kk^{-1} P_kj and the rest
+//     P_ij -= R_ki^T R_kj.
+//   * Solves by 16 components: products of tiles and vectors, the sums over
+//     lanes taken once per block.
+//   * Component blocks beyond K are neither gathered, nor updated, nor solved.
 //   * No condition probes: refinement is not offered at this size.
+// Segments (k_seg128) share a segment's Gram between four waves through LDS.
+#include <algorithm>
 #include <stdexcept>
 
 #include "batched.h"
 
 namespace mgpu {
 
-constexpr int kPartial128 = 10 * 1024 + 256;  // floats per segment partial: 10 blocks + 4 x 64 RHS partials
+namespace {
+
 constexpr int kThreads128 = 256;
+constexpr int k128Grid = 512;                     // work-groups of the light- and heavy-row kernels
+constexpr int kTiles = 36;                        // 16 x 16 tiles of the upper triangle
+constexpr int kPartial128 = kTiles * 256 + 128;   // floats per segment partial: tiles and RHS sums
 
-// Gram blocks of each wave (block row, block column; -1: none)
-__constant__ int kBI128[4][3] = {{0, 1, 1}, {2, 2, 2}, {3, 3, -1}, {3, 3, -1}};
-__constant__ int kBJ128[4][3] = {{0, 0, 1}, {0, 1, 2}, {0, 1, -1}, {2, 3, -1}};
+__device__ __forceinline__ int sigma(int h) { return 4 * (h & 3) + (h >> 2); }
+__device__ __forceinline__ constexpr int slot(int i, int j) { return j * (j + 1) / 2 + i; }  // tile (i, j), i <= j
 
-struct Lds128 {
-  union {
-    uint4 op[2][4][64][2];    // Gram operands: [buffer][component block][lane][hi, lo]
-    float Lf[128 * 129 / 2];  // the epilogue's L, row i at i (i + 1) / 2 (the operands are dead by then)
-  } u;
-  float csh[128];           // RHS sums c (alpha c + Lambda mu is the RHS)
-  float WT[2][4][128];      // the step's columns of -P (double-buffered by step parity)
-  float Wb[2][128];         // the step's RHS values
-  float qsh[4][128];        // the step's multipliers of every row (zero at and above the block)
-  float hb[2][64];          // rows 64-127: b and 1 / L_ii, for the back solve on wave 0
-  float us[128];            // the sampled row (SSE)
-  float ws[64];             // rows 64-127: L^{-1} b + z (SSE)
-  double sse[2];
-};
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-struct Gram128 {
-  f32x16 g[3];  // this wave's blocks
-  float bp;     // RHS partial of component 32w + l%32 over this lane's half of each chunk
-};
-
-__device__ __forceinline__ void zero_gram(Gram128& g) {
-#pragma unroll
-  for (int b = 0; b < 3; b++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) g.g[b][r] = 0.f;
-  g.bp = 0.f;
-}
-
-// Gram stream over the nonzeros [beg, end) of one row (or segment); every
-// wave of the work-group runs it with the same range.
 template <int NO>
-__device__ __forceinline__ void gram128(const SampleArgs& a, const Factors<NO>& F, Lds128& s, int beg, int end,
-                                        Gram128& g) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5;
-  const int comp = 32 * w + (lane & 31);
-  const int nch = (end - beg + 15) >> 4;
-  const int I0 = kBI128[w][0], J0 = kBJ128[w][0], I1 = kBI128[w][1], J1 = kBJ128[w][1];
-  const int I2 = kBI128[w][2], J2 = kBJ128[w][2];
-  // indices and residual of nonzero e0 + lane, lanes 0..15 (index -1: none)
-  auto load_ix = [&](int e0, int (&ix)[NO], float& r) {
-    const int e = e0 + lane;
-    const bool ok = lane < 16 && e < end;
+struct Lds128 {               // of the segment kernel
+  uint4 op[2][8][64][2];      // Gram operands: [buffer][component block][lane][hi, lo]
+  i32x4 ix[4][NO][8];         // each wave's copy of the chunk's indices
+  f32x4 r[4][8];              // and residuals
+};
+
+__device__ __forceinline__ f32x4 mul_add(f32x4 a, f32x4 b, f32x4 c) {
 #pragma unroll
-    for (int t = 0; t < NO; t++) ix[t] = ok ? a.rows.idx[(size_t)e * NO + t] : -1;
-    r = ok ? a.rows.r[e] : 0.f;
-  };
-  // this lane's 8 values of the chunk (component comp of nonzeros 8h..8h+7)
-  auto gather = [&](const int (&ix)[NO], float (&v)[8]) {
+  for (int s = 0; s < 4; s++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
+  return c;
+}
+
+// sum over the 16 lanes of a row of lanes
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  return x + __builtin_bit_cast(
+                 float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float sum16(float x) {
+  x = dpp_add<0x128>(x);  // row_ror:8, 4, 2, 1
+  x = dpp_add<0x124>(x);
+  x = dpp_add<0x122>(x);
+  return dpp_add<0x121>(x);
+}
+// sum over the four rows of lanes
+__device__ __forceinline__ float sum_rows(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// The diagonal tile x = L L^T: the row operations that take it to L^T, from
+// the first rows down, take the identity to L^{-1}, which is returned.  Four
+// rows (one register) at a time: their 4 x 4 block is broadcast and factored by
+// every lane, the rows are multiplied by the block's inverse factor E, and the
+// rows below get their rank-4 update.  A pivot that is not positive raises bad
+// and is replaced by 1.
+__device__ __forceinline__ f32x4 diag_factor(f32x4 x, int lane, int& bad) {
+  const int g = lane >> 4, n = lane & 15;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 id;
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      float x = ld_factor<128>(F.rs[0], __shfl(ix[0], 8 * h + t, 64), comp);
+  for (int v = 0; v < 4; v++) id[v] = 4 * v + g == sigma(n) ? 1.f : 0.f;
 #pragma unroll
-      for (int o = 1; o < NO; o++) x *= ld_factor<128>(F.rs[o], __shfl(ix[o], 8 * h + t, 64), comp);
-      v[t] = x;
+  for (int v = 0; v < 4; v++) {
+    float m[4][4], rs[4], E[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int w = 0; w <= u; w++) {
+        m[u][w] = rdlane(x[v], 16 * u + 4 * w + v);
+        asm volatile("" : "+v"(m[u][w]));  // compares and selects stay on the vector unit
+      }
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+      const bool ok = m[p][p] > 0.f;
+      bad = ok ? bad : 1;
+      rs[p] = __builtin_amdgcn_rsqf(ok ? m[p][p] : 1.f);
+#pragma unroll
+      for (int i = p + 1; i < 4; i++) m[i][p] *= rs[p];
+#pragma unroll
+      for (int i = p + 1; i < 4; i++)
+#pragma unroll
+        for (int w = p + 1; w <= i; w++) m[i][w] = fmaf(-m[i][p], m[w][p], m[i][w]);
+      E[p][p] = rs[p];
+#pragma unroll
+      for (int q = 0; q < p; q++) {
+        float t = 0.f;
+#pragma unroll
+        for (int k = q; k < p; k++) t = fmaf(-m[p][k], E[k][q], t);
+        E[p][q] = t * rs[p];
+      }
     }
-  };
-  if (nch == 0) return;
-  int ixc[NO], ixn[NO];
-  float rc, rn;
-  float v[8];
-  load_ix(beg, ixc, rc);
-  gather(ixc, v);
-  load_ix(beg + 16, ixn, rn);
-  for (int c = 0; c < nch; c++) {
-    const int buf = c & 1;
+    float e = 0.f;  // left operand: E's row n / 4 at hardware row n = 0, 4, 8, 12
 #pragma unroll
-    for (int t = 0; t < 8; t++) g.bp += v[t] * __shfl(rc, 8 * h + t, 64);
-    bf16x8 hi, lo;
-    split8(v, hi, lo);
-    s.u.op[buf][w][lane][0] = __builtin_bit_cast(uint4, hi);
-    s.u.op[buf][w][lane][1] = __builtin_bit_cast(uint4, lo);
-    __syncthreads();
-    // the next chunk's gathers (and the one after's indices) before this
-    // chunk's MFMAs
-    float vn[8];
-    if (c + 1 < nch) {
-      gather(ixn, vn);
+    for (int p = 0; p < 4; p++)
 #pragma unroll
-      for (int t = 0; t < NO; t++) ixc[t] = ixn[t];
-      rc = rn;
-      load_ix(beg + 16 * (c + 2), ixn, rn);
+      for (int q = 0; q <= p; q++) e = (n == 4 * p && g == q) ? E[p][q] : e;
+    const float xn = __builtin_amdgcn_mfma_f32_16x16x4f32(e, x[v], zero, 0, 0, 0)[0];
+    id[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(e, id[v], zero, 0, 0, 0)[0];
+    if (v < 3) {
+      const float u = (n & 3) > v ? -xn : 0.f;  // the rows below
+      x = __builtin_amdgcn_mfma_f32_16x16x4f32(u, xn, x, 0, 0, 0);
+      id = __builtin_amdgcn_mfma_f32_16x16x4f32(u, id[v], id, 0, 0, 0);
     }
-    auto blk = [&](f32x16& acc, int I, int J) {
-      const bf16x8 ha = __builtin_bit_cast(bf16x8, s.u.op[buf][I][lane][0]);
-      const bf16x8 la = __builtin_bit_cast(bf16x8, s.u.op[buf][I][lane][1]);
-      const bf16x8 hb = __builtin_bit_cast(bf16x8, s.u.op[buf][J][lane][0]);
-      const bf16x8 lb = __builtin_bit_cast(bf16x8, s.u.op[buf][J][lane][1]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ha, hb, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ha, lb, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(la, hb, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(la, lb, acc, 0, 0, 0);
-    };
-    blk(g.g[0], I0, J0);
-    blk(g.g[1], I1, J1);
-    if (I2 >= 0) blk(g.g[2], I2, J2);
-    if (c + 1 < nch) {
+  }
+  return id;
+}
+
+// Gram stream over the nonzeros of one segment, shared by four waves: wave w
+// gathers component blocks 2w and 2w + 1 and splits them into LDS
+// (double-buffered, one barrier per chunk, the next chunk's gathers under this
+// chunk's products); the tiles are shared out by operand reuse: 10 + 10 of the
+// two diagonal quadrants, 8 + 8 of the third.
+template <int NO>
+struct Gram128 {
+  const SampleArgs& a;
+  const Factors<NO>& F;
+  Lds128<NO>& s;
+  const int nt, lane, w, g, cn;
+  int beg = 0, end = 0;
+  int ixr[NO];
+  float rr;
+  float v[2][8];  // component 32w + 16h + cn of the lane's nonzeros of the chunk
+
+  __device__ Gram128(const SampleArgs& a_, const Factors<NO>& F_, Lds128<NO>& s_, int nt_)
+      : a(a_), F(F_), s(s_), nt(nt_), lane(threadIdx.x & 63), w(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)),
+        g(lane >> 4), cn(sigma(lane & 15)) {
 #pragma unroll
-      for (int t = 0; t < 8; t++) v[t] = vn[t];
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[h][q] = 0.f;
+  }
+  // indices and residual of nonzero e0 + lane, lanes 0..31 (index -1: none)
+  __device__ __forceinline__ void load_ix(int e0) {
+    const int e = e0 + (lane & 31);
+    const bool ok = e < end;
+#pragma unroll
+    for (int t = 0; t < NO; t++) ixr[t] = ok ? a.rows.idx[(size_t)e * NO + t] : -1;
+    rr = ok ? a.rows.r[e] : 0.f;
+  }
+  // their copy in LDS, and the chunk's factor values on their way
+  __device__ __forceinline__ void gather() {
+    if (lane < 32) {
+#pragma unroll
+      for (int t = 0; t < NO; t++) reinterpret_cast<int*>(s.ix[w][t])[lane] = ixr[t];
+      reinterpret_cast<float*>(s.r[w])[lane] = rr;
     }
+    lds_wait();
+#pragma unroll
+    for (int t = 0; t < NO; t++) {
+      const i32x4 ix[2] = {s.ix[w][t][2 * g], s.ix[w][t][2 * g + 1]};
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        if (2 * w + h >= nt) continue;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          const float x = ld_factor<128>(F.rs[t], ix[q >> 2][q & 3], 32 * w + 16 * h + cn);
+          v[h][q] = t == 0 ? x : v[h][q] * x;
+        }
+      }
+    }
+  }
+  // the indices of [b, e)'s first chunk, then its values
+  __device__ __forceinline__ void open(int b, int e) {
+    beg = b;
+    end = e;
+    load_ix(beg);
+  }
+  __device__ __forceinline__ void start() {
+    gather();
+    load_ix(beg + 32);
+  }
+  // acc: the tiles of the wave's quarter (see gram_tiles), sums: the RHS sums
+  // of blocks 2w and 2w + 1, partial over the lane's nonzeros
+  __device__ __forceinline__ void run(f32x4 (&acc)[10], float (&sums)[2]) {
+#pragma unroll
+    for (int q = 0; q < 10; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    sums[0] = sums[1] = 0.f;
+    const int nch = (end - beg + 31) >> 5;
+    for (int c = 0; c < nch; c++) {
+      const int buf = c & 1;
+      {
+        const f32x4 r[2] = {s.r[w][2 * g], s.r[w][2 * g + 1]};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+          for (int q = 0; q < 8; q++) sums[h] += v[h][q] * r[q >> 2][q & 3];
+          bf16x8 hi, lo;
+          split8(v[h], hi, lo);
+          s.op[buf][2 * w + h][lane][0] = __builtin_bit_cast(uint4, hi);
+          s.op[buf][2 * w + h][lane][1] = __builtin_bit_cast(uint4, lo);
+        }
+      }
+      __syncthreads();
+      if (c + 1 < nch) {
+        gather();
+        load_ix(beg + 32 * (c + 2));
+      }
+      auto hi = [&](int I) { return __builtin_bit_cast(bf16x8, s.op[buf][I][lane][0]); };
+      auto lo = [&](int I) { return __builtin_bit_cast(bf16x8, s.op[buf][I][lane][1]); };
+      auto product = [&](f32x4& d, bf16x8 ha, bf16x8 la, bf16x8 hb, bf16x8 lb) {
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ha, hb, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ha, lb, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la, hb, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la, lb, d, 0, 0, 0);
+      };
+      // the wave's columns J, and its rows: the quadrant's diagonal (waves 0,
+      // 1) or rows 0-1 / 2-3 (waves 2, 3) against columns 4-7
+      const int J0 = w == 0 ? 0 : 4;
+      bf16x8 hb[4], lb[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        hb[j] = hi(J0 + j);
+        lb[j] = lo(J0 + j);
+      }
+      if (w < 2) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (J0 + j < nt) {
+#pragma unroll
+            for (int i = 0; i <= j; i++) product(acc[j * (j + 1) / 2 + i], hb[i], lb[i], hb[j], lb[j]);
+          }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const bf16x8 ha = hi(2 * (w - 2) + i), la = lo(2 * (w - 2) + i);
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            if (4 + j < nt) product(acc[4 * i + j], ha, la, hb[j], lb[j]);
+        }
+      }
+    }
+  }
+};
+
+// f(q, i, j) for the Gram tiles of wave w that hold components below 16 nt
+template <typename F>
+__device__ __forceinline__ void gram_tiles(int w, int nt, F&& f) {
+  if (w < 2) {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (4 * w + j < nt) {
+#pragma unroll
+        for (int i = 0; i <= j; i++) f(j * (j + 1) / 2 + i, 4 * w + i, 4 * w + j);
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (4 + j < nt) f(4 * i + j, 2 * (w - 2) + i, 4 + j);
   }
 }
 
-// The row's sample (and its share of the train SSE when sse_partial is set)
-// from the work-group's Gram state; returns the SSE share on thread 0.
-__device__ double finish128(const SampleArgs& a, int row, Gram128 g, int it, float alpha, Lds128& s) {
-  int lane = threadIdx.x & 63;
-  opaque(lane);
-  const int w = threadIdx.x >> 6, half = lane >> 5, c32 = lane & 31;
-  const bool active = row >= 0;
-  // RHS sums c of the 128 components
-  {
-    const float c = g.bp + __shfl_xor(g.bp, 32, 64);
-    if (lane < 32) s.csh[32 * w + lane] = c;
-  }
-  // each wave keeps its Gram blocks as -(Lambda + alpha G)
-  const int nb = w < 2 ? 3 : 2;
-  int BI[3], BJ[3];
+// What the waves of a light- or heavy-row work-group share.
+constexpr int kWaves128 = 8;
+template <int NO, int NT>
+struct Shared128 {
+  f32x4 lam[slot(0, NT)][64];            // Lambda, in tiles
+  struct Wave {
+    f32x4 t[64];                     // transposition of L_kk^{-1}
+    f32x4 v[8][4];                   // the normals, then u: [block][g], register v = component 4v + g
+    i32x4 ix[NO][8];                 // the chunk's indices
+    f32x4 r[8];                      // and residuals
+  } wave[kWaves128];
+};
+
+template <int NO, int NT>
+__device__ __forceinline__ void load_lambda(const SampleArgs& a, Shared128<NO, NT>& s) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int q = w; q < slot(0, NT); q += kWaves128) {
+    int j = 0;
+    while (slot(0, j + 1) <= q) j++;
+    const float* l = a.Lambda_f + (16 * (q - slot(0, j)) + (lane >> 4)) * 128 + 16 * j + sigma(lane & 15);
+    f32x4 x;
 #pragma unroll
-  for (int q = 0; q < 3; q++) {
-    BI[q] = kBI128[w][q];
-    BJ[q] = kBJ128[w][q];
-  }
-  f32x16 e[3];
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    e[q] = g.g[q];
-    if (q >= nb) continue;
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-      const float4 l4 =
-          *reinterpret_cast<const float4*>(a.Lambda_f + (32 * BJ[q] + c32) * 128 + 32 * BI[q] + 8 * m + 4 * half);
-      const float el[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-      for (int t = 0; t < 4; t++) e[q][4 * m + t] = -fmaf(alpha, e[q][4 * m + t], el[t]);
-    }
-  }
-  __syncthreads();  // csh complete
-  const int i = 64 * w + lane;  // this lane's row (waves 0 and 1)
-  const bool rl = w < 2;
-  float c = 0.f, b = 0.f, inv_diag = 1.f, zi = 0.f;
-  bool bad = false;
-  if (rl) {
-    c = s.csh[i];
-    b = alpha * c;
-    if (a.Lmu_rows) {
-      if (active) b += a.Lmu_rows[(size_t)row * 128 + i];
-    } else {
-      b += a.Lmu_f[i];
-    }
-    zi = i < a.K ? normal_f32(a.seed, (uint32_t)(active ? row : 0), (uint32_t)i, (uint32_t)it,
-                              make_tag(TAG_LATENT, a.mode))
-                 : 0.f;
-  }
-  const int tri_i = i * (i + 1) / 2;
-#pragma unroll 1
-  for (int k0 = 0; k0 < 128; k0 += 4) {
-    opaque(lane);
-    const int J0 = k0 >> 5, cc = k0 & 31, pb = (k0 >> 2) & 1;
-    // 1. publish columns k0..k0+3 of -P (the owners of block column J0) and
-    // the RHS
-    if ((unsigned)(c32 - cc) < 4u) {
-      const int u = c32 - cc;
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        if (q >= nb || BJ[q] != J0) continue;
-#pragma unroll
-        for (int m = 0; m < 4; m++)
-          *reinterpret_cast<float4*>(&s.WT[pb][u][32 * BI[q] + 8 * m + 4 * half]) =
-              make_float4(e[q][4 * m], e[q][4 * m + 1], e[q][4 * m + 2], e[q][4 * m + 3]);
-      }
-    }
-    if (rl) s.Wb[pb][i] = b;
-    __syncthreads();
-    // 2. the 4 x 4 diagonal factor, this row's entries of L and the forward
-    // solve; the rows' multipliers go to LDS for the update
-    if (rl) {
-      const float w0 = -s.WT[pb][0][i], w1 = -s.WT[pb][1][i], w2 = -s.WT[pb][2][i], w3 = -s.WT[pb][3][i];
-      const float4 c0 = *reinterpret_cast<const float4*>(&s.WT[pb][0][k0]);
-      const float4 c1 = *reinterpret_cast<const float4*>(&s.WT[pb][1][k0]);
-      const float4 c2 = *reinterpret_cast<const float4*>(&s.WT[pb][2][k0]);
-      const float4 c3 = *reinterpret_cast<const float4*>(&s.WT[pb][3][k0]);
-      const float4 bd = *reinterpret_cast<const float4*>(&s.Wb[pb][k0]);
-      const float a00 = -c0.x;
-      bool bp = !(a00 > 0.f);
-      const float r0 = __builtin_amdgcn_rsqf(bp ? 1.f : a00);
-      const float l10 = -c0.y * r0, l20 = -c0.z * r0, l30 = -c0.w * r0;
-      const float a11 = -c1.y - l10 * l10;
-      bp = bp || !(a11 > 0.f);
-      const float r1 = __builtin_amdgcn_rsqf(a11 > 0.f ? a11 : 1.f);
-      const float l21 = (-c1.z - l20 * l10) * r1, l31 = (-c1.w - l30 * l10) * r1;
-      const float a22 = -c2.z - l20 * l20 - l21 * l21;
-      bp = bp || !(a22 > 0.f);
-      const float r2 = __builtin_amdgcn_rsqf(a22 > 0.f ? a22 : 1.f);
-      const float l32 = (-c2.w - l30 * l20 - l31 * l21) * r2;
-      const float a33 = -c3.w - l30 * l30 - l31 * l31 - l32 * l32;
-      bp = bp || !(a33 > 0.f);
-      const float r3 = __builtin_amdgcn_rsqf(a33 > 0.f ? a33 : 1.f);
-      bad = bad || bp;
-      const float y0 = bd.x * r0;
-      const float y1 = (bd.y - l10 * y0) * r1;
-      const float y2 = (bd.z - l20 * y0 - l21 * y1) * r2;
-      const float y3 = (bd.w - l30 * y0 - l31 * y1 - l32 * y2) * r3;
-      const float p0 = w0 * r0;
-      const float p1 = (w1 - p0 * l10) * r1;
-      const float p2 = (w2 - p0 * l20 - p1 * l21) * r2;
-      const float p3 = (w3 - p0 * l30 - p1 * l31 - p2 * l32) * r3;
-      if (k0 <= i) {
-        float* lr = s.u.Lf + tri_i + k0;
-        lr[0] = p0;
-        if (k0 + 1 <= i) lr[1] = p1;
-        if (k0 + 2 <= i) lr[2] = p2;
-        if (k0 + 3 <= i) lr[3] = p3;
-      }
-      const int t = i - k0;
-      const bool inb = t >= 0 && t < 4, below = t >= 4;
-      const float yt = t == 0 ? y0 : (t == 1 ? y1 : (t == 2 ? y2 : y3));
-      const float rt = t == 0 ? r0 : (t == 1 ? r1 : (t == 2 ? r2 : r3));
-      b = inb ? yt : (below ? b - (p0 * y0 + p1 * y1 + p2 * y2 + p3 * y3) : b);
-      inv_diag = inb ? rt : inv_diag;
-      if (k0 + 4 < 128) {
-        s.qsh[0][i] = below ? p0 : 0.f;
-        s.qsh[1][i] = below ? p1 : 0.f;
-        s.qsh[2][i] = below ? p2 : 0.f;
-        s.qsh[3][i] = below ? p3 : 0.f;
-      }
-    }
-    if (k0 + 4 >= 128) break;
-    __syncthreads();
-    // 3. -P += p p^T over this wave's blocks that still hold unfactored
-    // columns; the MFMA operand of block row X on lane l is the multiplier
-    // l / 32 (or 2 + l / 32) of row 32 X + l % 32
-    const int jmin = (k0 + 4) >> 5;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-      if (q >= nb || BJ[q] < jmin) continue;
-      const float a01 = s.qsh[half][32 * BI[q] + c32], a23 = s.qsh[2 + half][32 * BI[q] + c32];
-      const float b01 = s.qsh[half][32 * BJ[q] + c32], b23 = s.qsh[2 + half][32 * BJ[q] + c32];
-      e[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a01, b01, e[q], 0, 0, 0);
-      e[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a23, b23, e[q], 0, 0, 0);
-    }
-  }
-  if (bad && active && i == 0) atomicMax(a.fail, row + 1);  // the pivots are the same on every row lane
-  b += zi;
-  const float wv = b;  // L^{-1} b + z
-  // back solve L^T u = w on wave 0, lane l holding rows l and 64 + l
-  if (w == 1) {
-    s.hb[0][lane] = b;
-    s.hb[1][lane] = inv_diag;
-    s.ws[lane] = wv;
+    for (int v = 0; v < 4; v++) x[v] = l[4 * v * 128];
+    s.lam[q][lane] = x;
   }
   __syncthreads();
-  double sse = 0.0;
-  if (w == 0) {
-    float bA = b, iA = inv_diag, bB = s.hb[0][lane], iB = s.hb[1][lane];
-    for (int gq = 127; gq >= 64; gq -= 8) {
-      opaque(lane);
-      float La[8], Lb[8];
+}
+
+// One wave: the Gram tiles of the nonzeros [beg, end) and the RHS sums c
+// (component 16 I + sigma(n) of block I, on every row of lanes).
+template <int NO, int NT>
+__device__ __forceinline__ void gram_row(const SampleArgs& a, const Factors<NO>& F, typename Shared128<NO, NT>::Wave& s,
+                                         int beg, int end, f32x4 (&P)[slot(0, NT)], float (&c)[NT]) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, cn = sigma(lane & 15);
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = gq - u;
-        La[u] = s.u.Lf[j * (j + 1) / 2 + lane];
-        Lb[u] = s.u.Lf[j * (j + 1) / 2 + ((64 + lane) <= j ? 64 + lane : j)];
-      }
+  for (int q = 0; q < slot(0, NT); q++) P[q] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = gq - u;
-        const float xj = rdlane(bB * iB, j - 64);
-        bA -= La[u] * xj;
-        bB = (64 + lane < j) ? bB - Lb[u] * xj : (64 + lane == j ? xj : bB);
-      }
+  for (int I = 0; I < NT; I++) c[I] = 0.f;
+  int ixr[NO];
+  float rr;
+  auto load_ix = [&](int e0) {
+    const int e = e0 + (lane & 31);
+    const bool ok = e < end;
+#pragma unroll
+    for (int t = 0; t < NO; t++) ixr[t] = ok ? a.rows.idx[(size_t)e * NO + t] : -1;
+    rr = ok ? a.rows.r[e] : 0.f;
+  };
+  load_ix(beg);
+  for (int e0 = beg; e0 < end; e0 += 32) {
+    if (lane < 32) {
+#pragma unroll
+      for (int t = 0; t < NO; t++) reinterpret_cast<int*>(s.ix[t])[lane] = ixr[t];
+      reinterpret_cast<float*>(s.r)[lane] = rr;
     }
-    for (int gq = 63; gq >= 0; gq -= 8) {
-      opaque(lane);
-      float La[8];
+    lds_wait();
+    i32x4 ix[NO][2];
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = gq - u;
-        La[u] = s.u.Lf[j * (j + 1) / 2 + (lane <= j ? lane : j)];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j = gq - u;
-        const float xj = rdlane(bA * iA, j);
-        bA = (lane < j) ? bA - La[u] * xj : (lane == j ? xj : bA);
-      }
+    for (int t = 0; t < NO; t++) {
+      ix[t][0] = s.ix[t][2 * g];
+      ix[t][1] = s.ix[t][2 * g + 1];
     }
-    if (active) {
-      a.U[(size_t)row * 128 + lane] = bA;
-      a.U[(size_t)row * 128 + 64 + lane] = bB;
-    }
-    if (a.sse_partial) {
-      s.us[lane] = bA;
-      s.us[64 + lane] = bB;
-      lds_wait();
-      // (w^2 - u Lambda u) / alpha - 2 u c per component, plus the row's
-      // sum of squared residuals
-      float t = 0.f;
+    const f32x4 r[2] = {s.r[2 * g], s.r[2 * g + 1]};
+    load_ix(e0 + 32);
+    bf16x8 hi[NT], lo[NT];
 #pragma unroll
-      for (int hh = 0; hh < 2; hh++) {
-        const int ci = 64 * hh + lane;
-        const float* Lrow = a.Lambda_f + ci * 128;
-        float lu = 0.f;
-#pragma unroll 8
-        for (int q = 0; q < 32; q++) {
-          const float4 u4 = *reinterpret_cast<const float4*>(&s.us[4 * q]);
-          const float4 l4 = *reinterpret_cast<const float4*>(Lrow + 4 * q);
-          lu += l4.x * u4.x + l4.y * u4.y + l4.z * u4.z + l4.w * u4.w;
-        }
-        const float ww = hh ? s.ws[lane] : wv;
-        const float uu = hh ? bB : bA;
-        const float cc = s.csh[ci];
-        t += (ww * ww - uu * lu) / alpha - 2.f * uu * cc;
+    for (int I = 0; I < NT; I++) {
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        v[q] = ld_factor<128>(F.rs[0], ix[0][q >> 2][q & 3], 16 * I + cn);
+#pragma unroll
+        for (int t = 1; t < NO; t++) v[q] *= ld_factor<128>(F.rs[t], ix[t][q >> 2][q & 3], 16 * I + cn);
+        c[I] = fmaf(v[q], r[q >> 2][q & 3], c[I]);
       }
-      if (active) {
-        if (lane == 0) t += a.r2[row];
-        sse = (double)t;
+      split8(v, hi[I], lo[I]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+#pragma unroll
+      for (int i = 0; i < NT; i++) {
+        if (i > j) continue;
+        f32x4& d = P[slot(i, j)];
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], hi[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], lo[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], hi[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], lo[j], d, 0, 0, 0);
       }
     }
   }
-  __syncthreads();  // the LDS of this row is dead for the next
+#pragma unroll
+  for (int I = 0; I < NT; I++) c[I] = sum_rows(c[I]);
+}
+
+// One wave: the row's sample from its Gram tiles and RHS sums; returns the
+// lane's share of the train SSE (when sse_partial is set).
+template <int NO, int NT>
+__device__ __forceinline__ double finish_row(const SampleArgs& a, int row, int it, float alpha, const f32x4 (*lam)[64],
+                                             typename Shared128<NO, NT>::Wave& s, f32x4 (&P)[slot(0, NT)],
+                                             const float (&c)[NT]) {
+  int lane = threadIdx.x & 63;
+  opaque(lane);
+  const int g = lane >> 4, n = lane & 15, cn = sigma(n);
+  int bad = 0;
+  // the normals: block B of four components on lane B
+  if (lane < 32) {
+    uint32_t w[4];
+    philox_at(a.seed, (uint32_t)row, (uint32_t)lane, (uint32_t)it, make_tag(TAG_LATENT, a.mode), w);
+    float z[4];
+    box_muller_f32(w[0], w[1], z[0], z[1]);
+    box_muller_f32(w[2], w[3], z[2], z[3]);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      reinterpret_cast<float*>(&s.v[lane >> 2][u])[lane & 3] = 4 * lane + u < a.K ? z[u] : 0.f;
+  }
+  float b[NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) {
+    const int i = 16 * k + cn;
+    b[k] = fmaf(alpha, c[k], a.Lmu_rows ? a.Lmu_rows[(size_t)row * 128 + i] : a.Lmu_f[i]);
+  }
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+      if (i > j) continue;
+      const f32x4 l = lam[slot(i, j)][lane];
+#pragma unroll
+      for (int v = 0; v < 4; v++) P[slot(i, j)][v] = fmaf(alpha, P[slot(i, j)][v], l[v]);
+    }
+  }
+  // factorisation, and the forward solve y_k = L_kk^{-1} (b_k - sum_i R_ik^T y_i):
+  // y_k in the rows' order (register v = component 4v + g), b's reductions
+  // held per row of lanes until their block comes
+  f32x4 y[NT];
+  float f[NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) f[k] = 0.f;
+#pragma unroll
+  for (int k = 0; k < NT; k++) {
+    // (the fences keep the compiler from stretching registers across steps)
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4 li = diag_factor(P[slot(k, k)], lane, bad);
+    __builtin_amdgcn_sched_barrier(0);
+    P[slot(k, k)] = li;
+    if (k + 1 < NT) {
+      s.t[lane] = li;
+      lds_wait();
+      f32x4 la;  // as left operand: L_kk^{-1}[component cn][4v + g]
+      const float* T = reinterpret_cast<const float*>(s.t);
+#pragma unroll
+      for (int v = 0; v < 4; v++) la[v] = T[4 * (16 * (cn & 3) + 4 * g + v) + (cn >> 2)];
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+        if (j > k) P[slot(k, j)] = mul_add(la, P[slot(k, j)], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int i = 0; i < NT; i++) {
+        if (i <= k) continue;
+        const f32x4 m = -P[slot(k, i)];
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          if (j >= i) P[slot(i, j)] = mul_add(m, P[slot(k, j)], P[slot(i, j)]);
+      }
+    }
+    const float t = b[k] - sum_rows(f[k]);
+#pragma unroll
+    for (int v = 0; v < 4; v++) y[k][v] = sum16(li[v] * t);
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      if (j <= k) continue;
+#pragma unroll
+      for (int v = 0; v < 4; v++) f[j] = fmaf(P[slot(k, j)][v], y[k][v], f[j]);
+    }
+  }
+  // u_k = L_kk^{-T} (y_k + z_k - sum_j>k R_kj u_j), from the last block up; the
+  // sums over the lanes of a row taken when their block comes
+  lds_wait();
+  f32x4 t[NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) t[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  double sse = 0.0;
+  float ww = 0.f, uc = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NT; kk++) {
+    const int k = NT - 1 - kk;
+    const f32x4 z = s.v[k][g];
+    float u = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const float x = y[k][v] + z[v];
+      ww = n == 0 ? fmaf(x, x, ww) : ww;
+      u = fmaf(P[slot(k, k)][v], x - sum16(t[k][v]), u);
+    }
+    u = sum_rows(u);
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (i < k) t[i][v] = fmaf(P[slot(i, k)][v], u, t[i][v]);
+    if (g == 0) {
+      a.U[(size_t)row * 128 + 16 * k + cn] = u;
+      uc = fmaf(u, c[k], uc);
+      if (a.sse_partial) reinterpret_cast<float*>(&s.v[k][cn & 3])[cn >> 2] = u;
+    }
+  }
+  for (int i = 16 * NT + lane; i < 128; i += 64) a.U[(size_t)row * 128 + i] = 0.f;
+  if (a.sse_partial) {
+    // u^T G u - 2 u c + sum r^2, with u^T G u = (|L^T u|^2 - u Lambda u) / alpha
+    lds_wait();
+    float q1 = 0.f, q2 = 0.f;  // diagonal and off-diagonal tiles
+    for (int j = 0; j < NT; j++) {
+      const float uj = reinterpret_cast<const float*>(&s.v[j][cn & 3])[cn >> 2];
+      for (int i = 0; i <= j; i++) {
+        const f32x4 l = lam[slot(i, j)][lane], ui = s.v[i][g];
+        const float x = (l[0] * ui[0] + l[1] * ui[1] + l[2] * ui[2] + l[3] * ui[3]) * uj;
+        if (i == j) q1 += x;
+        else q2 += x;
+      }
+    }
+    sse = ((double)ww - q1 - 2.0 * q2) / alpha - 2.0 * uc;
+    if (lane == 0) sse += a.r2[row];
+  }
+  lds_wait();
+  if (bad && lane == 0) atomicMax(a.fail, row + 1);
   return sse;
 }
 
-// work-group SSE sum into sse_partial[slot] (wave 0 holds the shares)
-__device__ inline void write_sse128(const SampleArgs& a, double acc, int slot) {
+// work-group sum of the lanes' SSE shares into sse_partial[at]
+template <int NO, int NT>
+__device__ void write_sse128(const SampleArgs& a, double acc, int at, Shared128<NO, NT>& s) {
   if (!a.sse_partial) return;
-  if (threadIdx.x < 64) {
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (threadIdx.x == 0) a.sse_partial[slot] = acc;
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+  __syncthreads();
+  double* red = reinterpret_cast<double*>(s.lam);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = red[0];
+    for (int q = 1; q < kWaves128; q++) t += red[q];
+    a.sse_partial[at] = t;
   }
 }
 
+// the RHS sums of the wave's blocks over the four rows of lanes
 template <int NO>
-__global__ void __launch_bounds__(kThreads128, 3) k_light128(SampleArgs a, BatchPlan p) {
-  __shared__ Lds128 s;
+__device__ __forceinline__ void store_sums(Lds128<NO>& s, float* out, int w, const float (&sums)[2]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const float c = sum_rows(sums[h]);
+    if (lane < 16) out[32 * w + 16 * h + sigma(lane)] = c;
+  }
+}
+
+template <int NO, int NT>
+__global__ void __launch_bounds__(64 * kWaves128) k_light128(SampleArgs a, BatchPlan p) {
+  __shared__ Shared128<NO, NT> s;
   const Factors<NO> F = make_factors<NO, 128>(a.others);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int it = *a.iter;
   const float alpha = (float)(*a.alpha);
+  load_lambda(a, s);
   double sse = 0.0;
-  for (int q = blockIdx.x; q < p.n_pair; q += gridDim.x) {
+  for (int q = blockIdx.x + gridDim.x * w; q < p.n_pair; q += gridDim.x * kWaves128) {
     const int4 rng = p.pair_rng[q];
-    const int row = p.pair_row[q].x;
-    Gram128 g;
-    zero_gram(g);
-    gram128<NO>(a, F, s, rng.x, rng.y, g);
-    sse += finish128(a, row, g, it, alpha, s);
+    f32x4 P[slot(0, NT)];
+    float c[NT];
+    gram_row<NO, NT>(a, F, s.wave[w], rng.x, rng.y, P, c);
+    sse += finish_row<NO, NT>(a, p.pair_row[q].x, it, alpha, s.lam, s.wave[w], P, c);
   }
-  write_sse128(a, sse, blockIdx.x);
+  write_sse128(a, sse, blockIdx.x, s);
 }
 
 template <int NO>
-__global__ void __launch_bounds__(kThreads128) k_seg128(SampleArgs a, BatchPlan p) {
-  __shared__ Lds128 s;
+__global__ void __launch_bounds__(kThreads128, 3) k_seg128(SampleArgs a, BatchPlan p) {
+  __shared__ Lds128<NO> s;
   const Factors<NO> F = make_factors<NO, 128>(a.others);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = (a.K + 15) / 16;
+  Gram128<NO> G(a, F, s, nt);
   for (int sg = blockIdx.x; sg < p.n_seg; sg += gridDim.x) {
-    Gram128 g;
-    zero_gram(g);
-    gram128<NO>(a, F, s, p.seg_beg[sg], p.seg_end[sg], g);
+    f32x4 acc[10];
+    float sums[2];
+    G.open(p.seg_beg[sg], p.seg_end[sg]);
+    G.start();
+    G.run(acc, sums);
     float* out = p.partial + (size_t)sg * kPartial128;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-      const int I = kBI128[w][q], J = kBJ128[w][q];
-      if (I < 0) continue;
-      const int t = I * (I + 1) / 2 + J;
-#pragma unroll
-      for (int r = 0; r < 16; r++) out[t * 1024 + r * 64 + lane] = g.g[q][r];
-    }
-    out[10240 + w * 64 + lane] = g.bp;
+    gram_tiles(w, nt, [&](int t, int i, int j) { *reinterpret_cast<f32x4*>(out + 256 * slot(i, j) + 4 * lane) = acc[t]; });
+    store_sums(s, out + 256 * kTiles, w, sums);
     __syncthreads();  // the operand buffers are reused by the next segment
   }
 }
 
-__global__ void __launch_bounds__(kThreads128, 3) k_heavy128(SampleArgs a, BatchPlan p, int sse_slot0) {
-  __shared__ Lds128 s;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+template <int NT>
+__global__ void __launch_bounds__(64 * kWaves128) k_heavy128(SampleArgs a, BatchPlan p, int sse_slot0) {
+  __shared__ Shared128<1, NT> s;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int it = *a.iter;
   const float alpha = (float)(*a.alpha);
+  load_lambda(a, s);
   double sse = 0.0;
-  for (int q = blockIdx.x; q < p.n_heavy; q += gridDim.x) {
+  for (int q = blockIdx.x + gridDim.x * w; q < p.n_heavy; q += gridDim.x * kWaves128) {
     // the slot's summed partial (k_seg_sum leaves it in the first segment)
     const float* in = p.partial + (size_t)p.heavy_seg0[q] * kPartial128;
-    Gram128 g;
-    zero_gram(g);
+    f32x4 P[slot(0, NT)];
+    float c[NT];
 #pragma unroll
-    for (int qq = 0; qq < 3; qq++) {
-      const int I = kBI128[w][qq], J = kBJ128[w][qq];
-      if (I < 0) continue;
-      const int t = I * (I + 1) / 2 + J;
+    for (int t = 0; t < slot(0, NT); t++) P[t] = *reinterpret_cast<const f32x4*>(in + 256 * t + 4 * lane);
 #pragma unroll
-      for (int r = 0; r < 16; r++) g.g[qq][r] = in[t * 1024 + r * 64 + lane];
-    }
-    g.bp = in[10240 + w * 64 + lane];
-    sse += finish128(a, p.heavy[q], g, it, alpha, s);
+    for (int I = 0; I < NT; I++) c[I] = in[256 * kTiles + 16 * I + sigma(lane & 15)];
+    sse += finish_row<1, NT>(a, p.heavy[q], it, alpha, s.lam, s.wave[w], P, c);
   }
-  write_sse128(a, sse, sse_slot0 + blockIdx.x);
+  write_sse128(a, sse, sse_slot0 + blockIdx.x, s);
 }
 
-template <int NO>
-static void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
+template <int NO, int NT>
+void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
   const int gl = batched_light_grid(p), gh = batched_heavy_grid(p);
   const bool fork = p.n_seg > 0 && seg.stream;
   if (p.n_seg > 0) {
@@ -450,19 +606,42 @@ static void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, 
     if (fork) seg_fork(s, seg);
     hipLaunchKernelGGL((k_seg128<NO>), dim3(batched_seg_grid(p)), dim3(kThreads128), 0, ss, a, p);
     launch_seg_sum<kPartial128>(p, ss);
-    if (gh > 0) hipLaunchKernelGGL(k_heavy128, dim3(gh), dim3(kThreads128), 0, ss, a, p, gl);
+    if (gh > 0) hipLaunchKernelGGL((k_heavy128<NT>), dim3(gh), dim3(64 * kWaves128), 0, ss, a, p, gl);
     if (fork) seg_record_join(seg);
   }
-  if (gl > 0) hipLaunchKernelGGL((k_light128<NO>), dim3(gl), dim3(kThreads128), 0, s, a, p);
+  if (gl > 0) hipLaunchKernelGGL((k_light128<NO, NT>), dim3(gl), dim3(64 * kWaves128), 0, s, a, p);
   if (fork) seg_wait_join(s, seg);
 }
 
+// one kernel per number of component blocks for matrices and 3-mode tensors
+// (at K = 70 five of eight blocks are 15 of 36 tiles); larger tensors take all
+// eight
+template <int NO>
+void launch128_k(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
+  if constexpr (NO <= 2) {
+    switch ((a.K + 15) / 16) {
+      case 5: return launch128_t<NO, 5>(a, p, s, seg);
+      case 6: return launch128_t<NO, 6>(a, p, s, seg);
+      case 7: return launch128_t<NO, 7>(a, p, s, seg);
+      default: break;
+    }
+  }
+  launch128_t<NO, 8>(a, p, s, seg);
+}
+
+}  // namespace
+
+// A work-group's waves take rows gridDim.x apart, so that few rows spread over
+// the CUs first
+int batched128_light_grid(const BatchPlan& p) { return std::min(p.n_pair, k128Grid); }
+int batched128_heavy_grid(const BatchPlan& p) { return std::min(p.n_heavy, k128Grid); }
+
 void launch_sample_batched128(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
   switch (a.rows.nother) {
-    case 1: return launch128_t<1>(a, p, s, seg);
-    case 2: return launch128_t<2>(a, p, s, seg);
-    case 3: return launch128_t<3>(a, p, s, seg);
-    case 4: return launch128_t<4>(a, p, s, seg);
+    case 1: return launch128_k<1>(a, p, s, seg);
+    case 2: return launch128_k<2>(a, p, s, seg);
+    case 3: return launch128_k<3>(a, p, s, seg);
+    case 4: return launch128_k<4>(a, p, s, seg);
     default: break;
   }
 }
