@@ -61,8 +61,8 @@ __host__ __device__ __forceinline__ constexpr int stats_component(int t, int c) 
 
 template <typename T, int NT>
 __global__ void __launch_bounds__(256)
-    k_hyper_stats(const T* __restrict__ U, const float* __restrict__ sub, int ld, int N, int K, int cols,
-                  double* __restrict__ partial) {
+    k_hyper_stats(const T* __restrict__ U, const float* __restrict__ sub, const int* __restrict__ skip, int ld, int N,
+                  int K, int cols, double* __restrict__ partial) {
   constexpr bool kShared = NT > 4;                      // the waves share the tiles
   constexpr int NTILE = NT * (NT + 1) / 2;
   constexpr int WIDTH = 16 * NT + 256 * NTILE;
@@ -82,7 +82,9 @@ __global__ void __launch_bounds__(256)
 
   T raw[AHEAD][NT];
   float rsub[AHEAD][NT];
-  auto load = [&](T(&x)[NT], float(&y)[NT], int col) {
+  int out_of[AHEAD];  // columns left out (FP64 input only)
+  auto load = [&](T(&x)[NT], float(&y)[NT], int& o, int col) {
+    o = sizeof(T) == 8 && skip ? skip[min(col, N - 1)] : -1;
     const size_t at = (size_t)min(col, N - 1) * ld;
     if constexpr (sizeof(T) == 4 && NT > 1) {  // ld = 16 NT: entries c NT .. c NT + NT - 1
       typedef float vec __attribute__((ext_vector_type(NT == 2 ? 2 : 4)));
@@ -109,21 +111,22 @@ __global__ void __launch_bounds__(256)
   };
   if (b0 < b1) {
 #pragma unroll
-    for (int u = 0; u < AHEAD; u++) load(raw[u], rsub[u], first + u * STEP);
+    for (int u = 0; u < AHEAD; u++) load(raw[u], rsub[u], out_of[u], first + u * STEP);
   }
   for (int n0 = first - g; n0 < b1; n0 += AHEAD * STEP) {
 #pragma unroll
     for (int u = 0; u < AHEAD; u++) {
       const int col = n0 + g + u * STEP;
+      const bool in = col < b1 && out_of[u] < 0;
       double x[NT];
 #pragma unroll
       for (int q = 0; q < NT; q++) {
         double v = (double)raw[u][q];
         if (sizeof(T) == 4) v -= (double)rsub[u][q];
-        x[q] = (col < b1 && stats_component<T, NT>(q, c) < K) ? v : 0.0;
+        x[q] = (in && stats_component<T, NT>(q, c) < K) ? v : 0.0;
         sum[q] += x[q];
       }
-      load(raw[u], rsub[u], col + AHEAD * STEP);
+      load(raw[u], rsub[u], out_of[u], col + AHEAD * STEP);
       if constexpr (!kShared) {
         int id = 0;
 #pragma unroll
@@ -309,7 +312,7 @@ __global__ void __launch_bounds__(256) k_stats_reduce(const double* __restrict__
 }
 
 template <typename T>
-static void launch_stats(const T* U, const float* sub, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
+static void launch_stats(const T* U, const float* sub, const int* skip, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
                          const BartlettArgs& bart) {
   double* partial = ws + 2 * (K + K * K);
   const int cols = (N + nblk - 1) / nblk;
@@ -318,7 +321,8 @@ static void launch_stats(const T* U, const float* sub, int ld, int N, int K, dou
   switch (stats_tiles(K)) {
 #define MGPU_STATS_CASE(NT)                                                                                       \
   case NT:                                                                                                        \
-    hipLaunchKernelGGL((k_hyper_stats<T, NT>), dim3(nblk), dim3(256), 0, s, U, sub, ld, N, K, cols, partial);     \
+    hipLaunchKernelGGL((k_hyper_stats<T, NT>), dim3(nblk), dim3(256), 0, s, U, sub, skip, ld, N, K, cols,      \
+                       partial);                                                                                  \
     hipLaunchKernelGGL((k_stats_reduce<T, NT>), dim3(nred + nbart), dim3(256), 0, s, partial, nblk, K, ws, nbart, \
                        bart);                                                                                     \
     break;
@@ -333,11 +337,11 @@ static void launch_stats(const T* U, const float* sub, int ld, int N, int K, dou
 
 void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* ws, int nblk,
                             hipStream_t s, const BartlettArgs& bart) {
-  launch_stats<float>(U, sub, ld, N, K, ws, nblk, s, bart);
+  launch_stats<float>(U, sub, nullptr, ld, N, K, ws, nblk, s, bart);
 }
 void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
-                            const BartlettArgs& bart) {
-  launch_stats<double>(U, nullptr, ld, N, K, ws, nblk, s, bart);
+                            const BartlettArgs& bart, const int* skip) {
+  launch_stats<double>(U, nullptr, skip, ld, N, K, ws, nblk, s, bart);
 }
 
 // ------------------------------------------------------------------

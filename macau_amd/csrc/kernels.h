@@ -164,8 +164,9 @@ struct BartlettArgs {
 };
 void launch_hyper_stats_f32(const float* U, const float* sub, int ld, int N, int K, double* ws, int nblk,
                             hipStream_t s, const BartlettArgs& bart = BartlettArgs());
+// (f64: columns n with skip[n] >= 0 are left out)
 void launch_hyper_stats_f64(const double* U, int ld, int N, int K, double* ws, int nblk, hipStream_t s,
-                            const BartlettArgs& bart = BartlettArgs());
+                            const BartlettArgs& bart = BartlettArgs(), const int* skip = nullptr);
 
 struct NWArgs {
   int K = 0, KP = 0;
@@ -374,6 +375,29 @@ void launch_dots(const double* a, const double* b, int nr, int n, double* partia
                  const double* skip = nullptr, bool reduce = true, const int* nxt = nullptr,
                  const double* reg = nullptr);
 
+// --- F's non-empty columns (gram.hip) ---
+constexpr int kGramMax = 4096, kGramMaxCg = 2048;
+struct GramPlan {
+  int n = 0, np = 0;            // non-empty columns (0: no plan), padded to 64
+  const int* idx = nullptr;     // n: their ids, ascending
+  const int* pos = nullptr;     // per column: its place among them, or -1
+  const double* G = nullptr;    // their Gram matrix (np x np, zero in the padding), or null
+};
+// G of a plan whose idx and pos are set (waits for it); compact: F's columns
+// are already numbered by their place
+void launch_gram(const CsrDev& F, bool compact, const GramPlan& g, double* G, hipStream_t s);
+// KP = G P on the first n of ntot features, + (*reg) P on all (ld = nr <= 32);
+// nothing when *skip != 0
+void launch_gram_mm(const GramPlan& g, int ntot, int nr, const double* P, const double* reg, double* KP,
+                    const double* skip, hipStream_t s);
+// compact right-hand side Bc (nr x (n + nr)) of B (nr x nfeat) and W (nr x nr)
+// from S = sum of b b^T over the empty columns; *bad = 1 when S is singular (W = 0)
+void launch_gram_begin(const GramPlan& g, const double* S, const double* B, int nr, double* Bc, double* W, double* bad,
+                       hipStream_t s);
+// X (nr x nfeat) from the compact solution; M: nr x nr scratch
+void launch_gram_end(const GramPlan& g, const double* Xc, const double* W, const double* bad, const double* reg,
+                     const double* B, int nfeat, int nr, double* M, double* X, hipStream_t s);
+
 struct CgState {
   int nr = 0, n = 0;
   double* X = nullptr;
@@ -406,6 +430,10 @@ struct BetaArgs {
   uint64_t seed = 0;
   const int* iter = nullptr;
   int mode = 0;
+  // launch_beta_noise_add: with pos, Fty is written as the noise plus column
+  // pos[f] of Ftc (0 where pos[f] < 0)
+  const double* Ftc = nullptr;
+  const int* pos = nullptr;
 };
 void launch_beta_tmp(const BetaArgs& a, double* tmp, hipStream_t s);
 void launch_beta_noise_add(const BetaArgs& a, double* Fty, hipStream_t s);
@@ -443,8 +471,14 @@ struct BetaUniArgs {
 };
 // Lambda <- diag(Lambda), Lambda_f <- its diagonal, Lmu_f = lambda mu
 void launch_uni_diag(int K, int KP, double* Lambda, float* Lambda_f, float* Lmu_f, const double* mu, hipStream_t s);
-// sample_beta: the per-latent feature sweeps
-void launch_beta_uni(const BetaUniArgs& a, hipStream_t s);
+// sample_beta: 1 / A and the scaled normals of every feature, and the update of
+// those with empty columns; then the per-latent sweeps over the others
+void launch_beta_uni_pre(const BetaUniArgs& a, hipStream_t s);
+void launch_beta_uni_sweep(const BetaUniArgs& a, hipStream_t s);
+// the same sweeps on a Gram plan (gram.hip): Z = U - mu - Uhat (K x N), then
+// the sweep from Fz = F^T Z (K x nfeat)
+void launch_uni_resid(const BetaUniArgs& a, double* Z, hipStream_t s);
+void launch_uni_sweep(const BetaUniArgs& a, const GramPlan& g, const double* Fz, hipStream_t s);
 // partial: lambda_beta_uni_partials(K) doubles of scratch
 int lambda_beta_uni_partials(int K);
 void launch_lambda_beta_uni(const BetaUniArgs& a, double* partial, hipStream_t s);

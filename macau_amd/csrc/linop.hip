@@ -1512,7 +1512,8 @@ __global__ void __launch_bounds__(256) k_beta_draw(BetaArgs a, double* out) {
       if (i < a.K) {
         const size_t q = (size_t)c * a.K + i;
         if (WHICH == 0) out[q] = (double)a.U[(size_t)c * a.KP + i] + x[s] - a.mu[i];
-        else out[q] += sl * x[s];
+        else if (!a.pos) out[q] += sl * x[s];
+        else out[q] = (a.pos[c] >= 0 ? a.Ftc[(size_t)a.pos[c] * a.K + i] : 0.0) + sl * x[s];
       }
     }
   }
@@ -1564,9 +1565,15 @@ __global__ void __launch_bounds__(256) k_beta_draw_t(BetaArgs a, double* out) {
       for (int i = 0; i < KP; i++)
         if (i < K) out[(size_t)c * K + i] = (double)u[i] + x[i] - a.mu[i];
     } else {
+      const double* src = out + (size_t)c * K;
+      bool some = true;
+      if (a.pos) {
+        some = a.pos[c] >= 0;
+        src = a.Ftc + (size_t)(some ? a.pos[c] : 0) * K;
+      }
 #pragma unroll
       for (int i = 0; i < KP; i++)
-        if (i < K) out[(size_t)c * K + i] += sl * x[i];
+        if (i < K) out[(size_t)c * K + i] = (some ? src[i] : 0.0) + sl * x[i];
     }
   }
 }

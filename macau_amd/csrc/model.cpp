@@ -914,7 +914,7 @@ static void build_csr(int nrow, const std::vector<int>& r, const std::vector<int
 
 MacauPrior::MacauPrior(int nr, int nc, const std::vector<int>& rows, const std::vector<int>& cols,
                        const std::vector<double>& vals, bool bin, double lb, double t)
-    : nrow(nr), nfeat(nc), lambda_beta0(lb), tol(t), binary(bin) {
+    : nrow(nr), nfeat(nc), lambda_beta0(lb), tol(t), binary(bin), nloc(nc) {
   for (size_t e = 0; e < rows.size(); e++)
     if (rows[e] < 0 || rows[e] >= nr || cols[e] < 0 || cols[e] >= nc)
       throw std::runtime_error("side information index out of range");
@@ -925,7 +925,7 @@ MacauPrior::MacauPrior(int nr, int nc, const std::vector<int>& rows, const std::
 CsrDev MacauPrior::F() const {
   CsrDev c = F_plan;
   c.nrow = nrow;
-  c.ncol = nfeat;
+  c.ncol = nloc;
   c.row_ptr = dF_rowptr.as<int>();
   c.cols = dF_cols.as<int>();
   c.vals = binary ? nullptr : dF_vals.as<double>();
@@ -933,7 +933,7 @@ CsrDev MacauPrior::F() const {
 }
 CsrDev MacauPrior::Ft() const {
   CsrDev c = Ft_plan;
-  c.nrow = nfeat;
+  c.nrow = nloc;
   c.ncol = nrow;
   c.row_ptr = dFt_rowptr.as<int>();
   c.cols = dFt_cols.as<int>();
@@ -1023,7 +1023,7 @@ void MacauPrior::build_dense(int nrmax, hipStream_t s) {
   const bool ones = binary || std::all_of(F_vals.begin(), F_vals.end(), [](double v) { return v == 1.0; });
   if (!ones || nrmax < 32) return;
   std::vector<int> cand;
-  for (int j = 0; j < nfeat; j++) {
+  for (int j = 0; j < nloc; j++) {
     const long c = Ft_rowptr[j + 1] - Ft_rowptr[j];
     if (c * 64 >= nrow && c > kSpmmSegNnz) cand.push_back(j);
   }
@@ -1035,7 +1035,7 @@ void MacauPrior::build_dense(int nrmax, hipStream_t s) {
   std::sort(cand.begin(), cand.end());
   const int nd = (int)cand.size(), ndp = (nd + 15) / 16 * 16;
   const int ndw = (ndp + 31) / 32, nrw = (nrow + 31) / 32;
-  std::vector<int> pos(nfeat, -1);
+  std::vector<int> pos(nloc, -1);
   for (int j = 0; j < nd; j++) pos[cand[j]] = j;
   std::vector<int> dcol(ndp, cand[0]);
   std::copy(cand.begin(), cand.end(), dcol.begin());
@@ -1082,12 +1082,12 @@ void MacauPrior::build_dense(int nrmax, hipStream_t s) {
   const int nkc = (nrow + kDenseRowChunk - 1) / kDenseRowChunk;
   // columns of F without nonzeros, none within kEmptyReach columns either
   // way: no work unit (the CG forms their KP rows as reg * P)
-  std::vector<int> nxt(nfeat + 1, nfeat);
-  for (int j = nfeat - 1; j >= 0; j--) nxt[j] = Ft_rowptr[j + 1] > Ft_rowptr[j] ? j : nxt[j + 1];
-  std::vector<char> omit(nfeat, 0);
+  std::vector<int> nxt(nloc + 1, nloc);
+  for (int j = nloc - 1; j >= 0; j--) nxt[j] = Ft_rowptr[j + 1] > Ft_rowptr[j] ? j : nxt[j + 1];
+  std::vector<char> omit(nloc, 0);
   {
     int prev = -(1 << 30);  // the last column with nonzeros before j
-    for (int j = 0; j < nfeat; j++) {
+    for (int j = 0; j < nloc; j++) {
       if (Ft_rowptr[j + 1] > Ft_rowptr[j]) {
         prev = j;
         continue;
@@ -1144,12 +1144,73 @@ void MacauPrior::upload_side(int nrmax, hipStream_t s) {
   build_dense(nrmax, s);
 }
 
+// When G pays.  Measured per iteration, without | with it (rows x non-empty
+// columns x entries a column), and the time to form G once:
+//   sweep, K = 16:  20000 x 64 x 20     0.44 | 0.18 ms, + 1 ms
+//                   20000 x 256 x 200   2.58 | 0.25,    + 3
+//                   15000 x 500 x 1000  1.59 | 0.32,    < 1
+//                   300000 x 2000 x 30  5.55 | 2.30,    + 35
+//                   300000 x 4000 x 30  7.46 | 7.01,    + 95
+//   K = 32:         2000 x 1000 x 3     0.30 | 0.52,    + 2
+//                   20000 x 2000 x 3    0.93 | 1.49,    + 3
+//                   20000 x 2000 x 100  15.1 | 1.50,    + 6
+//   block CG:       20000 x 256 x 200   0.96 | 0.67,    + 1 (K = 16)
+//                   20000 x 2000 x 3    0.97 | 1.02,    + 3 (K = 32)
+//                   300000 x 2000 x 30  1.79 | 1.51,    + 34 (K = 16)
+// The sweep walks a column's entries at 2.5 ns each from LDS, 70 ns from memory,
+// after 0.3 us; on G it takes 0.25 us a column and reads G at 4 TB/s.  Forming G
+// (29 fs a row and pair of columns) is to be won back in 20 iterations.
+static bool gram_for_sweep(double n, double rows, double entries) {
+  const double walk = 0.3 * n + (beta_uni_in_lds((int)rows) ? 0.0025 : 0.07) * entries;
+  return 0.25 * n + 0.25e-3 * n * n + rows * n * n * 2.9e-8 / 20 < walk;  // us
+}
+// Block CG: G is read once per CG iteration in place of the entries; at most
+// about 5 ms go into forming it.
+static bool gram_for_cg(double n, double rows, double entries) {
+  return n <= kGramMaxCg && n * n <= 128 * entries && rows * n * n <= 1.7e11;
+}
+
+// Empty columns from which the block CG replaces them (by at most 32 features)
+constexpr int kGramMinEmpty = 128;
+
 void MacauPrior::init(Model& m, int mode) {
   ILatentPrior::init(m, mode);
   if (nrow != m.dims[mode])
     throw std::runtime_error("side information rows must equal the size of its data mode");
   const int K = m.num_latent, KP = m.KP, N = nrow;
-  upload_side(std::max(K, 40), m.stream);
+  compact = !use_ftf && K <= 32 && list_columns(nfeat - kGramMinEmpty, m.stream);
+  nloc = compact ? gram.n + K : nfeat;
+  if (compact) {
+    // the same entries in the same order, columns numbered by their place
+    std::vector<int> cols(F_cols.size()), ptr;
+    std::vector<int> place(nfeat, 0);
+    ptr.reserve(nloc + 1);
+    for (int j = 0; j < nfeat; j++)
+      if (Ft_rowptr[j + 1] > Ft_rowptr[j]) {
+        place[j] = (int)ptr.size();
+        ptr.push_back(Ft_rowptr[j]);
+      }
+    ptr.resize(nloc + 1, Ft_rowptr[nfeat]);
+    for (size_t e = 0; e < cols.size(); e++) cols[e] = place[F_cols[e]];
+    std::swap(F_cols, cols);
+    std::swap(Ft_rowptr, ptr);
+    upload_side(std::max(K, 40), m.stream);
+    std::swap(F_cols, cols);
+    std::swap(Ft_rowptr, ptr);
+    if (gram_for_cg(gram.n, N, (double)F_cols.size())) build_gram(m.stream);
+    gram_nblk = hyper_stats_blocks(nfeat, K);
+    gram_stats.alloc(hyper_stats_doubles(gram_nblk, K) * sizeof(double));
+    gram_F.alloc((size_t)K * nloc * sizeof(double));
+    gram_B.alloc((size_t)K * nloc * sizeof(double));
+    gram_X.alloc((size_t)K * nloc * sizeof(double));
+    gram_W.alloc((size_t)K * K * sizeof(double));
+    gram_M.alloc((size_t)K * K * sizeof(double));
+    cg.alloc(K, nloc, gram.G ? 0 : N, std::min(512, (nloc + 63) / 64));
+  } else {
+    upload_side(std::max(K, 40), m.stream);
+    // block CG buffers sized for the largest block (<= 40 right-hand sides)
+    cg.alloc(std::min(K, 40), nfeat, N);
+  }
   const size_t kf = (size_t)K * nfeat;
   beta.alloc(kf * sizeof(double));
   HIPCHK(hipMemsetAsync(beta.as<void>(), 0, beta.bytes(), m.stream));
@@ -1165,8 +1226,6 @@ void MacauPrior::init(Model& m, int mode) {
   bbt.alloc(hyper_stats_doubles(bbt_nblk, K) * sizeof(double));
   HIPCHK(hipMemsetAsync(bbt.as<void>(), 0, (K + K * K) * sizeof(double), m.stream));  // beta = 0
   partial_sumsq.alloc(256 * sizeof(double));
-  // block CG buffers sized for the largest block (<= 40 right-hand sides)
-  cg.alloc(std::min(K, 40), nfeat, N);
   if (use_ftf) {  // FtF = At_mul_A(F) once (latentprior.cpp:199-203)
     const size_t nn = (size_t)nfeat * nfeat * sizeof(double);
     FtF.alloc(nn);
@@ -1192,21 +1251,80 @@ void MacauPrior::init(Model& m, int mode) {
   HIPCHK(hipStreamSynchronize(m.stream));
 }
 
-void CgBuffers::alloc(int nr, int nfeat, int nsamples) {
+void CgBuffers::alloc(int nr, int nfeat, int nsamples, int nb) {
   nrmax = nr;
+  nblk = nb > 0 ? nb : dots_blocks(nfeat);
   X.alloc((size_t)nr * nfeat * sizeof(double));
   R.alloc((size_t)nr * nfeat * sizeof(double));
   P.alloc((size_t)nr * nfeat * sizeof(double));
   KP.alloc((size_t)nr * nfeat * sizeof(double));
   B.alloc((size_t)nr * nfeat * sizeof(double));
   inner.alloc((size_t)nr * std::max(nsamples, 1) * sizeof(double));
-  partial.alloc((size_t)dots_blocks(nfeat) * nr * nr * sizeof(double));
-  small.alloc((size_t)(5 * nr * nr + nr + 4) * sizeof(double));
+  partial.alloc((size_t)nblk * nr * nr * sizeof(double));
+  small.alloc((size_t)(5 * nr * nr + nr + 5) * sizeof(double));  // see SmallView, and solve_compact
 }
 
 CgBuffers::~CgBuffers() {
   for (auto& c : chunks)
     if (c.exec) (void)hipGraphExecDestroy(c.exec);
+}
+
+// The CG iterations of state c, with the operator's products launched by
+// `products` (ops identifies them in the chunk graphs' key); flags receives
+// done, iterations and failure.
+template <typename Products>
+static void cg_iterate(const CgState& c, const double* reg, double tol, CgBuffers& b, hipStream_t s, bool use_graph,
+                       const std::vector<uintptr_t>& ops, Products&& products, double (&flags)[3]) {
+  const double tolsq = tol * tol;
+  const double* dflags = c.small + 5 * c.nr * c.nr + c.nr;
+  // a chunk of iterations per host round trip: the first one iteration
+  // shorter than the previous solve needed (8 without one), then 2 at a
+  // time; kernels of iterations after convergence return immediately
+  // (device-side done flag)
+  auto launch_chunk = [&](hipStream_t st, int len) {
+    for (int q = 0; q < len; q++) {
+      products(st, dflags);
+      launch_cg_step_a(c, st);
+      launch_cg_update_xr(c, st);
+      launch_cg_step_b(c, tolsq, st);
+      launch_cg_update_p(c, st);
+    }
+  };
+  std::vector<uintptr_t> key;
+  if (use_graph) {
+    double tolsq_bits = tolsq;
+    uintptr_t tb = 0;
+    std::memcpy(&tb, &tolsq_bits, sizeof(tb));
+    key = {(uintptr_t)reg, (uintptr_t)c.X, (uintptr_t)c.small, (uintptr_t)c.nr, tb};
+    key.insert(key.end(), ops.begin(), ops.end());
+  }
+  // the chunk's graph for this configuration and length, captured once
+  auto chunk_exec = [&](int len) -> hipGraphExec_t {
+    std::vector<uintptr_t> k = key;
+    k.push_back((uintptr_t)len);
+    for (auto& ch : b.chunks)
+      if (ch.key == k) return ch.exec;
+    hipGraph_t g = nullptr;
+    hipGraphExec_t exec = nullptr;
+    HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    launch_chunk(s, len);
+    HIPCHK(hipStreamEndCapture(s, &g));
+    HIPCHK(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
+    (void)hipGraphDestroy(g);
+    b.chunks.push_back({k, exec});
+    return exec;
+  };
+  int len = b.last_iters >= 8 ? b.last_iters - 1 : 8;
+  for (int it = 0; it < 100000; it += len, len = 2) {
+    if (use_graph)
+      HIPCHK(hipGraphLaunch(chunk_exec(len), s));
+    else
+      launch_chunk(s, len);
+    HIPCHK(hipMemcpyAsync(flags, dflags, sizeof(flags), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (flags[0] != 0.0) break;
+  }
+  b.last_iters = (int)flags[1];
 }
 
 int blockcg_device(const CsrDev& F0, const CsrDev& Ft0, const double* reg, const double* B, int ld, int r0, int nr,
@@ -1239,69 +1357,94 @@ int blockcg_device(const CsrDev& F0, const CsrDev& Ft0, const double* reg, const
     Bb = b.B.as<double>();
   }
   launch_cg_init(c, Bb, s);
-  const double tolsq = tol * tol;
-  double flags[3] = {0, 0, 0};
-  const double* dflags = c.small + 5 * nr * nr + nr;
-  // a chunk of iterations per host round trip: the first one iteration
-  // shorter than the previous solve needed (8 without one), then 2 at a
-  // time; kernels of iterations after convergence return immediately
-  // (device-side done flag)
-  auto launch_chunk = [&](hipStream_t st, int len) {
-    for (int q = 0; q < len; q++) {
-      launch_spmm(F, c.P, nr, c.inner, nullptr, nullptr, st, dflags);
-      launch_spmm(Ft, c.inner, nr, c.KPm, reg, c.P, st, dflags);
-      launch_cg_step_a(c, st);
-      launch_cg_update_xr(c, st);
-      launch_cg_step_b(c, tolsq, st);
-      launch_cg_update_p(c, st);
-    }
-  };
-  std::vector<uintptr_t> key;
-  if (use_graph) {
-    double tolsq_bits = tolsq;
-    uintptr_t tb = 0;
-    std::memcpy(&tb, &tolsq_bits, sizeof(tb));
-    key = {(uintptr_t)reg, (uintptr_t)c.X, (uintptr_t)c.small, (uintptr_t)nr, tb};
-    for (const CsrDev* A : {&F, &Ft}) {
-      const uintptr_t f[] = {(uintptr_t)A->nrow,       (uintptr_t)A->ncol,      (uintptr_t)A->row_ptr,
-                             (uintptr_t)A->cols,       (uintptr_t)A->vals,      (uintptr_t)A->nseg,
-                             (uintptr_t)A->seg,        (uintptr_t)A->nmulti,    (uintptr_t)A->multi_row,
-                             (uintptr_t)A->multi_slot0, (uintptr_t)A->partial,  (uintptr_t)A->dense_role,
-                             (uintptr_t)A->dcol,       (uintptr_t)A->row_bits,  (uintptr_t)A->col_bits};
-      key.insert(key.end(), std::begin(f), std::end(f));
-    }
+  std::vector<uintptr_t> ops;
+  for (const CsrDev* A : {&F, &Ft}) {
+    const uintptr_t f[] = {(uintptr_t)A->nrow,       (uintptr_t)A->ncol,      (uintptr_t)A->row_ptr,
+                           (uintptr_t)A->cols,       (uintptr_t)A->vals,      (uintptr_t)A->nseg,
+                           (uintptr_t)A->seg,        (uintptr_t)A->nmulti,    (uintptr_t)A->multi_row,
+                           (uintptr_t)A->multi_slot0, (uintptr_t)A->partial,  (uintptr_t)A->dense_role,
+                           (uintptr_t)A->dcol,       (uintptr_t)A->row_bits,  (uintptr_t)A->col_bits};
+    ops.insert(ops.end(), std::begin(f), std::end(f));
   }
-  // the chunk's graph for this configuration and length, captured once
-  auto chunk_exec = [&](int len) -> hipGraphExec_t {
-    std::vector<uintptr_t> k = key;
-    k.push_back((uintptr_t)len);
-    for (auto& ch : b.chunks)
-      if (ch.key == k) return ch.exec;
-    hipGraph_t g = nullptr;
-    hipGraphExec_t exec = nullptr;
-    HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    launch_chunk(s, len);
-    HIPCHK(hipStreamEndCapture(s, &g));
-    HIPCHK(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
-    (void)hipGraphDestroy(g);
-    b.chunks.push_back({k, exec});
-    return exec;
-  };
-  int len = b.last_iters >= 8 ? b.last_iters - 1 : 8;
-  for (int it = 0; it < 100000; it += len, len = 2) {
-    if (use_graph)
-      HIPCHK(hipGraphLaunch(chunk_exec(len), s));
-    else
-      launch_chunk(s, len);
-    HIPCHK(hipMemcpyAsync(flags, dflags, sizeof(flags), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    if (flags[0] != 0.0) break;
-  }
-  b.last_iters = (int)flags[1];
+  double flags[3];
+  cg_iterate(c, reg, tol, b, s, use_graph, ops,
+             [&](hipStream_t st, const double* dflags) {
+               launch_spmm(F, c.P, nr, c.inner, nullptr, nullptr, st, dflags);
+               launch_spmm(Ft, c.inner, nr, c.KPm, reg, c.P, st, dflags);
+             },
+             flags);
   if (flags[2] != 0.0) throw std::runtime_error("block CG: Cholesky of a small system failed");
   launch_cg_finish(c, s);
   if (nr != ld) launch_rows_copy(c.X, nr, X, ld, 0, r0, nr, nfeat, s);
   return (int)flags[1];
+}
+
+bool MacauPrior::list_columns(int most, hipStream_t s) {
+  gram = GramPlan();
+  std::vector<int> idx, pos(nfeat, -1);
+  for (int j = 0; j < nfeat; j++)
+    if (Ft_rowptr[j + 1] > Ft_rowptr[j]) {
+      pos[j] = (int)idx.size();
+      idx.push_back(j);
+    }
+  if (idx.empty() || (int)idx.size() > most) return false;
+  upload(gram_idx, idx, s);
+  upload(gram_pos, pos, s);
+  HIPCHK(hipStreamSynchronize(s));  // idx and pos go out of scope
+  gram.n = (int)idx.size();
+  gram.np = (gram.n + 63) / 64 * 64;
+  gram.idx = gram_idx.as<int>();
+  gram.pos = gram_pos.as<int>();
+  return true;
+}
+
+void MacauPrior::build_gram(hipStream_t s) {
+  gramG.alloc((size_t)gram.np * gram.np * sizeof(double));
+  launch_gram(F(), compact, gram, gramG.as<double>(), s);
+  gram.G = gramG.as<double>();
+}
+
+void MacauPrior::solve_compact(const double* B, double* X, bool use_graph, hipStream_t s) {
+  const int nr = cg.nrmax;
+  const CsrDev fd = Fd(), ftd = Ftd();
+  const bool dense = !gram.G && nr == 32 && fd.dense_role == 1 && ftd.dense_role == 2;
+  const CsrDev f = dense ? fd : F(), ft = dense ? ftd : Ft();
+  const double* reg = lambda_beta_d.as<double>();
+  CgState c;
+  c.nr = nr;
+  c.n = nloc;
+  c.X = gram_X.as<double>();
+  c.R = cg.R.as<double>();
+  c.P = cg.P.as<double>();
+  c.KPm = cg.KP.as<double>();
+  c.inner = cg.inner.as<double>();
+  c.partial = cg.partial.as<double>();
+  c.nblk = cg.nblk;
+  c.small = cg.small.as<double>();
+  if (dense) {
+    c.nxt = ft.next_nonempty;
+    c.reg = reg;
+  }
+  double* bad = c.small + 5 * nr * nr + nr + 4;  // after the CG's own flags
+  launch_hyper_stats_f64(B, nr, nfeat, nr, gram_stats.as<double>(), gram_nblk, s, BartlettArgs(), gram.pos);
+  launch_gram_begin(gram, gram_stats.as<double>() + nr, B, nr, gram_B.as<double>(), gram_W.as<double>(), bad, s);
+  launch_cg_init(c, gram_B.as<double>(), s);
+  double flags[3];
+  cg_iterate(c, reg, tol, cg, s, use_graph,
+             {(uintptr_t)gram.G, (uintptr_t)gram.n, (uintptr_t)f.seg, (uintptr_t)ft.seg, (uintptr_t)dense},
+             [&](hipStream_t st, const double* dflags) {
+               if (gram.G) {
+                 launch_gram_mm(gram, nloc, nr, c.P, reg, c.KPm, dflags, st);
+               } else {
+                 launch_spmm(f, c.P, nr, c.inner, nullptr, nullptr, st, dflags);
+                 launch_spmm(ft, c.inner, nr, c.KPm, reg, c.P, st, dflags);
+               }
+             },
+             flags);
+  if (flags[2] != 0.0) throw std::runtime_error("block CG: Cholesky of a small system failed");
+  launch_cg_finish(c, s);
+  launch_gram_end(gram, c.X, gram_W.as<double>(), bad, reg, B, nfeat, nr, gram_M.as<double>(), X, s);
+  last_cg_iters = (int)flags[1];
 }
 
 void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
@@ -1330,7 +1473,11 @@ void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
   b.iter = m.d_iter_prior.as<int>();
   b.mode = mode;
   launch_beta_tmp(b, tmp.as<double>(), s);
-  launch_spmm(Ft(), tmp.as<double>(), K, Fty.as<double>(), nullptr, nullptr, s);
+  launch_spmm(Ft(), tmp.as<double>(), K, compact ? gram_F.as<double>() : Fty.as<double>(), nullptr, nullptr, s);
+  if (compact) {
+    b.Ftc = gram_F.as<double>();
+    b.pos = gram.pos;
+  }
   launch_beta_noise_add(b, Fty.as<double>(), s);
   if (use_ftf && ftf_solver == kFtfSpectral) {
     // beta = Ft_y (FtF + lambda_beta I)^{-1} (latentprior.cpp:280-288)
@@ -1351,7 +1498,9 @@ void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
     // solve_blockcg(beta, F, lambda_beta, Ft_y, tol, 32, 8) (linop.h:206-226)
     const int blocksize = 32, excess = 8;
     const CsrDev fd = Fd(), ftd = Ftd();
-    if (K <= excess + blocksize) {
+    if (compact) {
+      solve_compact(Fty.as<double>(), beta.as<double>(), m.use_graph, s);
+    } else if (K <= excess + blocksize) {
       last_cg_iters = blockcg_device(F(), Ft(), lambda_beta_d.as<double>(), Fty.as<double>(), K, 0, K, tol,
                                      beta.as<double>(), cg, s, m.use_graph, &fd, &ftd);
     } else {
@@ -1364,8 +1513,8 @@ void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
     }
   }
   // compute_uhat and the per-row prior term for the next half-sweep
-  launch_uhat_finish(F(), beta.as<double>(), K, KP, mu.as<double>(), Lambda.as<double>(), Uhat.as<float>(),
-                     Lmu_rows.as<float>(), tmp.as<double>(), s);
+  launch_uhat_finish(F(), compact ? gram_X.as<double>() : beta.as<double>(), K, KP, mu.as<double>(),
+                     Lambda.as<double>(), Uhat.as<float>(), Lmu_rows.as<float>(), tmp.as<double>(), s);
   // lambda_beta = sample_lambda_beta(beta, Lambda, nu0, mu0)
   launch_hyper_stats_f64(beta.as<double>(), K, nfeat, K, bbt.as<double>(), bbt_nblk, s);
   launch_lambda_beta(K, (double)nfeat, bbt.as<double>(), 1, Lambda.as<double>(), lambda_beta_d.as<double>(),
@@ -1482,7 +1631,13 @@ void MacauOnePrior::init(Model& m, int mode) {  // macauoneprior.cpp:16-38
   upload(dbatch, batch_meta.empty() ? std::vector<int4>{make_int4(-1, 0, 0, 0)} : batch_meta, m.stream);
   ainv.alloc(std::max<size_t>(kf, 1) * sizeof(double));
   nz.alloc(std::max<size_t>(kf, 1) * sizeof(double));
-  Zw.alloc(beta_uni_in_lds(N) ? sizeof(double) : (size_t)K * N * sizeof(double));
+  if (list_columns(kGramMax, m.stream) && gram_for_sweep(gram.n, nrow, (double)F_cols.size())) {
+    build_gram(m.stream);
+    tmp.alloc(std::max<size_t>((size_t)K * N, 1) * sizeof(double));
+    Fty.alloc(std::max<size_t>(kf, 1) * sizeof(double));
+  } else {
+    Zw.alloc(beta_uni_in_lds(N) ? sizeof(double) : (size_t)K * N * sizeof(double));
+  }
   lb_partial.alloc((size_t)lambda_beta_uni_partials(K) * sizeof(double));
   partial_sumsq.alloc(256 * sizeof(double));
   HIPCHK(hipStreamSynchronize(m.stream));
@@ -1527,7 +1682,14 @@ void MacauOnePrior::update_prior(Model& m, int mode) {  // macauoneprior.cpp:189
   b.seed = m.seed;
   b.iter = m.d_iter_prior.as<int>();
   b.mode = mode;
-  launch_beta_uni(b, s);
+  launch_beta_uni_pre(b, s);
+  if (gram.G) {
+    launch_uni_resid(b, tmp.as<double>(), s);
+    launch_spmm(Ft(), tmp.as<double>(), K, Fty.as<double>(), nullptr, nullptr, s);
+    launch_uni_sweep(b, gram, Fty.as<double>(), s);
+  } else {
+    launch_beta_uni_sweep(b, s);
+  }
   // compute_uhat, with the per-row prior term lambda (mu + Uhat_n) for the
   // next half-sweep; the FP64 Uhat stays in uhat64 for the next sweep
   launch_uhat_finish(F(), beta.as<double>(), K, KP, mu.as<double>(), Lambda.as<double>(), Uhat.as<float>(),

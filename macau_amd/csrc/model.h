@@ -62,8 +62,9 @@ class Model;
 struct CgBuffers {
   DevBuf X, R, P, KP, B, inner, partial, small;
   int nrmax = 0;
+  int nblk = 0;        // partials of the dot products
   int last_iters = 0;  // iterations of the previous solve (sizes the first chunk)
-  void alloc(int nrmax, int nfeat, int nsamples);
+  void alloc(int nrmax, int nfeat, int nsamples, int nblk = 0);  // nblk 0: dots_blocks(nfeat)
   // instantiated graphs of a chunk of CG iterations, one per launch
   // configuration (the kernels' arguments: operators, buffers, regulariser,
   // tolerance) and chunk length
@@ -168,6 +169,18 @@ class MacauPrior : public ILatentPrior {
   void build_dense(int nrmax, hipStream_t s);
   CsrDev Fd_plan, Ftd_plan;
   std::vector<DevBuf> dense_bufs, Ftd_plan_bufs;
+  // columns of the device copy of F: nfeat, or the non-empty ones and K empty
+  // ones that stand for all others (compact)
+  int nloc;
+  bool compact = false;
+  // the list of F's non-empty columns, when there are at most `most`, and G
+  bool list_columns(int most, hipStream_t s);
+  void build_gram(hipStream_t s);
+  GramPlan gram;
+  DevBuf gram_idx, gram_pos, gramG, gram_stats, gram_F, gram_B, gram_X, gram_W, gram_M;
+  int gram_nblk = 0;
+  // beta from Ft_y by block CG on the compact columns
+  void solve_compact(const double* B, double* X, bool use_graph, hipStream_t s);
 };
 
 // MacauOnePrior<SparseDoubleFeat> (macauoneprior.h:8-51): diagonal prior

@@ -11,6 +11,10 @@
 //   compute_uhat (the shared SpMM);
 //   sample_lambda_beta: lambda_beta_d ~ Gamma(0.1 + nfeat / 2, 1 / (0.1 + |beta_d|^2 / 2)).
 //
+// When F has at most kGramMax non-empty columns the sweep runs on their Gram
+// matrix (gram.hip); the sweep below walks the columns' entries and takes any
+// number of them.
+//
 // The feature chain of a latent is sequential, so it runs on one wave with
 // z in LDS (rows up to kUniLdsRows; a global buffer beyond).  Features whose
 // columns share no row commute (updating one leaves every z entry the other
@@ -280,18 +284,20 @@ void launch_uni_diag(int K, int KP, double* Lambda, float* Lambda_f, float* Lmu_
 
 bool beta_uni_in_lds(int N) { return N <= kUniLdsRows; }
 
-void launch_beta_uni(const BetaUniArgs& a, hipStream_t s) {
-  if (a.K <= 0) return;
-  if (a.nfeat > 0) {
-    size_t tot = (size_t)a.K * a.nfeat;
-    size_t g = (tot + 255) / 256;
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(k_beta_uni_pre, dim3((unsigned)g), dim3(256), 0, s, a);
-    if (beta_uni_in_lds(a.N))
-      hipLaunchKernelGGL(k_beta_uni_sweep<true>, dim3(a.K), dim3(64), 0, s, a);
-    else
-      hipLaunchKernelGGL(k_beta_uni_sweep<false>, dim3(a.K), dim3(64), 0, s, a);
-  }
+void launch_beta_uni_pre(const BetaUniArgs& a, hipStream_t s) {
+  if (a.K <= 0 || a.nfeat <= 0) return;
+  size_t tot = (size_t)a.K * a.nfeat;
+  size_t g = (tot + 255) / 256;
+  if (g > 4096) g = 4096;
+  hipLaunchKernelGGL(k_beta_uni_pre, dim3((unsigned)g), dim3(256), 0, s, a);
+}
+
+void launch_beta_uni_sweep(const BetaUniArgs& a, hipStream_t s) {
+  if (a.K <= 0 || a.nfeat <= 0) return;
+  if (beta_uni_in_lds(a.N))
+    hipLaunchKernelGGL(k_beta_uni_sweep<true>, dim3(a.K), dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_beta_uni_sweep<false>, dim3(a.K), dim3(64), 0, s, a);
 }
 
 int lambda_beta_uni_partials(int K) { return kLbBlocks * K; }
