@@ -69,6 +69,21 @@ __device__ __forceinline__ void split8(const float* x, bf16x8& hi, bf16x8& lo) {
   lo = __builtin_bit_cast(bf16x8, l);
 }
 
+// x to 24 bits: hi + mid + lo
+__device__ __forceinline__ void split8(const float* x, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+  uint32_t h[4];
+  float d[8];
+#pragma unroll
+  for (int p = 0; p < 4; p++) {
+    h[p] = pack_bf16(x[2 * p], x[2 * p + 1]);
+    asm volatile("" : "+v"(h[p]));
+    d[2 * p] = x[2 * p] - __uint_as_float(h[p] << 16);
+    d[2 * p + 1] = x[2 * p + 1] - __uint_as_float(h[p] & 0xffff0000u);
+  }
+  hi = __builtin_bit_cast(bf16x8, h);
+  split8(d, mid, lo);
+}
+
 // nonzero e0 + lane of [e0, end) for the first BLK lanes (index -1 and
 // residual 0 past the end)
 template <int NO, int BLK>

@@ -49,7 +49,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 template <int NO>
 struct Lds128 {               // of the segment kernel
-  uint4 op[2][8][64][2];      // Gram operands: [buffer][component block][lane][hi, lo]
+  uint4 op[2][8][64][3];      // Gram operands: [buffer][component block][lane][hi, mid, lo]
   i32x4 ix[4][NO][8];         // each wave's copy of the chunk's indices
   f32x4 r[4][8];              // and residuals
 };
@@ -217,10 +217,10 @@ struct Gram128 {
         for (int h = 0; h < 2; h++) {
 #pragma unroll
           for (int q = 0; q < 8; q++) sums[h] += v[h][q] * r[q >> 2][q & 3];
-          bf16x8 hi, lo;
-          split8(v[h], hi, lo);
-          s.op[buf][2 * w + h][lane][0] = __builtin_bit_cast(uint4, hi);
-          s.op[buf][2 * w + h][lane][1] = __builtin_bit_cast(uint4, lo);
+          bf16x8 x[3];
+          split8(v[h], x[0], x[1], x[2]);
+#pragma unroll
+          for (int t = 0; t < 3; t++) s.op[buf][2 * w + h][lane][t] = __builtin_bit_cast(uint4, x[t]);
         }
       }
       __syncthreads();
@@ -228,37 +228,37 @@ struct Gram128 {
         gather();
         load_ix(beg + 32 * (c + 2));
       }
-      auto hi = [&](int I) { return __builtin_bit_cast(bf16x8, s.op[buf][I][lane][0]); };
-      auto lo = [&](int I) { return __builtin_bit_cast(bf16x8, s.op[buf][I][lane][1]); };
-      auto product = [&](f32x4& d, bf16x8 ha, bf16x8 la, bf16x8 hb, bf16x8 lb) {
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ha, hb, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ha, lb, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la, hb, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la, lb, d, 0, 0, 0);
+      auto op = [&](int I, bf16x8 (&x)[3]) {
+#pragma unroll
+        for (int t = 0; t < 3; t++) x[t] = __builtin_bit_cast(bf16x8, s.op[buf][I][lane][t]);
+      };
+      auto product = [&](f32x4& d, const bf16x8 (&x)[3], const bf16x8 (&y)[3]) {
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+#pragma unroll
+          for (int u = 0; u < 3 - t; u++) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t], y[u], d, 0, 0, 0);
       };
       // the wave's columns J, and its rows: the quadrant's diagonal (waves 0,
       // 1) or rows 0-1 / 2-3 (waves 2, 3) against columns 4-7
       const int J0 = w == 0 ? 0 : 4;
-      bf16x8 hb[4], lb[4];
+      bf16x8 y[4][3];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        hb[j] = hi(J0 + j);
-        lb[j] = lo(J0 + j);
-      }
+      for (int j = 0; j < 4; j++) op(J0 + j, y[j]);
       if (w < 2) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
           if (J0 + j < nt) {
 #pragma unroll
-            for (int i = 0; i <= j; i++) product(acc[j * (j + 1) / 2 + i], hb[i], lb[i], hb[j], lb[j]);
+            for (int i = 0; i <= j; i++) product(acc[j * (j + 1) / 2 + i], y[i], y[j]);
           }
       } else {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-          const bf16x8 ha = hi(2 * (w - 2) + i), la = lo(2 * (w - 2) + i);
+          bf16x8 x[3];
+          op(2 * (w - 2) + i, x);
 #pragma unroll
           for (int j = 0; j < 4; j++)
-            if (4 + j < nt) product(acc[4 * i + j], ha, la, hb[j], lb[j]);
+            if (4 + j < nt) product(acc[4 * i + j], x, y[j]);
         }
       }
     }
@@ -294,6 +294,7 @@ struct Shared128 {
     f32x4 v[8][4];                   // the normals, then u: [block][g], register v = component 4v + g
     i32x4 ix[NO][8];                 // the chunk's indices
     f32x4 r[8];                      // and residuals
+    uint4 lo[NT][64];                // and the factors' low parts
   } wave[kWaves128];
 };
 
@@ -347,7 +348,7 @@ __device__ __forceinline__ void gram_row(const SampleArgs& a, const Factors<NO>&
     }
     const f32x4 r[2] = {s.r[2 * g], s.r[2 * g + 1]};
     load_ix(e0 + 32);
-    bf16x8 hi[NT], lo[NT];
+    bf16x8 hi[NT], mid[NT];
 #pragma unroll
     for (int I = 0; I < NT; I++) {
       float v[8];
@@ -358,7 +359,9 @@ __device__ __forceinline__ void gram_row(const SampleArgs& a, const Factors<NO>&
         for (int t = 1; t < NO; t++) v[q] *= ld_factor<128>(F.rs[t], ix[t][q >> 2][q & 3], 16 * I + cn);
         c[I] = fmaf(v[q], r[q >> 2][q & 3], c[I]);
       }
-      split8(v, hi[I], lo[I]);
+      bf16x8 lo;
+      split8(v, hi[I], mid[I], lo);
+      s.lo[I][lane] = __builtin_bit_cast(uint4, lo);
     }
 #pragma unroll
     for (int j = 0; j < NT; j++) {
@@ -367,10 +370,20 @@ __device__ __forceinline__ void gram_row(const SampleArgs& a, const Factors<NO>&
         if (i > j) continue;
         f32x4& d = P[slot(i, j)];
         d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], hi[j], d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], lo[j], d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], hi[j], d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], lo[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], mid[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid[i], hi[j], d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid[i], mid[j], d, 0, 0, 0);
       }
+    }
+#pragma unroll
+    for (int k = 0; k < NT; k++) {
+      const bf16x8 lo = __builtin_bit_cast(bf16x8, s.lo[k][lane]);
+#pragma unroll
+      for (int i = 0; i <= k; i++)
+        P[slot(i, k)] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], lo, P[slot(i, k)], 0, 0, 0);
+#pragma unroll
+      for (int j = k; j < NT; j++)
+        P[slot(k, j)] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, hi[j], P[slot(k, j)], 0, 0, 0);
     }
   }
 #pragma unroll
@@ -557,7 +570,7 @@ __global__ void __launch_bounds__(64 * kWaves128) k_light128(SampleArgs a, Batch
 }
 
 template <int NO>
-__global__ void __launch_bounds__(kThreads128, 3) k_seg128(SampleArgs a, BatchPlan p) {
+__global__ void __launch_bounds__(kThreads128, 2) k_seg128(SampleArgs a, BatchPlan p) {
   __shared__ Lds128<NO> s;
   const Factors<NO> F = make_factors<NO, 128>(a.others);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = (a.K + 15) / 16;
