@@ -171,6 +171,10 @@ __device__ __forceinline__ float frag_diag(const f32x16& acc, int lane) {
 // direction of the factors) from reading as ill-conditioned.  LANES lanes
 // hold the row (32: a half of the wave; 64: the whole wave); each passes y_i
 // of the three probes and z_i (zero for i >= K).
+__device__ __forceinline__ float probe_value(int K, float s1, float s2, float s3, float zz) {
+  const float kk = (float)K;
+  return kk * fmaxf(fmaxf(s1 / fmaxf(zz, 1e-30f), s2 / kk), s3 / kk);
+}
 template <int LANES>
 __device__ __forceinline__ float probe_estimate(int K, float y1, float y2, float y3, float z) {
   float s1 = y1 * y1, s2 = y2 * y2, s3 = y3 * y3, zz = z * z;
@@ -181,8 +185,7 @@ __device__ __forceinline__ float probe_estimate(int K, float y1, float y2, float
     s3 += __shfl_xor(s3, off, 64);
     zz += __shfl_xor(zz, off, 64);
   }
-  const float kk = (float)K;
-  return kk * fmaxf(fmaxf(s1 / fmaxf(zz, 1e-30f), s2 / kk), s3 / kk);
+  return probe_value(K, s1, s2, s3, zz);
 }
 
 // The row's entry in the refinement queue when its estimate exceeds the

@@ -34,7 +34,7 @@ constexpr int kDefaultLightCap = 8192, kDefaultHeavyCap = 2048, kDefaultSegCap =
 constexpr int kMaxLightCap = 16384, kMaxHeavyCap = 4096;
 
 struct BatchPlan {
-  int KP = 0;                  // padded latent size the plan's partials are sized for
+  int K = 0, KP = 0;           // latent size, and padded: the plan's partials are sized for it
   int n_light = 0;             // light rows (sorted by nnz, descending)
   const int* light = nullptr;  // row ids
   int n_seg = 0;               // segments of heavy rows
@@ -46,7 +46,7 @@ struct BatchPlan {
   const int* heavy_seg0 = nullptr; // first segment of each heavy slot (n_heavy + 1)
   float* partial = nullptr;        // per-segment Gram (KP*KP) and rhs (KP)
   // light rows as the finishing kernel takes them: pairs of consecutive
-  // light rows (KP = 32) or single rows (KP = 64, row y = -1)
+  // light rows (KP = 32) or single rows (KP >= 64, row y = -1)
   int n_pair = 0;
   const int4* pair_rng = nullptr;  // nnz ranges [x, y) and [z, w) (z = w = 0: no second row)
   const int2* pair_row = nullptr;  // row ids (y = -1: no second row)
@@ -122,6 +122,10 @@ struct SegStreams {
   hipEvent_t fork = nullptr, join = nullptr;
 };
 void launch_sample_batched(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg = {});
+// K in (16, 32] (KP = 32): four rows per wave, 16 x 16 tiles
+void launch_sample_batched32(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg = {});
+int batched32_light_grid(const BatchPlan& p);
+int batched32_heavy_grid(const BatchPlan& p);
 // K in (32, 64] (KP = 64): one row per wave, three 32 x 32 Gram blocks
 void launch_sample_batched64(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg = {});
 // K in (64, 128] (KP = 128): one row per wave, 16 x 16 tiles; no refinement

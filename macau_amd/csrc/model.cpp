@@ -416,11 +416,12 @@ void Model::set_iteration(int it) {
   host_iter = it;
 }
 
-BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int KP, std::vector<DevBuf>& B, hipStream_t s,
+BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int K, std::vector<DevBuf>& B, hipStream_t s,
                            int seg_len) {
   const int N = (int)row_ptr.size() - 1;
   // rows sorted by nnz (descending); rows above the segment length are split
   // (default 2048: fewer, longer segments measured faster than 1024 and 512)
+  const int KP = pad_latent_batched(K);
   if (seg_len < 64 || seg_len % 64) throw std::runtime_error("segment length must be a positive multiple of 64");
   const int seg = seg_len;
   std::vector<int> order(N);
@@ -470,6 +471,7 @@ BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int KP, std::vector<
   // per segment: the KP x KP Gram fragment and one RHS partial per lane (64)
   B[6].alloc(std::max<size_t>(sb.size(), 1) * (size_t)(KP * KP + 64) * sizeof(float));
   BatchPlan p;
+  p.K = K;
   p.KP = KP;
   p.n_light = (int)light.size();
   p.light = B[0].as<int>();
@@ -499,7 +501,7 @@ void Model::build_plans() {
       throw std::runtime_error("batched sampler: unsupported latent size / mode count");
     if (!batched_fits(others_of(m), nmodes - 1, KP))
       throw std::runtime_error("batched sampler: a factor matrix exceeds 2^31 bytes");
-    plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, tune[m].seg_len);
+    plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, tune[m].seg_len);
     apply_plan_shape(m);
   }
 }

@@ -89,7 +89,7 @@ int blockcg_device(const CsrDev& F, const CsrDev& Ft, const double* reg, const d
 
 // Work list of the batched sampler for one mode (rows sorted by nnz,
 // heavy rows split into segments).
-BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int KP, std::vector<DevBuf>& bufs, hipStream_t s,
+BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int K, std::vector<DevBuf>& bufs, hipStream_t s,
                            int seg_len = kDefaultSegLen);
 
 // latentprior.h:17-49

@@ -1,5 +1,5 @@
 // sampler_batched.hip -- nnz-bucketed per-row sampler with a split-BF16
-// MFMA Gram (K in (16, 32]).
+// MFMA Gram for K <= 16, and the batched samplers' dispatch.
 //
 // Same mathematics as sample_latent_blas (latentprior.cpp:361-385) and
 // sample_latent_tensor (latentprior.cpp:118-161): per row
@@ -8,11 +8,11 @@
 //
 // Work decomposition of one half-sweep (BatchPlan, built on the host):
 //   * rows with more than 2048 nonzeros are split into 2048-nnz segments;
-//     k_seg32 computes each segment's partial Gram and RHS (one wave per
+//     k_seg16 computes each segment's partial Gram and RHS (one wave per
 //     segment), k_seg_sum adds each row's partials in segment order (one
-//     thread per partial entry), and k_heavy32 finishes two rows per wave;
+//     thread per partial entry), and k_heavy16 finishes two rows per wave;
 //   * the other rows, sorted by nnz (descending), are taken two per wave by
-//     k_light32 (similar nnz in a pair keeps both halves busy).
+//     k_light16 (similar nnz in a pair keeps both halves busy).
 // Gram: each MFMA step takes 16 nonzeros (lanes 0-31 the first 8, lanes
 // 32-63 the next 8; lane l holds component l%32), splits every value into
 // hi = bf16(x) and lo = bf16(x - hi), and accumulates G += Hi Hi^T + Hi Lo^T
@@ -67,10 +67,11 @@ bool batched_fits(const FactorSet& f, int nother, int KP) {
 // So each wave keeps the index loads of block k+2 and the BLK / 2 gathers of
 // block k+1 in flight while it multiplies block k.
 // ---------------------------------------------------------------------------
-// Block sizes: 32 nonzeros in the light-row kernel (its values in flight
-// take 16 registers per block, which keeps it at 4 waves per SIMD), 64 in the
-// segment kernel (few registers; more loads in flight per wave).
-constexpr int kBlkLight = 32, kBlkSeg = 64;
+// Block sizes: 64 nonzeros in the segment kernel and for few light rows (more
+// loads in flight per wave: 17.8 against 21.2 us at 2000 rows x 200 nonzeros,
+// 15.4 against 15.6 at 5000 x 80, K = 10), 32 for many (their values in flight
+// take 16 registers per block, which keeps the kernel at 4 waves per SIMD).
+constexpr int kBlkSeg = 64, kBlk64Pairs = 4096;
 
 template <int NO, int BLK>
 struct BlkLds {
@@ -204,11 +205,13 @@ struct PairLds {
 };
 
 // Finish two rows whose Gram fragments and RHS partials are in accA/accB,
+// taking ceil(K / 4) steps: what lies beyond is the identity (all 8 of the padded
+// matrix: 21.7 us at 5000 rows x 80 nonzeros, K = 10; the 3 needed: 15.6),
 // bpA/bpB (rowB < 0: no second row).  Returns this lane's SSE share.
 //
 // P = Lambda + alpha G stays in the MFMA accumulator layout (lane l, register
 // r holds entry (8(r/4) + 4(l/32) + r%4, l%32)), negated, for the whole
-// factorisation.  Right-looking Cholesky in 4-column blocks, k0 = 0, 4, .., 28:
+// factorisation.  Right-looking Cholesky in 4-column blocks, k0 = 0, 4, 8, 12:
 //   1. the lanes holding columns k0..k0+3 publish them to LDS; lane i of half
 //      h (row i of the pair's row h) reads its 4 entries, the 4 x 4 diagonal
 //      block and its RHS, factors the block redundantly (L_D, y_D), forms its
@@ -236,7 +239,7 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
   {
     const float* lc = a.Lambda_f + i * 32 + 4 * half;
 #pragma unroll
-    for (int m = 0; m < 4; m++) {
+    for (int m = 0; m < 2; m++) {
       const float4 l4 = *reinterpret_cast<const float4*>(lc + 8 * m);
       accA[4 * m] = -fmaf(alpha, accA[4 * m], l4.x);
       accA[4 * m + 1] = -fmaf(alpha, accA[4 * m + 1], l4.y);
@@ -275,13 +278,14 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
   const int tri_i = i * (i + 1) / 2;
   float* const Lh = s.Lf + half * kTri32;
 #pragma unroll
-  for (int k0 = 0; k0 < 32; k0 += 4) {
+  for (int k0 = 0; k0 < 16; k0 += 4) {
+    if (k0 >= a.K) continue;  // uniform
     opaque(i);
     // 1. publish columns k0..k0+3 of -P (lanes k0..k0+3 of both halves)
     const int m = k0 >> 3;
     if ((unsigned)(i - k0) < 4u) {
 #pragma unroll
-      for (int mm = 0; mm < 4; mm++) {
+      for (int mm = 0; mm < 2; mm++) {
         if (mm < m) continue;  // rows above the block row are not read
         *reinterpret_cast<float4*>(&s.WT[0][i - k0][8 * mm + 4 * half]) =
             make_float4(accA[4 * mm], accA[4 * mm + 1], accA[4 * mm + 2], accA[4 * mm + 3]);
@@ -336,7 +340,7 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
       if (k0 + 3 <= i) lr[3] = p3;
     }
     const int t = i - k0;
-    const bool inb = t >= 0 && t < 4, below = t >= 4;
+    const bool inb = t >= 0 && t < 4, below = t >= 4 && i < 16;  // rows 16 and beyond: the identity, not published
     const float yt = t == 0 ? y0 : (t == 1 ? y1 : (t == 2 ? y2 : y3));
     const float rt = t == 0 ? r0 : (t == 1 ? r1 : (t == 2 ? r2 : r3));
     b = inb ? yt : (below ? b - (p0 * y0 + p1 * y1 + p2 * y2 + p3 * y3) : b);
@@ -356,7 +360,7 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
       x3 = fwd(x3, *reinterpret_cast<const float4*>(&s.Wb[half][3][k0]));
     }
     // 2. -P += p p^T over the rows below the block, both matrices
-    if (k0 + 4 < 32) {
+    if (k0 + 4 < 16) {
       const float q0 = below ? p0 : 0.f, q1 = below ? p1 : 0.f, q2 = below ? p2 : 0.f, q3 = below ? p3 : 0.f;
       // swap(old, src): old's lanes 32-63 <-> src's lanes 0-31, so
       // .x = (q0 of A rows | q1 of A rows), .y = (q0 of B rows | q1 of B rows)
@@ -379,7 +383,8 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
   // readlane.  (For lanes i > j the read lands in later rows and is unused.)
   lds_wait();
 #pragma unroll
-  for (int g = 31; g >= 0; g -= 8) {
+  for (int g = 15; g >= 0; g -= 8) {
+    if (g - 7 >= a.K) continue;  // uniform
     opaque(i);
     float Lc[8];
 #pragma unroll
@@ -387,6 +392,7 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
 #pragma unroll
     for (int u = 0; u < 8; u++) {
       const int j = g - u;
+      if ((j & ~3) >= a.K) continue;  // steps not taken
       const float xl = b * inv_diag;  // final value on lane j
       const float xa = rdlane(xl, j), xb = rdlane(xl, 32 + j);
       const float xj = half ? xb : xa;
@@ -396,6 +402,9 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
   if (active) a.U[(size_t)row * 32 + i] = b;
   if (probe) {
     const float est = probe_estimate<32>(a.K, x1, x2, x3, zi);
+    if (i >= (a.K + 3) / 4 * 4)  // rows the steps did not reach: the identity
+      for (int k = 0; k <= i; k++) Lh[tri_i + k] = k == i ? 1.f : 0.f;
+    lds_wait();
     refine_enqueue<32, 32>(a, active ? row : -1, half ? nnzB : nnzA, i, half * 32, est, Lh + tri_i);
   }
   if (!a.sse_partial) return 0.f;
@@ -423,10 +432,10 @@ __device__ float finish_pair(const SampleArgs& a, int rowA, int rowB, f32x16 acc
 // ranges come from the plan in one load, and the next pair's ranges and its
 // first two index blocks are loaded while the current pair is multiplied and
 // finished, so a pair's stream starts with its indices already in registers.
-template <int NO>
-__global__ void __launch_bounds__(64, 4) k_light32(SampleArgs a, BatchPlan p) {
+template <int NO, int BLK>
+__global__ void __launch_bounds__(64, BLK == 64 ? 2 : 4) k_light16(SampleArgs a, BatchPlan p) {
   __shared__ PairLds s;
-  __shared__ BlkLds<NO, kBlkLight> blk;
+  __shared__ BlkLds<NO, BLK> blk;
   const Factors<NO> F = make_factors<NO, 32>(a.others);
   const int it = *a.iter;
   const float alpha = (float)(*a.alpha);
@@ -439,7 +448,7 @@ __global__ void __launch_bounds__(64, 4) k_light32(SampleArgs a, BatchPlan p) {
   if (q < p.n_pair) {
     rng = p.pair_rng[q];
     rows = p.pair_row[q];
-    GramStream<NO, true, kBlkLight>::first_blocks(a, rng, lane, b0, b1);
+    GramStream<NO, true, BLK>::first_blocks(a, rng, lane, b0, b1);
   }
   for (; q < p.n_pair; q += gridDim.x) {
     const int qn = q + gridDim.x;
@@ -456,8 +465,8 @@ __global__ void __launch_bounds__(64, 4) k_light32(SampleArgs a, BatchPlan p) {
       accB[r] = 0.f;
     }
     float bpA = 0.f, bpB = 0.f;
-    GramStream<NO, true, kBlkLight>(a, F, blk, rng.x, rng.y, rng.z, rng.w).run(b0, b1, accA, bpA, accB, bpB);
-    if (qn < p.n_pair) GramStream<NO, true, kBlkLight>::first_blocks(a, rng_n, lane, b0, b1);
+    GramStream<NO, true, BLK>(a, F, blk, rng.x, rng.y, rng.z, rng.w).run(b0, b1, accA, bpA, accB, bpB);
+    if (qn < p.n_pair) GramStream<NO, true, BLK>::first_blocks(a, rng_n, lane, b0, b1);
     sse += (double)finish_pair(a, rows.x, rows.y, accA, accB, bpA, bpB, it, alpha, s, rng.y - rng.x,
                                rng.w - rng.z);
     rng = rng_n;
@@ -467,7 +476,7 @@ __global__ void __launch_bounds__(64, 4) k_light32(SampleArgs a, BatchPlan p) {
 }
 
 template <int NO>
-__global__ void __launch_bounds__(64) k_seg32(SampleArgs a, BatchPlan p) {
+__global__ void __launch_bounds__(64) k_seg16(SampleArgs a, BatchPlan p) {
   __shared__ BlkLds<NO, kBlkSeg> blk;
   const Factors<NO> F = make_factors<NO, 32>(a.others);
   const int lane = threadIdx.x;
@@ -496,7 +505,7 @@ __device__ __forceinline__ void slot_partial(const BatchPlan& p, int slot, int l
   bp = in[1024 + lane];
 }
 
-__global__ void __launch_bounds__(64, 4) k_heavy32(SampleArgs a, BatchPlan p, int sse_slot0) {
+__global__ void __launch_bounds__(64, 4) k_heavy16(SampleArgs a, BatchPlan p, int sse_slot0) {
   __shared__ PairLds s;
   const int lane = threadIdx.x;
   const int it = *a.iter;
@@ -523,12 +532,14 @@ __global__ void __launch_bounds__(64, 4) k_heavy32(SampleArgs a, BatchPlan p, in
 int batched_light_grid(const BatchPlan& p) {
   if (p.KP == 128) return batched128_light_grid(p);
   if (p.KP >= 64) return batched64_light_grid(p);  // one row per work-group
+  if (p.K > 16) return batched32_light_grid(p);
   const int cap = p.light_cap > 0 ? p.light_cap : kDefaultLightCap;
   return p.n_pair < cap ? p.n_pair : cap;
 }
 int batched_heavy_grid(const BatchPlan& p) {
   if (p.KP == 128) return batched128_heavy_grid(p);
   if (p.KP >= 64) return batched64_heavy_grid(p);
+  if (p.K > 16) return batched32_heavy_grid(p);
   const int npairs = (p.n_heavy + 1) / 2;
   const int cap = p.heavy_cap > 0 ? p.heavy_cap : kDefaultHeavyCap;
   return npairs < cap ? npairs : cap;
@@ -546,14 +557,15 @@ static void launch_batched_t(const SampleArgs& a, const BatchPlan& p, hipStream_
     const hipStream_t ss = fork ? seg.stream : s;
     if (fork) seg_fork(s, seg);
     const int gs = batched_seg_grid(p);
-    hipLaunchKernelGGL((k_seg32<NO>), dim3(gs), dim3(64), 0, ss, a, p);
+    hipLaunchKernelGGL((k_seg16<NO>), dim3(gs), dim3(64), 0, ss, a, p);
     launch_seg_sum<kPartial>(p, ss);
     // the heavy rows depend only on their segments: finished on the segment
     // stream too, beside the light rows
-    if (gh > 0) hipLaunchKernelGGL(k_heavy32, dim3(gh), dim3(64), 0, ss, a, p, gl);
+    if (gh > 0) hipLaunchKernelGGL(k_heavy16, dim3(gh), dim3(64), 0, ss, a, p, gl);
     if (fork) seg_record_join(seg);
   }
-  if (gl > 0) hipLaunchKernelGGL((k_light32<NO>), dim3(gl), dim3(64), 0, s, a, p);
+  if (gl > 0 && p.n_pair <= kBlk64Pairs) hipLaunchKernelGGL((k_light16<NO, 64>), dim3(gl), dim3(64), 0, s, a, p);
+  else if (gl > 0) hipLaunchKernelGGL((k_light16<NO, 32>), dim3(gl), dim3(64), 0, s, a, p);
   if (fork) seg_wait_join(s, seg);
   launch_refine(a, s);
 }
@@ -565,6 +577,7 @@ void launch_sample_batched(const SampleArgs& a, const BatchPlan& p, hipStream_t 
     throw std::runtime_error("batched sampler: plan and latent size disagree or are unsupported");
   if (a.KP == 64) return launch_sample_batched64(a, p, s, seg);
   if (a.KP == 128) return launch_sample_batched128(a, p, s, seg);
+  if (a.K > 16) return launch_sample_batched32(a, p, s, seg);
   switch (a.rows.nother) {
     case 1: return launch_batched_t<1>(a, p, s, seg);
     case 2: return launch_batched_t<2>(a, p, s, seg);

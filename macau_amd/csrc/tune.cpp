@@ -163,11 +163,11 @@ std::vector<std::pair<double, double>> Model::autotune(int reps, const std::stri
     TuneChoice best = def;
     // the default shape, measured with the same repetitions as the candidates
     tune[m] = def;
-    plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, def.seg_len);
+    plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, def.seg_len);
     apply_plan_shape(m);
     double best_ms = time_mode(m, reps);
     for (int sl : seg_lens) {
-      plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, sl);
+      plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, sl);
       for (int lc : light_caps)
         for (int hc : heavy_caps)
           for (int sc : seg_caps) {
@@ -189,17 +189,17 @@ std::vector<std::pair<double, double>> Model::autotune(int reps, const std::stri
     // the candidate is more than 1% faster
     const int confirm = 4 * reps;
     tune[m] = def;
-    plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, def.seg_len);
+    plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, def.seg_len);
     apply_plan_shape(m);
     const double d_ms = time_mode(m, confirm);
     tune[m] = best;
-    plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, best.seg_len);
+    plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, best.seg_len);
     apply_plan_shape(m);
     const double b_ms = time_mode(m, confirm);
     if (!(b_ms < 0.99 * d_ms)) {
       best = def;
       tune[m] = def;
-      plans[m] = build_batch_plan(rows[m].row_ptr, KP, plan_bufs[m], stream, def.seg_len);
+      plans[m] = build_batch_plan(rows[m].row_ptr, num_latent, plan_bufs[m], stream, def.seg_len);
       apply_plan_shape(m);
     }
     tune[m].tuned = true;
