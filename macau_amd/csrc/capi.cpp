@@ -278,9 +278,7 @@ int macau_get_latents(macau_model* h, int mode, double* out) {
   API_BEGIN
   Model& m = M(h);
   if (mode < 0 || mode >= m.nmodes) throw std::runtime_error("mode out of range");
-  std::vector<double> U;
-  m.download_latents(mode, U);
-  memcpy(out, U.data(), U.size() * sizeof(double));
+  m.download_latents(mode, out);
   API_END_INT
 }
 int macau_get_hyper(macau_model* h, int mode, double* mu, double* Lambda) {

@@ -292,7 +292,7 @@ class Model {
   void iterate(int n);                 // n Gibbs iterations after init()
   void sync() { HIPCHK(hipStreamSynchronize(stream)); }
   void check_fail();
-  void download_latents(int mode, std::vector<double>& out);  // K x N col-major
+  void download_latents(int mode, double* out);  // K x N col-major
   double noise_precision();
   void set_iteration(int it);
   void capture_graph(bool on) { use_graph = on; }
@@ -324,7 +324,7 @@ class Model {
   std::vector<double> test_vals;
   long long ntest = 0;
   // device order of the test cells: device cell t is test cell test_perm[t]
-  std::vector<long long> test_perm;
+  std::vector<int> test_perm;
   // a per-test-cell device vector (d_pred, d_pred_var, ...) in the caller's order
   std::vector<double> test_to_host(const DevBuf& d);
 
