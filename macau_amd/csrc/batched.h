@@ -43,6 +43,20 @@ __device__ __forceinline__ float ld_factor(__amdgpu_buffer_rsrc_t rs, int ix, in
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, ix * (CS * 4) + comp * 4, 0, 0));
 }
 
+// The same in two parts, for several components of one column: the byte offset
+// of component comp, and the load `off` components further, which the opaque
+// offset puts into the instruction (one shift-add a column instead of one a
+// component; for ix = -1 the sum stays below 2^32, out of range).
+template <int CS>
+__device__ __forceinline__ int factor_at(int ix, int comp) {
+  int at = ix * (CS * 4) + comp * 4;
+  asm("" : "+v"(at));
+  return at;
+}
+__device__ __forceinline__ float ld_at(__amdgpu_buffer_rsrc_t rs, int at, int off) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at + 4 * off, 0, 0));
+}
+
 // x = hi + lo with hi = bf16(x) (round to nearest) and lo = bf16(x - hi),
 // eight values packed in the MFMA operand order (element 2p in the low half
 // of register p).  hi is converted once, packed (v_cvt_pk_bf16_f32), and

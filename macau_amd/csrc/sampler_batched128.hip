@@ -348,15 +348,20 @@ __device__ __forceinline__ void gram_row(const SampleArgs& a, const Factors<NO>&
     }
     const f32x4 r[2] = {s.r[2 * g], s.r[2 * g + 1]};
     load_ix(e0 + 32);
+    int at[NO][8];
+#pragma unroll
+    for (int t = 0; t < NO; t++)
+#pragma unroll
+      for (int q = 0; q < 8; q++) at[t][q] = factor_at<128>(ix[t][q >> 2][q & 3], cn);
     bf16x8 hi[NT], mid[NT];
 #pragma unroll
     for (int I = 0; I < NT; I++) {
       float v[8];
 #pragma unroll
       for (int q = 0; q < 8; q++) {
-        v[q] = ld_factor<128>(F.rs[0], ix[0][q >> 2][q & 3], 16 * I + cn);
+        v[q] = ld_at(F.rs[0], at[0][q], 16 * I);
 #pragma unroll
-        for (int t = 1; t < NO; t++) v[q] *= ld_factor<128>(F.rs[t], ix[t][q >> 2][q & 3], 16 * I + cn);
+        for (int t = 1; t < NO; t++) v[q] *= ld_at(F.rs[t], at[t][q], 16 * I);
         c[I] = fmaf(v[q], r[q >> 2][q & 3], c[I]);
       }
       bf16x8 lo;

@@ -30,7 +30,9 @@
 // row do alike (4 x 4 blocks, broadcasts) is done for four rows at once.  Two rows
 // a wave with 32 x 32 tiles took 538 us at 138000 rows x 133 nonzeros and 275 at
 // 27000 x 680 (17.7 MB of factors, read through the last-level cache), these
-// take 380 and 260.
+// take 353 and 230.  Bound by vector instructions (the split, the RHS, the
+// finish: about half of the time at two waves a SIMD) and the gathers' latency;
+// three waves a SIMD spill 21 registers and take 364 and 239.
 // Adaptive noise: for the last mode the train SSE of the new samples is
 // accumulated as u^T G u - 2 u^T c + sum r^2 per row, with
 // u^T G u = (|L^{-1} b + z|^2 - u^T Lambda u) / alpha (since L^T u = L^{-1} b + z),
@@ -178,14 +180,18 @@ struct QuadStream {
       ix[t][1] = *reinterpret_cast<const i32x4*>(&L.ix[buf][t][32 * c + 8 * g + 4]);
     }
 #pragma unroll
-    for (int h = 0; h < NT; h++)
+    for (int i = 0; i < 8; i++) {
+      int at[NO];
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        float x = ld_factor<32>(F.rs[0], ix[0][i >> 2][i & 3], n + 16 * h);
+      for (int t = 0; t < NO; t++) at[t] = factor_at<32>(ix[t][i >> 2][i & 3], n);
 #pragma unroll
-        for (int t = 1; t < NO; t++) x *= ld_factor<32>(F.rs[t], ix[t][i >> 2][i & 3], n + 16 * h);
+      for (int h = 0; h < NT; h++) {
+        float x = ld_at(F.rs[0], at[0], 16 * h);
+#pragma unroll
+        for (int t = 1; t < NO; t++) x *= ld_at(F.rs[t], at[t], 16 * h);
         v[c][h][i] = x;
       }
+    }
   }
   // chunk c of the current block (in v and buffer buf ^ 1) into T and cs, and
   // the gathers of the next block's chunk c (staged in buffer buf)
@@ -558,7 +564,7 @@ __device__ __forceinline__ float finish_quad(const SampleArgs& a, int4 rows, int
 // next rows' ranges and their first two index blocks are loaded while the
 // current ones are finished.
 template <int NO>
-__global__ void __launch_bounds__(64, NO == 1 ? 3 : 2) k_light32(SampleArgs a, BatchPlan p) {
+__global__ void __launch_bounds__(64, 2) k_light32(SampleArgs a, BatchPlan p) {
   __shared__ QuadLds<NO> S;
   const Factors<NO> F = make_factors<NO, 32>(a.others);
   const int it = *a.iter;
@@ -746,8 +752,8 @@ static int rows_per_group(const BatchPlan& p) {
 }
 
 // Four rows a wave: without a cap of the plan's, 16384 waves, which take the
-// rows in 2 strides at 138000 x 32 (372 us; 8192 waves 402, 3072 530: fewer
-// waves with more rows each end less evenly).
+// rows in 2 strides at 138000 x 32 (5% less time than 8192 waves, 30% less than
+// 3072: fewer waves with more rows each end less evenly).
 int batched32_light_grid(const BatchPlan& p) {
   const int r = rows_per_group(p), n = r ? (p.n_light + r - 1) / r : (p.n_pair + 1) / 2;
   const int cap = p.light_cap > 0 ? p.light_cap : 2 * kDefaultLightCap;
