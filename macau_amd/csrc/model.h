@@ -355,8 +355,8 @@ class Model {
   int host_iter = 0;  // iterations launched so far
   // iteration graphs: [0] without, [1] with the previous iteration's
   // deferred last-mode prior update at its start
-  hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
-  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t graph_exec[3] = {nullptr, nullptr, nullptr};
+  hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
   bool prior_pending = false;  // the last mode's prior update of the last launched iteration is deferred
   void drop_graphs();
 
