@@ -1108,7 +1108,9 @@ __global__ void __launch_bounds__(64) k_cg_step_a(const double* partial, int nbl
 // one launch instead of two.  The work-groups count themselves on the
 // spare flag (reset by k_cg_norms); the last one resets it.  Its release
 // fence writes back only the few partial sums this kernel wrote.
-template <int STEP>
+// A strand adds up to PER partials, all requested at once: 8 for at most 128 of
+// them (a compact solve's), 32 for 512.
+template <int STEP, int PER>
 __global__ void __launch_bounds__(256)
     k_cg_reduce_step(double* partial, int nblk, int nr, double* small, double tolsq) {
   constexpr int kStrands = 16, kEntries = 256 / kStrands;
@@ -1120,17 +1122,16 @@ __global__ void __launch_bounds__(256)
   __shared__ unsigned last;
   const int e = threadIdx.x % kEntries, g = threadIdx.x / kEntries;
   const int q = blockIdx.x * kEntries + e;
-  // a strand's (at most 512 / 16) partials loaded at once, at clamped
-  // addresses, and added in block order
-  constexpr int kPer = 512 / kStrands;
+  // a strand's partials loaded at once, at clamped addresses, and added in
+  // block order
   double acc = 0.0;
   {
     const int qc = min(q, width - 1);
-    double w[kPer];
+    double w[PER];
 #pragma unroll
-    for (int u = 0; u < kPer; u++) w[u] = partial[(size_t)min(g + kStrands * u, nblk - 1) * width + qc];
+    for (int u = 0; u < PER; u++) w[u] = partial[(size_t)min(g + kStrands * u, nblk - 1) * width + qc];
 #pragma unroll
-    for (int u = 0; u < kPer; u++)
+    for (int u = 0; u < PER; u++)
       if (g + kStrands * u < nblk) acc += w[u];
   }
   if (q >= width) acc = 0.0;
@@ -1422,10 +1423,10 @@ static bool fold_steps(const CgState& c) { return c.nblk > 1; }
 static void launch_reduce_step(const CgState& c, int step, double tolsq, hipStream_t s) {
   if (c.nblk > 512) throw std::logic_error("k_cg_reduce_step sums at most 512 partials");
   const dim3 grid((c.nr * c.nr + 15) / 16);
-  if (step == 0)
-    hipLaunchKernelGGL(k_cg_reduce_step<0>, grid, dim3(256), 0, s, c.partial, c.nblk, c.nr, c.small, tolsq);
-  else
-    hipLaunchKernelGGL(k_cg_reduce_step<1>, grid, dim3(256), 0, s, c.partial, c.nblk, c.nr, c.small, tolsq);
+  const bool few = c.nblk <= 128;
+  const auto kern = step == 0 ? (few ? k_cg_reduce_step<0, 8> : k_cg_reduce_step<0, 32>)
+                              : (few ? k_cg_reduce_step<1, 8> : k_cg_reduce_step<1, 32>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, c.partial, c.nblk, c.nr, c.small, tolsq);
 }
 
 void launch_cg_step_a(const CgState& c, hipStream_t s) {
