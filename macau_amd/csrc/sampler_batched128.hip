@@ -265,7 +265,7 @@ struct Gram128 {
   }
 };
 
-// f(q, i, j) for the Gram tiles of wave w that hold components below 16 nt
+// f(q, i, j) for the Gram tiles of wave w in the first nt component blocks
 template <typename F>
 __device__ __forceinline__ void gram_tiles(int w, int nt, F&& f) {
   if (w < 2) {
@@ -574,8 +574,10 @@ __global__ void __launch_bounds__(64 * kWaves128) k_light128(SampleArgs a, Batch
   write_sse128(a, sse, blockIdx.x, s);
 }
 
+// nb: the component blocks that the finishing kernel reads.  It may be compiled
+// for more than K has, so the tiles beyond (zero) are stored too.
 template <int NO>
-__global__ void __launch_bounds__(kThreads128, 2) k_seg128(SampleArgs a, BatchPlan p) {
+__global__ void __launch_bounds__(kThreads128, 2) k_seg128(SampleArgs a, BatchPlan p, int nb) {
   __shared__ Lds128<NO> s;
   const Factors<NO> F = make_factors<NO, 128>(a.others);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = (a.K + 15) / 16;
@@ -587,7 +589,7 @@ __global__ void __launch_bounds__(kThreads128, 2) k_seg128(SampleArgs a, BatchPl
     G.start();
     G.run(acc, sums);
     float* out = p.partial + (size_t)sg * kPartial128;
-    gram_tiles(w, nt, [&](int t, int i, int j) { *reinterpret_cast<f32x4*>(out + 256 * slot(i, j) + 4 * lane) = acc[t]; });
+    gram_tiles(w, nb, [&](int t, int i, int j) { *reinterpret_cast<f32x4*>(out + 256 * slot(i, j) + 4 * lane) = acc[t]; });
     store_sums(s, out + 256 * kTiles, w, sums);
     __syncthreads();  // the operand buffers are reused by the next segment
   }
@@ -622,7 +624,7 @@ void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const S
   if (p.n_seg > 0) {
     const hipStream_t ss = fork ? seg.stream : s;
     if (fork) seg_fork(s, seg);
-    hipLaunchKernelGGL((k_seg128<NO>), dim3(batched_seg_grid(p)), dim3(kThreads128), 0, ss, a, p);
+    hipLaunchKernelGGL((k_seg128<NO>), dim3(batched_seg_grid(p)), dim3(kThreads128), 0, ss, a, p, NT);
     launch_seg_sum<kPartial128>(p, ss);
     if (gh > 0) hipLaunchKernelGGL((k_heavy128<NT>), dim3(gh), dim3(64 * kWaves128), 0, ss, a, p, gl);
     if (fork) seg_record_join(seg);
