@@ -37,7 +37,7 @@ namespace mgpu {
 namespace {
 
 constexpr int kThreads128 = 256;
-constexpr int k128Grid = 512;                     // work-groups of the light- and heavy-row kernels
+constexpr int k128Grid = 256;                     // work-groups of the light- and heavy-row kernels: one a CU
 constexpr int kTiles = 36;                        // 16 x 16 tiles of the upper triangle
 constexpr int kPartial128 = kTiles * 256 + 128;   // floats per segment partial: tiles and RHS sums
 
@@ -574,6 +574,66 @@ __global__ void __launch_bounds__(64 * kWaves128) k_light128(SampleArgs a, Batch
   write_sse128(a, sse, blockIdx.x, s);
 }
 
+// The same for fewer rows than the chip holds waves: S waves (2, 4 or 8) take a
+// share of a row's nonzeros each, and one of them, in turn, finishes the row
+// while the others go on to the next.  Their tiles are added through the LDS
+// that holds the factors' low parts, NT tiles at a time: each of the S waves adds
+// its share of those tiles, in the order of the waves.
+template <int NO, int NT>
+__global__ void __launch_bounds__(64 * kWaves128) k_light128w(SampleArgs a, BatchPlan p, int S) {
+  __shared__ Shared128<NO, NT> s;
+  const Factors<NO> F = make_factors<NO, 128>(a.others);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int it = *a.iter;
+  const float alpha = (float)(*a.alpha);
+  load_lambda(a, s);
+  const int R = kWaves128 / S, u = w % R, part = w / R;  // rows a turn; the wave's row and share
+  double sse = 0.0;
+  int turn = 0;
+  for (int q0 = blockIdx.x; q0 < p.n_pair; q0 += gridDim.x * R, turn++) {
+    const int q = q0 + gridDim.x * u;
+    const int4 rng = q < p.n_pair ? p.pair_rng[q] : make_int4(0, 0, 0, 0);
+    const int share = (rng.y - rng.x + 32 * S - 1) / (32 * S) * 32;
+    const int b = min(rng.x + part * share, rng.y);
+    f32x4 P[slot(0, NT)];
+    float c[NT];
+    gram_row<NO, NT>(a, F, s.wave[w], b, min(b + share, rng.y), P, c);
+    const int f = turn % S;  // the share whose wave finishes
+    if (lane < 16) {
+#pragma unroll
+      for (int I = 0; I < NT; I++) reinterpret_cast<float*>(s.wave[w].t)[16 * I + lane] = c[I];
+    }
+#pragma unroll
+    for (int t0 = 0; t0 < slot(0, NT); t0 += NT) {
+#pragma unroll
+      for (int k = 0; k < NT; k++)
+        if (t0 + k < slot(0, NT)) s.wave[w].lo[k][lane] = __builtin_bit_cast(uint4, P[t0 + k]);
+      __syncthreads();
+      for (int k = part; k < NT && t0 + k < slot(0, NT); k += S) {
+        f32x4 x = __builtin_bit_cast(f32x4, s.wave[u].lo[k][lane]);
+        for (int m = 1; m < S; m++) x += __builtin_bit_cast(f32x4, s.wave[m * R + u].lo[k][lane]);
+        s.wave[f * R + u].lo[k][lane] = __builtin_bit_cast(uint4, x);
+      }
+      if (t0 == 0 && part == f) {
+#pragma unroll
+        for (int I = 0; I < NT; I++) {
+          c[I] = 0.f;
+          for (int m = 0; m < S; m++) c[I] += reinterpret_cast<const float*>(s.wave[m * R + u].t)[16 * I + (lane & 15)];
+        }
+      }
+      __syncthreads();
+      if (part == f) {
+#pragma unroll
+        for (int k = 0; k < NT; k++)
+          if (t0 + k < slot(0, NT)) P[t0 + k] = __builtin_bit_cast(f32x4, s.wave[w].lo[k][lane]);
+      }
+    }
+    if (part == f && q < p.n_pair)
+      sse += finish_row<NO, NT>(a, p.pair_row[q].x, it, alpha, s.lam, s.wave[w], P, c);
+  }
+  write_sse128(a, sse, blockIdx.x, s);
+}
+
 // nb: the component blocks that the finishing kernel reads.  It may be compiled
 // for more than K has, so the tiles beyond (zero) are stored too.
 template <int NO>
@@ -617,6 +677,23 @@ __global__ void __launch_bounds__(64 * kWaves128) k_heavy128(SampleArgs a, Batch
   write_sse128(a, sse, sse_slot0 + blockIdx.x, s);
 }
 
+// Waves that share a light row: as many as the rows leave free of the chip's 2048
+// (one work-group of eight a CU).  A wave takes 2 to 4 us for 32 nonzeros (the
+// gathers of one 16-component block after the other), the finish of a row 40 us.
+// Half-sweep in us with 1 | 2 | 4 | 8 waves a row, by rows x nonzeros, K = 128:
+//   64 x 100         43 | 45 | 40 | 39
+//   64 x 2000       242 | 186 | 116 | 82
+//   300 x 200        56 | 55 | 49 | 76
+//   300 x 2000      241 | 184 | 122 | 147
+//   1000 x 100       48 | 52 | 79 | 139
+//   1000 x 1000     158 | 133 | 155 | 209
+//   2000 x 1000     227 | 241 | 294 | 411
+// (a second round of work-groups, from 257 rows on with a grid of 512: 102 us at
+// 300 x 200, 463 at 300 x 2000).
+int waves_per_row(const BatchPlan& p) {
+  return p.n_light <= k128Grid ? 8 : p.n_light <= 2 * k128Grid ? 4 : p.n_light <= 4 * k128Grid ? 2 : 1;
+}
+
 template <int NO, int NT>
 void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
   const int gl = batched_light_grid(p), gh = batched_heavy_grid(p);
@@ -629,7 +706,9 @@ void launch128_t(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const S
     if (gh > 0) hipLaunchKernelGGL((k_heavy128<NT>), dim3(gh), dim3(64 * kWaves128), 0, ss, a, p, gl);
     if (fork) seg_record_join(seg);
   }
-  if (gl > 0) hipLaunchKernelGGL((k_light128<NO, NT>), dim3(gl), dim3(64 * kWaves128), 0, s, a, p);
+  const int S = waves_per_row(p);
+  if (gl > 0 && S > 1) hipLaunchKernelGGL((k_light128w<NO, NT>), dim3(gl), dim3(64 * kWaves128), 0, s, a, p, S);
+  else if (gl > 0) hipLaunchKernelGGL((k_light128<NO, NT>), dim3(gl), dim3(64 * kWaves128), 0, s, a, p);
   if (fork) seg_wait_join(s, seg);
 }
 

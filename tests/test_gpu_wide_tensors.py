@@ -35,6 +35,30 @@ def _leave_nan(nbytes):
     assert hip.hipFree(p) == 0
 
 
+# rows at the edges of the ways they are shared out: eight, four, two waves a row,
+# one, and a wave's second row
+@pytest.mark.parametrize("N,K,nother", [
+    (1, 128, 1), (255, 65, 1), (256, 97, 2), (257, 128, 1), (300, 80, 4), (511, 100, 1), (512, 128, 3), (513, 81, 1),
+    (1023, 112, 1), (1024, 66, 2), (1025, 128, 1), (2049, 113, 1)])
+def test_wide_rows_per_wave(N, K, nother):
+    announce("wide rows N=%d K=%d other=%d" % (N, K, nother))
+    rng = np.random.default_rng(N + K)
+    nb = 400
+    edges = [2049, 1, 31, 32, 33, 63, 64, 65, 128, 255, 256, 257, 2048, 0]
+    deg = np.array([edges[i % len(edges)] if i < 2 * len(edges) else int(rng.integers(0, 12)) for i in range(N)])
+    rng.shuffle(deg)
+    r = np.repeat(np.arange(N), deg)
+    idx = np.stack([r] + [rng.integers(0, nb, len(r)) for _ in range(nother)], 1).astype(np.int32)
+    modes, mean, _ = O.tensor_rows(idx, rng.standard_normal(len(r)), [N] + [nb] * nother)
+    others = [f32(0.7 * rng.standard_normal((nb, K))) for _ in range(nother)]
+    Lam, mu = f32(spd(rng, K, 2.0)), f32(rng.standard_normal(K))
+    ref = O.sample_latents(K, modes[0], mean, others, 3.0, mu, Lam, SEED, 2, 0)
+    got = gpu_sample_latents(K, modes[0], mean, others, 3.0, mu, Lam, SEED, 2, 0, _lib.SAMPLER_BATCHED)
+    e = row_rel_err(got, ref)
+    print("wide rows: row err %.3e" % e)
+    assert e < TOL
+
+
 @pytest.mark.parametrize("nother", [1, 2, 3, 4])
 @pytest.mark.parametrize("K", [65, 80, 81, 97, 112, 113])
 def test_wide_tensor_rows(K, nother):
