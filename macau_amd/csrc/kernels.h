@@ -37,6 +37,7 @@ struct BatchPlan {
   int K = 0, KP = 0;           // latent size, and padded: the plan's partials are sized for it
   int n_light = 0;             // light rows (sorted by nnz, descending)
   const int* light = nullptr;  // row ids
+  int light_max = 0;           // nonzeros of the longest one
   int n_seg = 0;               // segments of heavy rows
   const int* seg_row = nullptr;    // heavy-row slot of each segment
   const int* seg_beg = nullptr;    // first nnz

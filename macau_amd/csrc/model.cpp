@@ -468,6 +468,7 @@ BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int K, std::vector<D
   p.K = K;
   p.KP = KP;
   p.n_light = (int)light.size();
+  if (p.n_light) p.light_max = row_ptr[light[0] + 1] - row_ptr[light[0]];
   p.light = B[0].as<int>();
   p.n_seg = (int)sb.size();
   p.seg_row = B[1].as<int>();

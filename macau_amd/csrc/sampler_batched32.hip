@@ -22,8 +22,8 @@
 // lo = bf16(x - hi), and a tile accumulates Hi Hi^T + Hi Lo^T + Lo Hi^T + Lo Lo^T
 // in FP32.  Without Lo Lo^T the diagonal loses a positive bias of ~5e-6 |x|^2
 // per product, which rows of few nonzeros against a weak prior direction turn
-// into row errors near 1e-4.  Where rows are few there is a middle part too (24
-// bits; the split is then nearly all of the error).  The RHS accumulates in FP32
+// into row errors near 1e-4.  Up to kThreeParts light rows there is a middle part
+// too (24 bits; the split is then nearly all of the error).  The RHS accumulates in FP32
 // on the vector ALU.
 // Finish (finish_quad): row q of the four is taken over by lanes 16q .. 16q + 15,
 // which hold rows n and n + 16 of its matrix: everything that all lanes of a
@@ -48,6 +48,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 2;                                 // 16-component blocks
 constexpr int kTiles32 = 3;                           // their tiles
+constexpr int kThreeParts = 12000;                    // light rows up to which factors are split into three parts
 constexpr int kPartial32 = kTiles32 * 256 + NT * 64;  // floats per segment partial: tiles and RHS sums per lane
 
 __device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
@@ -563,7 +564,7 @@ __device__ __forceinline__ float finish_quad(const SampleArgs& a, int4 rows, int
 // (G = grid).  Row ids and ranges come from the plan in one load a pair, and the
 // next rows' ranges and their first two index blocks are loaded while the
 // current ones are finished.
-template <int NO>
+template <int NO, int PARTS>
 __global__ void __launch_bounds__(64, 2) k_light32(SampleArgs a, BatchPlan p) {
   __shared__ QuadLds<NO> S;
   const Factors<NO> F = make_factors<NO, 32>(a.others);
@@ -584,7 +585,7 @@ __global__ void __launch_bounds__(64, 2) k_light32(SampleArgs a, BatchPlan p) {
   int q = blockIdx.x;
   BlkReg<NO> b0, b1;
   if (q < n) plan(q);
-  QuadStream<NO, 4, 2> gs(a, F, S.blk, rng);
+  QuadStream<NO, 4, PARTS> gs(a, F, S.blk, rng);
   if (q < n) gs.first_blocks(b0, b1);
   while (q < n) {
     f32x4 T[4][kTiles32];
@@ -738,17 +739,25 @@ __global__ void __launch_bounds__(64) k_heavy32(SampleArgs a, BatchPlan p, int s
 }
 
 // Light rows per work-group of four waves (0: four a wave, k_light32).  Half-sweep
-// in us with 1 | 2 | 4 rows | four a wave, by rows x nonzeros a row, K = 32 (all
-// with two parts a factor; three cost the first three 2 to 28%):
-//   350 x 170        15.5 | 21 | 32 | 88
-//   8000 x 500       135 | 91 | 75 | 123
-//   15000 x 4        174 | 93 | 52 | 37
-//   40000 x 100      487 | 254 | 154 | 121
+// in us with 1 | 2 | 4 rows | four a wave, by rows x nonzeros a row, K = 32, three
+// parts a factor:
+//   300 x 512        19 | 21 | 25 | 43
+//   1500 x 256       32 | 23 | 24 | 31
+//   3000 x 1         45 | 28 | 19 | 19
+//   5000 x 128       69 | 44 | 31 | 30
+//   5000 x 500       97 | 74 | 58 | 66   (27000 factor columns)
+//   8000 x 1        102 | 58 | 36 | 23
+//   8000 x 500      145 | 104 | 83 | 73
+//   8000, up to 2048 (power law)  105 | 102 | 148   (2 | 4 rows | four a wave)
 // Few rows: the time is that of the longest row's gathers, one block of 64 after
 // the other, and of one finish.  Many: the finish of four rows at once by every
-// wave counts, and a work-group's three idle waves in it do not pay.
+// wave counts, and a work-group's three idle waves in it do not pay, unless the
+// longest rows, four of them one after the other on a wave, take longer still.
 static int rows_per_group(const BatchPlan& p) {
-  return p.n_light <= 512 ? 1 : p.n_light <= 1024 ? 2 : p.n_light <= 12000 ? 4 : 0;
+  if (p.n_light <= 512) return 1;
+  if (p.n_light <= 1024) return 2;
+  if (p.n_light <= 3000) return 4;
+  return p.n_light <= kThreeParts && p.light_max > p.n_light / 12 ? 4 : 0;
 }
 
 // Four rows a wave: without a cap of the plan's, 16384 waves, which take the
@@ -785,7 +794,9 @@ static void launch_batched32_t(const SampleArgs& a, const BatchPlan& p, hipStrea
       case 1: hipLaunchKernelGGL((k_light32w<NO, 1>), dim3(gl), dim3(256), 0, s, a, p); break;
       case 2: hipLaunchKernelGGL((k_light32w<NO, 2>), dim3(gl), dim3(256), 0, s, a, p); break;
       case 4: hipLaunchKernelGGL((k_light32w<NO, 4>), dim3(gl), dim3(256), 0, s, a, p); break;
-      default: hipLaunchKernelGGL((k_light32<NO>), dim3(gl), dim3(64), 0, s, a, p);
+      default:
+        if (p.n_light <= kThreeParts) hipLaunchKernelGGL((k_light32<NO, 3>), dim3(gl), dim3(64), 0, s, a, p);
+        else hipLaunchKernelGGL((k_light32<NO, 2>), dim3(gl), dim3(64), 0, s, a, p);
     }
   }
   if (fork) seg_wait_join(s, seg);
