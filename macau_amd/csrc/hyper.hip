@@ -45,10 +45,14 @@ static int stats_width(int K) {
   const int nt = stats_tiles(K);
   return 16 * nt + 128 * nt * (nt + 1);
 }
-// One work-group per 32 columns up to one per CU; half as many above K = 64,
-// where a partial is 74 KB and the reduction's reads begin to count
+// One work-group per 32 columns up to one per CU.  Above K = 64 a wave has one
+// step's loads in flight, so many columns take two work-groups a CU; fewer do not,
+// because a partial is 74 KB and the reduction's reads count.  Statistics and draw
+// in us with 128 | 256 | 512 | 1024 work-groups, K = 128, FP32:
+//   10000 columns   77 | 72 | 74 | 73      100000    232 | 147 | 123 | 129
+//   20000           94 | 79 | 77 | 81     1000000   1789 | 942 | 684 | 661
 int hyper_stats_blocks(int N, int K) {
-  const int cap = K > 64 ? 128 : 256;
+  const int cap = K > 64 && N >= 32768 ? 512 : 256;
   return std::max(1, std::min(cap, (N + 31) / 32));
 }
 size_t hyper_stats_doubles(int nblk, int K) { return (size_t)2 * (K + K * K) + (size_t)nblk * stats_width(K); }
