@@ -79,14 +79,23 @@ static void write_csv(const std::string& fn, const std::vector<double>& colmajor
 // ------------------------------------------------------------------
 // data layer (sparsetensor.cpp:11-60, 78-117; bpmfutils.h:57-82)
 // ------------------------------------------------------------------
-// 0 .. n-1 ordered by key(i) in [0, nkeys), equal keys in their order.  Counting:
-// the cells' comparison sorts took 33 of the 53 ms of a 100-iteration call on
-// 400000 cells.
+// 0 .. n-1 ordered by key(i) >= 0, equal keys in their order.  Counting: the
+// cells' comparison sorts took 33 of the 53 ms of a 100-iteration call on 400000
+// cells.  Keys far beyond n (a few cells of a huge matrix) are compared instead,
+// where clearing the counts would take longer (8 s up to 2^31).
 template <typename Key>
-static std::vector<int> order_by(size_t n, int nkeys, Key&& key) {
-  std::vector<int> pos(nkeys + 1, 0), order(n);
+static std::vector<int> order_by(size_t n, Key&& key) {
+  std::vector<int> order(n);
+  int top = -1;
+  for (size_t i = 0; i < n; i++) top = std::max(top, (int)key(i));
+  if ((size_t)(top + 1LL) > 16 * n + (1 << 20)) {
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key(a) < key(b); });
+    return order;
+  }
+  std::vector<int> pos(top + 2LL, 0);
   for (size_t i = 0; i < n; i++) pos[key(i) + 1]++;
-  for (int k = 0; k < nkeys; k++) pos[k + 1] += pos[k];
+  for (int k = 0; k <= top; k++) pos[k + 1] += pos[k];
   for (size_t i = 0; i < n; i++) order[pos[key(i)]++] = (int)i;
   return order;
 }
@@ -101,8 +110,8 @@ static void sum_duplicates(const int* idx, int nnz, const double* vals, const in
       throw std::runtime_error("MatrixData: index out of range");
   }
   const int *row = idx, *col = idx + nnz;
-  const std::vector<int> by_row = order_by(nnz, dims[0], [&](size_t e) { return row[e]; });
-  const std::vector<int> by_col = order_by(nnz, dims[1], [&](size_t e) { return col[by_row[e]]; });
+  const std::vector<int> by_row = order_by(nnz, [&](size_t e) { return row[e]; });
+  const std::vector<int> by_col = order_by(nnz, [&](size_t e) { return col[by_row[e]]; });
   r.clear();
   c.clear();
   v.clear();
@@ -202,7 +211,7 @@ void Model::setRelationDataTest(const int* idx, int nm, const double* vals, int 
       for (int m = 0; m < nm; m++)
         if (idx[(size_t)m * nnz_in + e] < 0 || idx[(size_t)m * nnz_in + e] >= d[m])
           throw std::runtime_error("SparseMode: mode value larger than mode_size");
-    for (int q : order_by(nnz_in, d[0], [&](size_t e) { return idx[e]; })) {
+    for (int q : order_by(nnz_in, [&](size_t e) { return idx[e]; })) {
       for (int m = 0; m < nm; m++) test_idx.push_back(idx[(size_t)m * nnz_in + q]);
       test_vals.push_back(vals[q]);
     }
@@ -322,9 +331,7 @@ void Model::init() {
     int km = 0;
     for (int m = 1; m < nmodes; m++)
       if (dims[m] > dims[km]) km = m;
-    int nkeys = 0;
-    for (long long t = 0; t < ntest; t++) nkeys = std::max(nkeys, test_idx[(size_t)t * nmodes + km] + 1);
-    test_perm = order_by(ntest, nkeys, [&](size_t t) { return test_idx[t * nmodes + km]; });
+    test_perm = order_by(ntest, [&](size_t t) { return test_idx[t * nmodes + km]; });
     std::vector<int> didx((size_t)ntest * nmodes);
     std::vector<double> dvals(ntest);
     for (long long t = 0; t < ntest; t++) {
@@ -422,7 +429,7 @@ BatchPlan build_batch_plan(const std::vector<int>& row_ptr, int K, std::vector<D
   const int seg = seg_len;
   int most = 0;
   for (int n = 0; n < N; n++) most = std::max(most, row_ptr[n + 1] - row_ptr[n]);
-  const std::vector<int> order = order_by(N, most + 1, [&](size_t n) { return most - (row_ptr[n + 1] - row_ptr[n]); });
+  const std::vector<int> order = order_by(N, [&](size_t n) { return most - (row_ptr[n + 1] - row_ptr[n]); });
   std::vector<int> light, heavy, hseg0, sr, sb, se;
   for (int q = 0; q < N; q++) {
     const int r = order[q];
