@@ -608,13 +608,18 @@ void Model::launch_pending_prior() {
 // iteration at 5000 x 2000, K = 10, where the kernels on the critical path take 60.
 constexpr int kGraphIters = 4;
 
-void Model::iterate(int n) {
-  if (!initialized) throw std::runtime_error("model not initialized");
-  bool graphable = use_graph;
+bool Model::graphable() const {
+  if (!use_graph) return false;
   for (auto& p : priors) {
     const auto* mp = dynamic_cast<const MacauPrior*>(p.get());
-    if (mp && !mp->capturable()) graphable = false;
+    if (mp && !mp->capturable()) return false;
   }
+  return true;
+}
+
+void Model::iterate(int n) {
+  if (!initialized) throw std::runtime_error("model not initialized");
+  const bool graphable = this->graphable();
   for (int i = 0; i < n;) {
     int len = 1;
     if (graphable) {
@@ -747,15 +752,18 @@ void Model::run() {
     if (verbose && i == burnin) printf(" ====== Burn-in complete, averaging samples ====== \n");
     const double starti = tick();
     // a failed factorisation stops the chain within kFailPollIters iterations
-    // (every iteration when the host reads the state anyway): the iterations
-    // until the next look are enqueued together
+    // (every iteration when the host reads the state anyway).  Replayed ones are
+    // enqueued together up to the next look; where the host takes part in an
+    // iteration, Ctrl-C is looked at after each.
     const bool need_host = verbose || (save_model && i >= burnin);
     int len = 1;
-    if (!need_host) len = std::min(kFailPollIters, (save_model ? burnin : burnin + nsamples) - i);
+    if (!need_host && graphable()) len = std::min(kFailPollIters, (save_model ? burnin : burnin + nsamples) - i);
     iterate(len);
     i += len;
-    sync();
-    check_fail();
+    if (need_host || len > 1 || i % kFailPollIters == 0) {
+      sync();
+      check_fail();
+    }
     if (need_host) {
       noise->rmse_test_onesample = host_eval_out(0);
       noise->rmse_test = host_eval_out(1);

@@ -290,6 +290,7 @@ class Model {
 
   // extensions
   void iterate(int n);                 // n Gibbs iterations after init()
+  bool graphable() const;              // iterations are replayed as graphs
   void sync() { HIPCHK(hipStreamSynchronize(stream)); }
   void check_fail();
   void download_latents(int mode, double* out);  // K x N col-major
