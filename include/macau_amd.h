@@ -152,10 +152,10 @@ int macau_get_refine_stats(macau_model* m, long long* flagged, long long* refine
  * state as it was, writes each mode's half-sweep ms with the default and the
  * chosen shape to default_ms[nmodes] / tuned_ms[nmodes] (either may be
  * NULL) and, when record_path is not NULL, appends the choices to that
- * table.  macau_init looks the shape up by (GPU architecture, padded latent
- * size, other modes, rows, nonzeros, log2 row-degree histogram) in the table
- * named by the environment variable MACAU_AMD_TUNE_CACHE, then in
- * tuning.txt beside the library.  Plain-sampler models have nothing to tune.
+ * table.  macau_init looks the shape up by (GPU architecture, the latent
+ * size's kernels: K <= 16, 32, 64 or 128, other modes, rows, nonzeros, log2
+ * row-degree histogram) in the table named by the environment variable
+ * MACAU_AMD_TUNE_CACHE, then in tuning.txt beside the library.  Plain-sampler models have nothing to tune.
  * macau_get_tuning writes (segment length, light cap, heavy cap, segment
  * cap) of a mode to knobs[4] and returns 1 if they come from the tuner or
  * the table, 0 for the defaults, -1 on error. */

@@ -531,9 +531,10 @@ int macau_get_tuning(macau_model* m, int mode, int* knobs) {
   if (!x.initialized) throw std::runtime_error("model not initialized");
   if (mode < 0 || mode >= x.nmodes) throw std::runtime_error("mode out of range");
   const TuneChoice& c = x.tune[mode];
+  const bool batched = (int)x.plans.size() == x.nmodes;
   knobs[0] = c.seg_len;
-  knobs[1] = c.light_cap ? c.light_cap : kDefaultLightCap;
-  knobs[2] = c.heavy_cap ? c.heavy_cap : kDefaultHeavyCap;
+  knobs[1] = c.light_cap ? c.light_cap : batched ? batched_light_default(x.plans[mode]) : kDefaultLightCap;
+  knobs[2] = c.heavy_cap ? c.heavy_cap : batched ? batched_heavy_default(x.plans[mode]) : kDefaultHeavyCap;
   knobs[3] = c.seg_cap ? c.seg_cap : kDefaultSegCap;
   return c.tuned ? 1 : 0;
   API_END_VAL(-1)

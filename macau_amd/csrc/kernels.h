@@ -31,6 +31,7 @@ struct FactorSet {
 constexpr int kDefaultSegLen = 2048;
 constexpr int kDefaultLightCap = 8192, kDefaultHeavyCap = 2048, kDefaultSegCap = 16384;
 // largest light / heavy caps the autotuner tries (SSE partial slots are sized for them)
+constexpr int k128Grid = 256;  // K > 64: work-groups of the light- and heavy-row kernels, one a CU
 constexpr int kMaxLightCap = 16384, kMaxHeavyCap = 4096;
 
 struct BatchPlan {
@@ -53,8 +54,8 @@ struct BatchPlan {
   const int2* pair_row = nullptr;  // row ids (y = -1: no second row)
   // launch shape (0 = the defaults below); chosen by the autotuner
   int seg_len = kDefaultSegLen;    // nonzeros per heavy-row segment (set when the plan is built)
-  int light_cap = 0;               // most work-groups of the light-row kernel (default 8192)
-  int heavy_cap = 0;               // most work-groups of the heavy-row finishing kernel (default 2048)
+  int light_cap = 0;               // most work-groups of the light-row kernel (0: batched_light_default)
+  int heavy_cap = 0;               // most work-groups of the heavy-row finishing kernel (0: batched_heavy_default)
   int seg_cap = 0;                 // most work-groups of the segment kernel (default 16384)
 };
 
@@ -134,6 +135,11 @@ void launch_sample_batched64(const SampleArgs& a, const BatchPlan& p, hipStream_
 void launch_sample_batched128(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg = {});
 int batched128_light_grid(const BatchPlan& p);
 int batched128_heavy_grid(const BatchPlan& p);
+// the caps that a plan without its own gets: what they count differs between the
+// kernels (pairs of rows, fours, or work-groups of eight waves above K = 64)
+int batched_light_default(const BatchPlan& p);
+int batched_heavy_default(const BatchPlan& p);
+int batched32_light_default(const BatchPlan& p);
 int batched64_light_grid(const BatchPlan& p);
 int batched64_heavy_grid(const BatchPlan& p);
 int batched_supported(int KP, int nother);

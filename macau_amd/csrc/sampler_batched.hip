@@ -529,11 +529,16 @@ __global__ void __launch_bounds__(64, 4) k_heavy16(SampleArgs a, BatchPlan p, in
   write_sse(a, sse, sse_slot0 + blockIdx.x);
 }
 
+int batched_light_default(const BatchPlan& p) {
+  if (p.KP == 128) return k128Grid;
+  return p.KP == 32 && p.K > 16 ? batched32_light_default(p) : kDefaultLightCap;
+}
+int batched_heavy_default(const BatchPlan& p) { return p.KP == 128 ? k128Grid : kDefaultHeavyCap; }
 int batched_light_grid(const BatchPlan& p) {
   if (p.KP == 128) return batched128_light_grid(p);
   if (p.KP >= 64) return batched64_light_grid(p);  // one row per work-group
   if (p.K > 16) return batched32_light_grid(p);
-  const int cap = p.light_cap > 0 ? p.light_cap : kDefaultLightCap;
+  const int cap = p.light_cap > 0 ? p.light_cap : batched_light_default(p);
   return p.n_pair < cap ? p.n_pair : cap;
 }
 int batched_heavy_grid(const BatchPlan& p) {

@@ -37,7 +37,6 @@ namespace mgpu {
 namespace {
 
 constexpr int kThreads128 = 256;
-constexpr int k128Grid = 256;                     // work-groups of the light- and heavy-row kernels: one a CU
 constexpr int kTiles = 36;                        // 16 x 16 tiles of the upper triangle
 constexpr int kPartial128 = kTiles * 256 + 128;   // floats per segment partial: tiles and RHS sums
 
@@ -732,8 +731,12 @@ void launch128_k(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const S
 
 // A work-group's waves take rows gridDim.x apart, so that few rows spread over
 // the CUs first
-int batched128_light_grid(const BatchPlan& p) { return std::min(p.n_pair, k128Grid); }
-int batched128_heavy_grid(const BatchPlan& p) { return std::min(p.n_heavy, k128Grid); }
+int batched128_light_grid(const BatchPlan& p) {
+  return std::min(p.n_pair, p.light_cap > 0 ? p.light_cap : batched_light_default(p));
+}
+int batched128_heavy_grid(const BatchPlan& p) {
+  return std::min(p.n_heavy, p.heavy_cap > 0 ? p.heavy_cap : batched_heavy_default(p));
+}
 
 void launch_sample_batched128(const SampleArgs& a, const BatchPlan& p, hipStream_t s, const SegStreams& seg) {
   switch (a.rows.nother) {

@@ -763,9 +763,12 @@ static int rows_per_group(const BatchPlan& p) {
 // Four rows a wave: without a cap of the plan's, 16384 waves, which take the
 // rows in 2 strides at 138000 x 32 (5% less time than 8192 waves, 30% less than
 // 3072: fewer waves with more rows each end less evenly).
+int batched32_light_default(const BatchPlan& p) {
+  return rows_per_group(p) ? kDefaultLightCap : 2 * kDefaultLightCap;
+}
 int batched32_light_grid(const BatchPlan& p) {
   const int r = rows_per_group(p), n = r ? (p.n_light + r - 1) / r : (p.n_pair + 1) / 2;
-  const int cap = p.light_cap > 0 ? p.light_cap : 2 * kDefaultLightCap;
+  const int cap = p.light_cap > 0 ? p.light_cap : batched32_light_default(p);
   return n < cap ? n : cap;
 }
 int batched32_heavy_grid(const BatchPlan& p) {

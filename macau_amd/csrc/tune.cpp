@@ -11,7 +11,7 @@
 // mode are saved before and restored after the timing runs, so tuning leaves
 // the chain where it was.
 //
-// Choices are recorded per (GPU architecture, padded latent size, number of
+// Choices are recorded per (GPU architecture, the latent size's kernels, number of
 // other modes, rows, nonzeros, histogram of log2 row degrees) in a text table
 // and looked up at initialisation: first in the file named by
 // MACAU_AMD_TUNE_CACHE, then in tuning.txt beside the library
@@ -74,6 +74,11 @@ std::vector<TuneEntry> read_table(const std::string& path) {
 
 }  // namespace
 
+// The kernels that a shape was measured on: the padded latent size, apart for K up
+// to 16, with a revision where the caps have come to count other work-groups (a
+// table's older entries are then not found).
+static const char* tune_kernels(int K) { return K <= 16 ? "16" : K <= 32 ? "32.2" : K <= 64 ? "64" : "128.2"; }
+
 std::string Model::tune_key(int mode) const {
   // histogram of floor(log2(degree + 1)), hashed (FNV-1a 64)
   const std::vector<int>& rp = rows[mode].row_ptr;
@@ -91,7 +96,7 @@ std::string Model::tune_key(int mode) const {
       h *= 1099511628211ull;
     }
   char buf[256];
-  snprintf(buf, sizeof(buf), "%s %d %d %d %lld %016llx", gpu_arch().c_str(), KP, nmodes - 1, dims[mode],
+  snprintf(buf, sizeof(buf), "%s %s %d %d %lld %016llx", gpu_arch().c_str(), tune_kernels(num_latent), nmodes - 1, dims[mode],
            (long long)rp.back(), (unsigned long long)h);
   return buf;
 }
@@ -115,8 +120,9 @@ void Model::apply_cached_tuning() {
 }
 
 void Model::apply_plan_shape(int m) {
-  plans[m].light_cap = tune[m].light_cap;
-  plans[m].heavy_cap = tune[m].heavy_cap;
+  // (a table's caps too within what the SSE slots are sized for)
+  plans[m].light_cap = std::min(tune[m].light_cap, kMaxLightCap);
+  plans[m].heavy_cap = std::min(tune[m].heavy_cap, kMaxHeavyCap);
   plans[m].seg_cap = tune[m].seg_cap;
 }
 
@@ -154,8 +160,11 @@ std::vector<std::pair<double, double>> Model::autotune(int reps, const std::stri
     return (double)ms / r;
   };
   const int seg_lens[] = {1024, 2048, 4096};
-  const int light_caps[] = {2048, 4096, 8192, 16384};
-  const int heavy_caps[] = {1024, 2048, 4096};
+  // (work-groups of eight waves above K = 64)
+  const std::vector<int> light_caps =
+      num_latent > 64 ? std::vector<int>{128, 256, 512, 1024} : std::vector<int>{2048, 4096, 8192, 16384};
+  const std::vector<int> heavy_caps =
+      num_latent > 64 ? std::vector<int>{128, 256, 512} : std::vector<int>{1024, 2048, 4096};
   const int seg_caps[] = {4096, 16384, 65536};
   std::vector<std::string> records;
   for (int m = 0; m < nmodes; m++) {
