@@ -119,7 +119,8 @@ int macau_get_last_cg_iters(macau_model* m, int mode);
  * latentprior.cpp:280-288): 0 = the mode has no F^T F branch, 1 = blocked
  * Cholesky every iteration, 2 = eigendecomposition of F^T F at setup and two
  * products per iteration (the default; environment variable
- * MACAU_AMD_FTF_SOLVER=cholesky selects 1). */
+ * MACAU_AMD_FTF_SOLVER=cholesky selects 1, and so does an eigendecomposition
+ * that does not solve random right-hand sides to 1e-9). */
 int macau_get_ftf_solver(macau_model* m, int mode);
 
 /* ---- refinement of ill-conditioned rows (batched sampler; no reference

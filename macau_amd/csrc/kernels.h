@@ -353,7 +353,9 @@ void launch_ftf_solve(const double* FtF, int n, const double* reg, double* W, do
 // false with a reason when the eigensolver is unavailable or fails;
 // launch_spectral_solve sets X = Q diag(d + *reg)^{-1} Q^T B through
 // Y (n x nrhs) and part (plan.S x n x nrhs), a non-positive d_j + *reg
-// setting *fail to kFailDenseChol
+// setting *fail to kFailDenseChol.  With idx (n columns of nfeat, ascending) and
+// pos (each column's place among them, or -1) B and X have all nfeat columns and
+// the others' X is B / *reg; launch_spectral_take gives their A
 struct SpectralPlan {
   int S = 1;       // inner-dimension chunks
   int tchunk = 0;  // chunk depth
@@ -362,7 +364,8 @@ SpectralPlan spectral_plan(int n, int nrhs);
 bool spectral_factor(double* A, int n, double* d, double* Qt, hipStream_t s, std::string* why);
 void launch_spectral_solve(const double* Q, const double* Qt, const double* d, int n, const double* reg,
                            const double* B, double* Y, double* part, const SpectralPlan& p, double* X, int nrhs,
-                           int* fail, hipStream_t s);
+                           const int* idx, const int* pos, int nfeat, int* fail, hipStream_t s);
+void launch_spectral_take(const double* G, int nfeat, const int* idx, int n, double* A, hipStream_t s);
 constexpr int kSpmmSegNnz = 256;
 constexpr int kSpmmLongNnz = 32;
 // out[:, r] = sum_c A[r,c] in[:, c] (+ (*reg) * add[:, r]); vectors have ld = nr

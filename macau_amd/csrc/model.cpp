@@ -1190,6 +1190,11 @@ static bool gram_for_cg(double n, double rows, double entries) {
   return n <= kGramMaxCg && n * n <= 128 * entries && rows * n * n <= 1.7e11;
 }
 
+// A solve through the eigenvectors, with 1/1000 of the largest eigenvalue as
+// regulariser, leaves at most this of right-hand sides of size 1 (rounding: some
+// 1e-11); otherwise F^T F + lambda_beta I is factored in every iteration
+constexpr double kSpectralTol = 1e-9;
+
 // Empty columns from which the block CG replaces them (by at most 32 features)
 constexpr int kGramMinEmpty = 128;
 
@@ -1256,19 +1261,60 @@ void MacauPrior::init(Model& m, int mode) {
     if (env && std::strcmp(env, "cholesky") == 0) {
       ftf_note = "MACAU_AMD_FTF_SOLVER=cholesky";
     } else {
-      ftf_d.alloc((size_t)nfeat * sizeof(double));
-      if (spectral_factor(FtF.as<double>(), nfeat, ftf_d.as<double>(), Wchol.as<double>(), m.stream, &ftf_note)) {
-        ftf_solver = kFtfSpectral;
-        ftf_plan = spectral_plan(nfeat, K);
-        ftf_y.alloc(kf * sizeof(double));
-        ftf_part.alloc((size_t)ftf_plan.S * kf * sizeof(double));
-      } else {
-        // the eigensolver may have overwritten F^T F: form it again
-        launch_ftf(F(), Ft(), FtF.as<double>(), m.stream);
+      ftf_n = list_columns(nfeat - 1, m.stream) ? gram.n : nfeat;
+      const size_t sq = (size_t)ftf_n * ftf_n * sizeof(double), ks = (size_t)K * ftf_n * sizeof(double);
+      DevBuf Q(sq), Qt(sq);
+      launch_spectral_take(FtF.as<double>(), nfeat, gram.idx, ftf_n, Q.as<double>(), m.stream);
+      ftf_d.alloc((size_t)ftf_n * sizeof(double));
+      if (spectral_factor(Q.as<double>(), ftf_n, ftf_d.as<double>(), Qt.as<double>(), m.stream, &ftf_note)) {
+        ftf_plan = spectral_plan(ftf_n, K);
+        ftf_y.alloc(ks);
+        ftf_part.alloc(ftf_plan.S * ks);
+        std::swap(FtF, Q);
+        std::swap(Wchol, Qt);
+        const double err = spectral_error(K, m.stream);
+        if (err <= kSpectralTol) {
+          ftf_solver = kFtfSpectral;
+        } else {
+          ftf_note = "eigenvectors of F^T F off by " + std::to_string(err);
+          std::swap(FtF, Q);
+          std::swap(Wchol, Qt);
+        }
       }
     }
   }
   HIPCHK(hipStreamSynchronize(m.stream));
+}
+
+double MacauPrior::spectral_error(int K, hipStream_t s) {
+  const size_t n = (size_t)K * nfeat;
+  std::vector<double> b(n), r(n), d(ftf_n);
+  uint32_t x = 12345;
+  for (double& v : b) {
+    x = x * 1664525u + 1013904223u;
+    v = x >> 31 ? 1.0 : -1.0;
+  }
+  HIPCHK(hipMemcpyAsync(d.data(), ftf_d.as<void>(), ftf_n * sizeof(double), hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  DevBuf B, reg, fail, X(n * sizeof(double)), in((size_t)K * nrow * sizeof(double)), out(n * sizeof(double));
+  upload(B, b, s);
+  const double top = d.back();  // the largest eigenvalue
+  upload_scalar<double>(reg, top > 0.0 ? 1e-3 * top : 1.0, s);
+  upload_scalar<int>(fail, 0, s);
+  launch_spectral_solve(FtF.as<double>(), Wchol.as<double>(), ftf_d.as<double>(), ftf_n, reg.as<double>(),
+                        B.as<double>(), ftf_y.as<double>(), ftf_part.as<double>(), ftf_plan, X.as<double>(), K,
+                        gram.idx, gram.pos, nfeat, fail.as<int>(), s);
+  launch_spmm(F(), X.as<double>(), K, in.as<double>(), nullptr, nullptr, s);
+  launch_spmm(Ft(), in.as<double>(), K, out.as<double>(), reg.as<double>(), X.as<double>(), s);
+  HIPCHK(hipMemcpyAsync(r.data(), out.as<void>(), n * sizeof(double), hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  double worst = 0.0;
+  for (size_t q = 0; q < n; q++) {
+    const double e = std::fabs(r[q] - b[q]);
+    if (std::isnan(e)) return e;
+    worst = std::max(worst, e);
+  }
+  return worst;
 }
 
 void CgBuffers::alloc(int nr, int nfeat, int nsamples, int nb) {
@@ -1502,9 +1548,9 @@ void MacauPrior::update_prior(Model& m, int mode) {  // latentprior.cpp:254-264
   if (use_ftf && ftf_solver == kFtfSpectral) {
     // beta = Ft_y (FtF + lambda_beta I)^{-1} (latentprior.cpp:280-288)
     // through the eigendecomposition of FtF made at init
-    launch_spectral_solve(FtF.as<double>(), Wchol.as<double>(), ftf_d.as<double>(), nfeat, lambda_beta_d.as<double>(),
+    launch_spectral_solve(FtF.as<double>(), Wchol.as<double>(), ftf_d.as<double>(), ftf_n, lambda_beta_d.as<double>(),
                           Fty.as<double>(), ftf_y.as<double>(), ftf_part.as<double>(), ftf_plan, beta.as<double>(), K,
-                          m.d_fail.as<int>(), s);
+                          gram.idx, gram.pos, nfeat, m.d_fail.as<int>(), s);
     last_cg_iters = 0;
   } else if (use_ftf) {
     // K = FtF + lambda_beta I; chol_decomp(K); chol_solve_t(K, Ft_y);

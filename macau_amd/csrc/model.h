@@ -155,6 +155,9 @@ class MacauPrior : public ILatentPrior {
   std::string ftf_note;  // why the spectral solve is not used, when it is not
   DevBuf ftf_d, ftf_y, ftf_part;
   SpectralPlan ftf_plan;
+  int ftf_n = 0;  // columns decomposed: the non-empty ones
+  // the solve's largest error on random right-hand sides, relative to them
+  double spectral_error(int K, hipStream_t s);
   CsrDev F() const;
   CsrDev Ft() const;
   // uploads F and F^T and builds their SpMM work lists (nrmax right-hand sides)

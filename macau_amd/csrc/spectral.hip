@@ -8,7 +8,10 @@
 // FP64), turns every later solve into
 //     Y = Q^T B,   Y[j][:] /= (d_j + lambda_beta),   X = Q Y,
 // two n x n by n x nrhs FP64 products that stream Q from HBM once each, in
-// place of n / 32 dependent factor and solve steps.  Q is kept twice (Q and
+// place of n / 32 dependent factor and solve steps.  F's empty columns are left
+// out of the decomposition and taken as B / lambda_beta: the eigensolver's vectors
+// for the large null space that they make were not orthogonal for some matrices
+// (15000 x 2000 with 1100 empty columns: those columns off by up to 9e-2).  Q is kept twice (Q and
 // Q^T, both column-major) so both products read M's columns contiguously.
 // A non-positive d_j + lambda_beta sets the same fail flag as a non-positive
 // Cholesky pivot.
@@ -37,13 +40,15 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // part[blockIdx.y][r][k] = sum over t in chunk blockIdx.y of M[t + r n] X[t][k]
 // (M column-major n x n, so the sum runs down column r of M: out = M^T X).
+// With idx, row t of X is its row idx[t].
 // Work-group (x, y, z): rows r0 .. r0 + 127, inner chunk y, columns
 // k0 .. k0 + 31.  Wave w owns rows r0 + 32 w .. + 31 as 2 x 2 FP64 MFMA
 // tiles of 16 x 16 (v_mfma_f64_16x16x4f64: lane l holds A[l % 16][l / 16],
 // B[l / 16][l % 16] and D[4 v + l / 16][l % 16], v = 0..3).  The next
 // slab's global loads are issued before the current slab is consumed.
 __global__ void __launch_bounds__(256, 3) k_spec_mm(const double* __restrict__ M, int n, const double* __restrict__ X,
-                                                 int nrhs, int tchunk, double* __restrict__ part) {
+                                                 const int* __restrict__ idx, int nrhs, int tchunk,
+                                                 double* __restrict__ part) {
   __shared__ __align__(16) double Ms[kSmRows][kMsLd];  // [row][inner]
   __shared__ __align__(16) double Xs[kSmT][kXsLd];     // [inner][column]
   const int r0 = blockIdx.x * kSmRows;
@@ -65,7 +70,7 @@ __global__ void __launch_bounds__(256, 3) k_spec_mm(const double* __restrict__ M
     for (int u = 0; u < 4; u++) {
       const int q = tid + 256 * u;
       const int gt = t0 + (q >> 5), gk = k0 + (q & 31);
-      xv[u] = (gt < te && gk < nrhs) ? X[(size_t)gt * nrhs + gk] : 0.0;
+      xv[u] = (gt < te && gk < nrhs) ? X[(size_t)(idx ? idx[gt] : gt) * nrhs + gk] : 0.0;
     }
   };
   f64x4 acc[2][2];
@@ -135,6 +140,39 @@ __global__ void __launch_bounds__(256) k_spec_reduce(const double* __restrict__ 
   }
 }
 
+// X over all nfeat columns: the sums of part where pos[f] >= 0, B / *reg elsewhere
+__global__ void __launch_bounds__(256) k_spec_expand(const double* __restrict__ part, int S, int n, int nrhs,
+                                                     const int* __restrict__ pos, int nfeat,
+                                                     const double* __restrict__ B, const double* reg,
+                                                     double* __restrict__ X, int* fail) {
+  const size_t tot = (size_t)nfeat * nrhs, stride = (size_t)n * nrhs;
+  double den = *reg;
+  if (!(den > 0.0)) {
+    atomicMax(fail, kFailDenseChol);
+    den = 1.0;
+  }
+  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot; q += (size_t)gridDim.x * blockDim.x) {
+    const int p = pos[q / nrhs];
+    double s = 0.0;
+    if (p >= 0) {
+      for (int b = 0; b < S; b++) s += part[b * stride + (size_t)p * nrhs + q % nrhs];
+    } else {
+      s = B[q] / den;
+    }
+    X[q] = s;
+  }
+}
+
+// A[i][j] = G[idx[i]][idx[j]] of the nfeat x nfeat matrix G (idx null: all of it)
+__global__ void __launch_bounds__(256) k_spec_take(const double* __restrict__ G, int nfeat,
+                                                   const int* __restrict__ idx, int n, double* __restrict__ A) {
+  const size_t tot = (size_t)n * n;
+  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot; q += (size_t)gridDim.x * blockDim.x) {
+    const int i = (int)(q % n), j = (int)(q / n);
+    A[q] = G[(size_t)(idx ? idx[i] : i) + (size_t)(idx ? idx[j] : j) * nfeat];
+  }
+}
+
 // Qt = Q^T for column-major n x n matrices, 32 x 32 tiles through LDS
 __global__ void __launch_bounds__(256) k_transpose(const double* __restrict__ Q, int n, double* __restrict__ Qt) {
   __shared__ double T[32][33];
@@ -175,17 +213,27 @@ static int reduce_grid(size_t work) {
   return (int)g;
 }
 
+void launch_spectral_take(const double* G, int nfeat, const int* idx, int n, double* A, hipStream_t s) {
+  hipLaunchKernelGGL(k_spec_take, dim3(reduce_grid((size_t)n * n)), dim3(256), 0, s, G, nfeat, idx, n, A);
+}
+
 void launch_spectral_solve(const double* Q, const double* Qt, const double* d, int n, const double* reg,
                            const double* B, double* Y, double* part, const SpectralPlan& p, double* X, int nrhs,
-                           int* fail, hipStream_t s) {
+                           const int* idx, const int* pos, int nfeat, int* fail, hipStream_t s) {
   const dim3 grid((n + kSmRows - 1) / kSmRows, p.S, (nrhs + kSmK - 1) / kSmK);
   const int rg = reduce_grid((size_t)n * nrhs);
   // Y = diag(d + reg)^{-1} Q^T B
-  hipLaunchKernelGGL(k_spec_mm, grid, dim3(256), 0, s, Q, n, B, nrhs, p.tchunk, part);
+  hipLaunchKernelGGL(k_spec_mm, grid, dim3(256), 0, s, Q, n, B, idx, nrhs, p.tchunk, part);
   hipLaunchKernelGGL(k_spec_reduce<true>, dim3(rg), dim3(256), 0, s, (const double*)part, p.S, n, nrhs, d, reg, Y,
                      fail);
   // X = Q Y: column r of Q^T is row r of Q
-  hipLaunchKernelGGL(k_spec_mm, grid, dim3(256), 0, s, Qt, n, (const double*)Y, nrhs, p.tchunk, part);
+  hipLaunchKernelGGL(k_spec_mm, grid, dim3(256), 0, s, Qt, n, (const double*)Y, (const int*)nullptr, nrhs, p.tchunk,
+                     part);
+  if (pos) {
+    hipLaunchKernelGGL(k_spec_expand, dim3(reduce_grid((size_t)nfeat * nrhs)), dim3(256), 0, s, (const double*)part,
+                       p.S, n, nrhs, pos, nfeat, B, reg, X, fail);
+    return;
+  }
   hipLaunchKernelGGL(k_spec_reduce<false>, dim3(rg), dim3(256), 0, s, (const double*)part, p.S, n, nrhs, nullptr,
                      nullptr, X, fail);
 }
