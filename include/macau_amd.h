@@ -176,8 +176,12 @@ typedef struct macau_batch macau_batch;
 macau_batch* macau_batch_create(macau_model* const* models, int n);
 void macau_batch_free(macau_batch* b);
 /* 1 (default): one graph per iteration of all models; 0: each model replays
- * its own iteration graph on its own streams, all queued before any wait */
+ * its own iteration graph on its own streams, all queued before any wait (the
+ * same chains).  In a process that holds another HIP runtime than the one the
+ * library was built against, PyTorch's for instance, 1 is taken as 0: the one
+ * graph has crashed there. */
 int macau_batch_set_graph(macau_batch* b, int on);
+int macau_batch_graph_available(void);              /* 1 if 1 is not taken as 0 in this process */
 int macau_batch_iterate(macau_batch* b, int n);     /* n iterations of every model, asynchronous */
 int macau_batch_synchronize(macau_batch* b);        /* wait; raise sampler failures */
 

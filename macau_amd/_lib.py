@@ -74,6 +74,7 @@ SIGNATURES = {
     "macau_batch_create": (_p, [_p, _i]),
     "macau_batch_free": (None, [_p]),
     "macau_batch_set_graph": (_i, [_p, _i]),
+    "macau_batch_graph_available": (_i, []),
     "macau_batch_iterate": (_i, [_p, _i]),
     "macau_batch_synchronize": (_i, [_p]),
     "macau_sample_latents": (_i, [_i, _i, _i, _p, _p, _p, _d, _p, _p, _d, _p, _p, _p, _ull, _i, _i, _i, _p]),

@@ -11,10 +11,33 @@
 // so a model advanced in a batch gives the same chain as the same model
 // advanced alone.  Without the batch graph (use_graph off) each model
 // replays its own iteration graph on its own streams, one after another on
-// the host and side by side on the device.
+// the host and side by side on the device.  The same is done where
+// batch_graph_available() does not hold.
 #include "batch.h"
 
+#include <link.h>
+
+#include <cstring>
+
 namespace mgpu {
+
+// A batch's graph is replayed only under the HIP runtime that the library was
+// built against, alone in its process: with the older runtime that PyTorch
+// brings along, launching it ended in a segmentation fault on the host (each
+// model's own graph runs there).
+bool batch_graph_available() {
+  int version = 0, copies = 0;
+  if (hipRuntimeGetVersion(&version) != hipSuccess || version / 100000 != HIP_VERSION / 100000) return false;
+  dl_iterate_phdr(
+      [](dl_phdr_info* info, size_t, void* n) {
+        const char* base = std::strrchr(info->dlpi_name, '/');
+        base = base ? base + 1 : info->dlpi_name;
+        if (std::strncmp(base, "libamdhip64.so", 14) == 0) ++*static_cast<int*>(n);
+        return 0;
+      },
+      &copies);
+  return copies == 1;
+}
 
 ModelBatch::ModelBatch(std::vector<Model*> ms) : models(std::move(ms)) {
   if (models.empty()) throw std::runtime_error("a batch needs at least one model");
@@ -57,11 +80,12 @@ void ModelBatch::launch_all() {
 }
 
 void ModelBatch::iterate(int n) {
-  if (n > 0 && launched_any && use_graph != last_graph) {
+  const bool one_graph = use_graph && (exec || batch_graph_available());
+  if (n > 0 && launched_any && one_graph != last_graph) {
     // switching between the two launch forms: the new form's streams wait
     // for the work the other form queued
     for (size_t q = 0; q < models.size(); q++) {
-      if (use_graph) {
+      if (one_graph) {
         HIPCHK(hipEventRecord(ev_join[q], models[q]->stream));
         HIPCHK(hipStreamWaitEvent(root, ev_join[q], 0));
       } else {
@@ -72,9 +96,9 @@ void ModelBatch::iterate(int n) {
   }
   if (n > 0) {
     launched_any = true;
-    last_graph = use_graph;
+    last_graph = one_graph;
   }
-  if (!use_graph) {
+  if (!one_graph) {
     // every model replays its own iteration (its own graph) on its own
     // streams; nothing orders the models, so the hardware queues run them
     // side by side

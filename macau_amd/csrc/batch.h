@@ -6,6 +6,9 @@
 
 namespace mgpu {
 
+// whether a batch may advance all models by one graph in this process
+bool batch_graph_available();
+
 class ModelBatch {
  public:
   explicit ModelBatch(std::vector<Model*> models);  // not owned; each initialised

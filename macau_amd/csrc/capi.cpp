@@ -558,6 +558,12 @@ static ModelBatch& B(macau_batch* h) {
   return *h->b;
 }
 
+int macau_batch_graph_available(void) {
+  API_BEGIN
+  return batch_graph_available() ? 1 : 0;
+  API_END_VAL(0)
+}
+
 int macau_batch_set_graph(macau_batch* b, int on) {
   API_BEGIN
   B(b).use_graph = on != 0;
