@@ -349,8 +349,8 @@ void launch_ftf(const CsrDev& F, const CsrDev& Ft, double* FtF, hipStream_t s);
 void launch_ftf_solve(const double* FtF, int n, const double* reg, double* W, double* X, int nrhs, int* fail,
                       hipStream_t s);
 // the same solve through F^T F = Q diag(d) Q^T: spectral_factor overwrites
-// A (F^T F, lower triangle) with Q, fills d (n) and Qt = Q^T and returns
-// false with a reason when the eigensolver is unavailable or fails;
+// A (F^T F) with Q, fills d (n) and Qt = Q^T (through A + shift I, shift of the
+// size of A's diagonal) and returns false with a reason when the eigensolver is unavailable or fails;
 // launch_spectral_solve sets X = Q diag(d + *reg)^{-1} Q^T B through
 // Y (n x nrhs) and part (plan.S x n x nrhs), a non-positive d_j + *reg
 // setting *fail to kFailDenseChol.  With idx (n columns of nfeat, ascending) and
@@ -361,7 +361,7 @@ struct SpectralPlan {
   int tchunk = 0;  // chunk depth
 };
 SpectralPlan spectral_plan(int n, int nrhs);
-bool spectral_factor(double* A, int n, double* d, double* Qt, hipStream_t s, std::string* why);
+bool spectral_factor(double* A, int n, double shift, double* d, double* Qt, hipStream_t s, std::string* why);
 void launch_spectral_solve(const double* Q, const double* Qt, const double* d, int n, const double* reg,
                            const double* B, double* Y, double* part, const SpectralPlan& p, double* X, int nrhs,
                            const int* idx, const int* pos, int nfeat, int* fail, hipStream_t s);

@@ -1266,7 +1266,10 @@ void MacauPrior::init(Model& m, int mode) {
       DevBuf Q(sq), Qt(sq);
       launch_spectral_take(FtF.as<double>(), nfeat, gram.idx, ftf_n, Q.as<double>(), m.stream);
       ftf_d.alloc((size_t)ftf_n * sizeof(double));
-      if (spectral_factor(Q.as<double>(), ftf_n, ftf_d.as<double>(), Qt.as<double>(), m.stream, &ftf_note)) {
+      double shift = (double)F_cols.size();  // to the mean of F^T F's diagonal
+      if (!binary) shift = std::inner_product(F_vals.begin(), F_vals.end(), F_vals.begin(), 0.0);
+      shift = shift > 0.0 && std::isfinite(shift) ? shift / ftf_n : 1.0;
+      if (spectral_factor(Q.as<double>(), ftf_n, shift, ftf_d.as<double>(), Qt.as<double>(), m.stream, &ftf_note)) {
         ftf_plan = spectral_plan(ftf_n, K);
         ftf_y.alloc(ks);
         ftf_part.alloc(ftf_plan.S * ks);

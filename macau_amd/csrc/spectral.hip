@@ -9,9 +9,13 @@
 //     Y = Q^T B,   Y[j][:] /= (d_j + lambda_beta),   X = Q Y,
 // two n x n by n x nrhs FP64 products that stream Q from HBM once each, in
 // place of n / 32 dependent factor and solve steps.  F's empty columns are left
-// out of the decomposition and taken as B / lambda_beta: the eigensolver's vectors
-// for the large null space that they make were not orthogonal for some matrices
-// (15000 x 2000 with 1100 empty columns: those columns off by up to 9e-2).  Q is kept twice (Q and
+// out of the decomposition and taken as B / lambda_beta.  A + shift I is
+// decomposed, shift of the size of A's diagonal: in a null space (empty or equal
+// columns, fewer rows than columns) the tridiagonal form has entries near 1e-160,
+// whose squares underflow, and the eigensolver's vectors there are not orthogonal
+// for some matrices (15000 x 2000 with 1100 empty columns: 26 of 40, max |Q^T Q - I|
+// up to 0.4; their non-empty columns alone up to 9e-10; 3e-14 for all with the
+// shift).  Q is kept twice (Q and
 // Q^T, both column-major) so both products read M's columns contiguously.
 // A non-positive d_j + lambda_beta sets the same fail flag as a non-positive
 // Cholesky pivot.
@@ -271,7 +275,13 @@ const SolverApi& solver_api() {
 }
 }  // namespace
 
-bool spectral_factor(double* A, int n, double* d, double* Qt, hipStream_t s, std::string* why) {
+// x[i stride] += v, i = 0 .. n-1
+__global__ void __launch_bounds__(256) k_shift(double* x, int n, size_t stride, double v) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) x[i * stride] += v;
+}
+
+bool spectral_factor(double* A, int n, double shift, double* d, double* Qt, hipStream_t s, std::string* why) {
   const SolverApi& api = solver_api();
   if (!api.error.empty()) {
     if (why) *why = api.error;
@@ -286,12 +296,14 @@ bool spectral_factor(double* A, int n, double* d, double* Qt, hipStream_t s, std
   int* info = nullptr;
   bool ok = api.set_stream(h, s) == rocblas_status_success && hipMalloc(&E, (size_t)n * sizeof(double)) == hipSuccess &&
             hipMalloc(&info, sizeof(int)) == hipSuccess;
+  if (ok) hipLaunchKernelGGL(k_shift, dim3((n + 255) / 256), dim3(256), 0, s, A, n, (size_t)n + 1, shift);
   if (ok) ok = api.dsyevd(h, rocblas_evect_original, rocblas_fill_lower, n, A, n, d, E, info) == rocblas_status_success;
   int hinfo = -1;
   if (ok) ok = hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess &&
                hipStreamSynchronize(s) == hipSuccess && hinfo == 0;
   if (!ok && why) *why = "rocsolver_dsyevd failed (info " + std::to_string(hinfo) + ")";
   if (ok) {
+    hipLaunchKernelGGL(k_shift, dim3((n + 255) / 256), dim3(256), 0, s, d, n, (size_t)1, -shift);
     hipLaunchKernelGGL(k_transpose, dim3((n + 31) / 32, (n + 31) / 32), dim3(256), 0, s, (const double*)A, n, Qt);
     ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
     if (!ok && why) *why = "transposing the eigenvectors failed";

@@ -50,3 +50,29 @@ def test_spectral_solve_with_empty_columns(seed, N, nf, K, values, monkeypatch):
     e = [np.linalg.norm(beta[0][s] - beta[1][s]) / np.linalg.norm(beta[1][s]) for s in (fc, empty)]
     print("beta: used columns %.1e, empty ones %.1e" % tuple(e))
     assert e[0] < 2.2e-8 and e[1] < 1e-13
+
+
+# equal columns among the non-empty ones make a null space too; without a shift
+# of the decomposed matrix the eigenvectors of these two were not orthogonal there
+@pytest.mark.parametrize("seed,nf", [(18, 1872), (29, 1921)])
+def test_equal_columns_keep_the_spectral_solve(seed, nf, monkeypatch):
+    announce("F^T F with equal columns seed=%d nf=%d" % (seed, nf))
+    rng = np.random.default_rng(seed)
+    assert rng.integers(800, 2000) == nf
+    N, K = 12000, 8
+    fr, fc = _fingerprints(rng, N, nf, 60)
+    r = np.arange(N)
+    beta = []
+    for solver in ("spectral", "cholesky"):
+        monkeypatch.setenv("MACAU_AMD_FTF_SOLVER", solver)
+        m = GpuModel(2, K, 4.0)
+        m.data(np.stack([r, r % 20], 1), np.sin(r), [N, 20], np.stack([r[:50], r[:50] % 20], 1), np.sin(r[:50]))
+        m.prior((fr, fc, None, N, nf), 5.0, 1e-6, 10000)
+        m.prior()
+        m.setup(2, 50, 1, _lib.SAMPLER_BATCHED)
+        assert _lib.lib().macau_get_ftf_solver(m.h, 0) == (2 if solver == "spectral" else 1)
+        m.iterate(1)
+        beta.append(m.link(0, nf))
+    e = np.linalg.norm(beta[0] - beta[1]) / np.linalg.norm(beta[1])
+    print("beta: %.1e" % e)
+    assert e < 2.2e-8
