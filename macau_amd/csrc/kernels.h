@@ -350,9 +350,9 @@ void launch_ftf_solve(const double* FtF, int n, const double* reg, double* W, do
                       hipStream_t s);
 // the same solve through F^T F = Q diag(d) Q^T: spectral_factor overwrites
 // A (F^T F) with Q, fills d (n) and Qt = Q^T (through A + shift I, shift of the
-// size of A's diagonal) and returns false with a reason when the eigensolver is unavailable or fails;
-// launch_spectral_solve sets X = Q diag(d + *reg)^{-1} Q^T B through
-// Y (n x nrhs) and part (plan.S x n x nrhs), a non-positive d_j + *reg
+// size of A's diagonal) and returns false with a reason when the eigensolver is
+// unavailable or fails; launch_spectral_solve sets X = Q diag(d + *reg)^{-1} Q^T B
+// through Y (n x nrhs) and part (plan.S x n x nrhs), a non-positive d_j + *reg
 // setting *fail to kFailDenseChol.  With idx (n columns of nfeat, ascending) and
 // pos (each column's place among them, or -1) B and X have all nfeat columns and
 // the others' X is B / *reg; launch_spectral_take gives their A

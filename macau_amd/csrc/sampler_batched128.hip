@@ -1,5 +1,6 @@
 // sampler_batched128.hip -- the batched per-row sampler for K in (64, 128]:
-// split-BF16 MFMA Gram of a 128 x 128 precision matrix, one row per wave.
+// split-BF16 MFMA Gram of a 128 x 128 precision matrix, one row per wave (up to
+// 1024 rows: two, four or eight waves share its Gram, k_light128w).
 //
 // Same mathematics as the K <= 64 samplers (sample_latent_blas,
 // latentprior.cpp:361-385): P = Lambda + alpha G = L L^T, b = alpha c +
@@ -18,7 +19,9 @@
 // eight waves, in tiles), a 1 KB transposition buffer per wave, and the normals.
 //   * Gram: per 32-nonzero chunk lane (g, n) gathers component sigma(n) of each
 //     block of nonzeros 8g .. 8g + 7, which is the operand layout of
-//     v_mfma_f32_16x16x32_bf16 (HiHi^T + HiLo^T + LoHi^T + LoLo^T per tile).
+//     v_mfma_f32_16x16x32_bf16.  A factor enters in three BF16 parts (24 bits),
+//     a tile takes six of their nine products: HiHi^T + HiMid^T + MidHi^T +
+//     MidMid^T + HiLo^T + LoHi^T.
 //   * Factorisation by 16 columns: the diagonal tile gives L_kk^{-1} (see
 //     diag_factor), row k's tiles become R_kj = L_kk^{-1} P_kj and the rest
 //     P_ij -= R_ki^T R_kj.
