@@ -340,14 +340,25 @@ def load_traffic(name):
 
 def cg_bytes_per_iteration(w):
     """Algorithmic HBM bytes of one block-CG iteration (linop.h:279-332) for
-    the row side information: F and F^T read once each by the two SpMMs
-    (int32 index + FP64 value per nonzero), and 13 streaming passes over an
-    nrhs x nfeat FP64 block (KP written, P read by the SpMM gather and the
-    P^T KP product, KP read twice, X and R read and written, R read for
-    R R^T, P read and written by the direction update, reg P read)."""
+    the row side information, and the columns it runs on: F and F^T read once
+    each by the two SpMMs (int32 index + FP64 value per nonzero), or the Gram
+    matrix of the non-empty columns where the solve takes that, and 13
+    streaming passes over an nrhs x columns FP64 block (KP written, P read by
+    the product's gather and the P^T KP product, KP read twice, X and R read
+    and written, R read for R R^T, P read and written by the direction update,
+    reg P read).  From 128 empty columns on, K columns stand for them all (K up
+    to 32)."""
     F = w["side"][0]
     K = w["settings"]["num_latent"]
-    return 2 * F.nnz * 12 + 13 * K * F.shape[1] * 8
+    used = nonempty_columns(F)
+    if K > 32 or F.shape[1] - used < 128:
+        return 2 * F.nnz * 12 + 13 * K * F.shape[1] * 8, F.shape[1]
+    gram = used <= 2048 and used ** 2 <= 128 * F.nnz and F.shape[0] * used ** 2 <= 1.7e11
+    return (8 * used ** 2 if gram else 2 * F.nnz * 12) + 13 * K * (used + K) * 8, used + K
+
+
+def nonempty_columns(F):
+    return len(np.unique(F.tocoo().col))
 
 
 def autotune(w, args, log):
@@ -510,7 +521,7 @@ def main():
     ap.add_argument("--cpu-iters", type=int, default=25)
     ap.add_argument("--sampler", choices=["batched", "batched-norefine", "plain"], default=None,
                     help="batched-norefine: the batched sampler without the condition probes and refinement")
-    ap.add_argument("--hw-queues", type=int, default=16, choices=range(1, 33), metavar="1..32",
+    ap.add_argument("--hw-queues", type=int, default=4, choices=range(1, 33), metavar="1..32",
                     help="hardware queues per process for --workload c5 (GPU_MAX_HW_QUEUES)")
     ap.add_argument("--tune", action="store_true",
                     help="time the default launch shapes, run the autotuner, time the tuned shapes")
@@ -524,10 +535,10 @@ def main():
         print("[bench] " + msg, file=sys.stderr, flush=True)
 
     if args.workload == "c5":
-        # 64 models with a graph and streams each: with 16 hardware queues per
-        # process (HIP's default is 4) they serialise least (batch it/s with
-        # 4, 8, 12, 16, 32 queues: 24.7, 23.8, 24.8, 27.2, 12.8); read when the
-        # library first touches the GPU, so set before that
+        # 64 models with a graph and streams each: batch it/s with HIP's default
+        # of 4 hardware queues per process, with 8 and with 16: 62.6, 43.7, 42.2
+        # (one graph of all models: 60 with each); read when the library first
+        # touches the GPU, so set before that
         os.environ["GPU_MAX_HW_QUEUES"] = str(args.hw_queues)
         return bench_c5(args, log)
     t0 = time.perf_counter()
@@ -625,10 +636,11 @@ def main():
         solver = res[head]["cg"][-2]
         if solver == 2:
             # (F^T F + lambda_beta I)^{-1} as Q diag(d + lambda_beta)^{-1} Q^T: two n x n FP64
-            # products per iteration stream Q and Q^T once each
-            qb = 2.0 * nf * nf * 8
+            # products per iteration stream Q and Q^T (of the non-empty columns) once each
+            used = nonempty_columns(w["side"][0])
+            qb = 2.0 * used * used * 8
             gbs = qb / (ph[nm] * 1e-3) / 1e9
-            out["ftf_spectral"] = {"features": nf, "prior_rows_ms": float(ph[nm]), "eigenvector_bytes": qb,
+            out["ftf_spectral"] = {"features": nf, "nonempty_features": used, "prior_rows_ms": float(ph[nm]), "eigenvector_bytes": qb,
                                    "setup_s_incl_eigendecomposition": res[head]["setup_s"],
                                    "achieved_GBs_lower_bound": gbs, "frac_of_hbm_peak": gbs / PEAK_HBM_GBS,
                                    "note": "time includes the two products, the beta noise draw, F^T Y, Uhat "
@@ -643,9 +655,10 @@ def main():
     elif w["side"][0] is not None:
         # the row prior update is dominated by the block CG for the link matrix
         iters = res[head]["cg"][0]
-        cgb = cg_bytes_per_iteration(w) * max(iters, 1)
+        per_iter, columns = cg_bytes_per_iteration(w)
+        cgb = per_iter * max(iters, 1)
         gbs = cgb / (ph[nm] * 1e-3) / 1e9
-        out["block_cg"] = {"iters_per_solve": iters, "prior_rows_ms": float(ph[nm]),
+        out["block_cg"] = {"iters_per_solve": iters, "columns": columns, "prior_rows_ms": float(ph[nm]),
                            "algorithmic_bytes_per_solve": cgb, "achieved_GBs_lower_bound": gbs,
                            "frac_of_hbm_peak": gbs / PEAK_HBM_GBS,
                            "note": "time includes the beta noise draw, Uhat and lambda_beta updates"}
